@@ -239,18 +239,19 @@ int grouped_class_blocks(int cls, int kind);
 hipError_t launch_grouped(int cls, int kind, const GroupProblem *probs,
                           const GroupTile *tiles, int64_t ntiles, int nblocks, hipStream_t st);
 // k-means assignment (hml_k_kmeans.hip).  Screened form: kKmWaves waves
-// per workgroup, each on its own 16-row tile; NI = dims / 16 rounded up, NT
-// centroid tiles of 16 per screening pass.  Direct form (up to 8 dims, or
-// clusters x dims < 1024 up to 32 dims): kKmDirectWaves waves, each on 64
-// rows, one per lane; NI = dims.  KC centroids per LDS chunk; tiles = wave tiles of rows.
+// per workgroup, each on its own 32-row tile (xfloats floats of LDS); ni =
+// dims / 16 rounded up.  Direct form (up to 32 dims, few clusters):
+// kKmDirectWaves waves, each on 64 rows, one per lane; ni = dims.  KC
+// centroids per LDS chunk; tiles = wave tiles of rows.
 constexpr int kKmWaves = 8;
 constexpr size_t kKmLdsBytes = 163840;      // all of a CU's LDS
 constexpr int kKmDirectWaves = 4;
 constexpr size_t kKmDirectLdsBytes = 65536; // centroid chunk of the direct form
 constexpr int kKmDirectMaxDims = 32;
+constexpr int64_t kKmDirectWork = 240;      // dims x clusters below which it runs
 struct KmeansPlan {
   bool direct = false;
-  int ni = 1, nt = 1, KC = 0;
+  int ni = 1, KC = 0, xfloats = 0;
   size_t lds = 0;
   int64_t tiles = 0;
 };

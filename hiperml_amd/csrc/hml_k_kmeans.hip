@@ -8,34 +8,55 @@
 // (delta = x - c, one rounding per step), first k strictly below the
 // running minimum (from FLT_MAX).  Same result here, different machine:
 //
-//  1. Screening on the FP32 matrix cores.  |x - c|^2 = |x|^2 + s_k with
-//     s_k = |c_k|^2 - 2 x.c_k, and x.c_k for a 16-row tile against 16
-//     centroids is one v_mfma_f32_16x16x4f32 per 4 dims: a skinny GEMM
-//     (rows x dims) * (dims x centroids).  Lane l = 16q + r holds row r,
-//     dims 16i + 4q .. +3 (i < NI) from row-contiguous loads; the centroid
-//     operand uses the same dim order, so MFMA j = 4i + e, k-slot q covers
-//     dim 16i + 4q + e.  The result lane l holds x_r . c_{16t + 4q + i}.
+//  1. Screening on the 16-bit matrix cores.  |x - c|^2 = |x|^2 - 2 a_k with
+//     a_k = x.c_k - |c_k|^2 / 2, and x.c_k for 32 rows against 32 centroids
+//     is a product of bf16 terms x = xh + xl, c = ch + cl (round to
+//     nearest): three v_mfma_f32_32x32x16_bf16 per 16 dims (cl.xh, ch.xl,
+//     ch.xh), the accumulator starting at -|c|^2 / 2.  FP32 MFMAs would take
+//     5 times as long for the same dims.
 //  2. A bound on how far the reference's float distance can be from
-//     |x|^2 + s~_k (the screened value): with S_k = (|x| + |c_k|)^2 +
-//     |s~_k|, the reference's rounding (D + 3 roundings of nonnegative
-//     terms) and the screen's (D-term dot and norm, one subtraction) are
-//     each below (2D + 4) 2^-24 S_k; the margin m_k = 4 (D + 4) 2^-24 S_k
-//     covers both with slack for rounding the margin itself.  Only
-//     centroids with s~_k - m_k <= min_j (s~_j + m_j) can be the exact
-//     argmin; NaN or infinite screens make every centroid a candidate.
-//  3. Exact refinement of the candidates (usually one per row) with the
-//     reference's own arithmetic, from LDS copies of the row and the
-//     centroid; the four lanes of a row refine disjoint candidate sets in
-//     ascending k and combine by (distance, index), which is the
-//     reference's "first strict minimum".
+//     |x|^2 - 2 a~_k (the screened value), in units of 2^-24 (|x| + |c_k|)^2:
+//       2D + 4   the reference's own roundings;
+//       D        the norm;
+//       96 KS    the accumulation, KS = D / 16 rounded up: 48 KS products
+//                added with an error of at most 2^-23 of the running sum's
+//                bound |x||c_k| + |c_k|^2 / 2 each, doubled in 2 a_k;
+//       96       the split: xl, cl round at 2^-18 of x, c, and xl.cl (2^-18)
+//                is left out: 3 2^-18 |x||c_k|, doubled, |x||c_k| being at
+//                most (|x| + |c_k|)^2 / 4;
+//       64       the index kept in the low 4 bits of a~_k.
+//     Their sum is below 4D + 96 KS + 256.  With M that factor times (|x| +
+//     max |c|)^2, only centroids with a~_k >= max a~ - M can be the exact
+//     argmin (each side's distance may be off by M, 2 a~ by 2 M).
+//  3. Each lane keeps the two largest a~ of its even and of its odd centroid
+//     tiles.  If a row's second largest value lies below the limit its
+//     argmin is known (the usual case: no distance is computed).  Otherwise
+//     the trackers' centroids above the limit are compared by the
+//     reference's own arithmetic, or, when a value that no tracker names
+//     could be above it, the tile is screened again and every centroid above
+//     the limit compared.  The two lanes of a row hold disjoint centroids
+//     and combine by (distance, index): the reference's "first strict
+//     minimum".
 //
-// Centroids live in LDS (zero padded to 16 NI dims, row stride 16 NI + 4
-// floats), staged once per workgroup when they fit, else chunk by chunk per
-// row step with the workgroup's waves in lockstep.  Candidates are found
-// per pass of NT x 16 centroids; passes and chunks combine in ascending k
-// with a strict comparison, so any partition gives the same answer.
+// What bounds it: for few centroids the row stream (2^24 rows, 32 dims x 16
+// clusters: 0.38 ms, 5.8 TB/s, was 0.54), for many the matrix cores and the
+// three vector instructions per (row, centroid) of the trackers, which both
+// are busy 0.4 and 0.7 of the time at 32 x 256 (1.01 ms, was 3.08); 32 x 64
+// 0.46 ms (was 1.04), 64 x 64 0.96 (was 1.75), 2^23 rows 64 x 256 0.92 (was
+// 3.11).  64 rows per wave halve the LDS reads per row but held 2-3 waves
+// per SIMD: 2-15% slower.  Four trackers per lane make the second screening
+// rarer and cost registers: up to 10% slower.  Rows equidistant from many
+// centroids cost up to two screenings and a distance per candidate.
+//
+// Centroids live in LDS as bf16 terms in MFMA operand order (a fragment is
+// one conflict-free 16-byte read per lane) beside their norms, staged once
+// per workgroup when they fit, else chunk by chunk per row step with the
+// workgroup's waves in lockstep.  Every wave streams its rows 32 at a time
+// straight into its own LDS area (buffer_load ... lds), the next tile's load
+// in flight while this one is screened.
 #include <float.h>
 
+#include <algorithm>
 #include <utility>
 
 #include "hml_internal.h"
@@ -46,6 +67,10 @@ namespace {
 
 constexpr uint32_t kNone = 0xffffffffu;
 
+// s_waitcnt immediates (gfx9 encoding): vmcnt(0) lgkmcnt(0), and lgkmcnt(0)
+constexpr int kWaitAll = 0x0070;
+constexpr int kWaitLgkm0 = 0xC07F;
+
 struct KmParams {
   const float *rows;
   const float *ctrds;
@@ -53,12 +78,9 @@ struct KmParams {
   int64_t nrows;
   int64_t steps;  // row steps of kKmWaves wave tiles per workgroup (uniform)
   int32_t D, K;
-  int32_t KC;     // centroids per LDS chunk (multiple of 16 NT)
+  int32_t KC;     // centroids per LDS chunk (screened: a multiple of 32)
+  int32_t xfloats;  // screened: floats of one wave's row tile in LDS
 };
-
-__device__ __forceinline__ f4 mfma4(float a, float b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -66,10 +88,6 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Exact distance of LDS row xr to LDS centroid cr over nd4 groups of 4
-// dims (dims past D are zero in both, and adding (+0)^2 to a nonnegative
-// sum changes nothing).  The groups are read 4 at a time before their
-// arithmetic, so the LDS latency is paid once per 16 dims.
 template <bool FUSED>
 __device__ __forceinline__ float exact_step(float dist, float x, float c) {
   const float delta = x - c;
@@ -81,238 +99,374 @@ __device__ __forceinline__ float exact_step(float dist, float x, float c) {
   }
 }
 
-template <bool FUSED, int NI>
-__device__ __forceinline__ float exact_dist(const float *xr, const float *cr, int nd4) {
+// Reference distance of row xr to centroid cr, both in global memory at any
+// 4-byte alignment; 16 dims of each are loaded before their arithmetic.
+struct __attribute__((packed, aligned(4))) KmQuad {
+  float v[4];
+};
+template <bool FUSED, int KS>
+__device__ __forceinline__ float exact_dist(const float *__restrict__ xr,
+                                            const float *__restrict__ cr, int D) {
   float dist = 0.f;
 #pragma unroll
-  for (int g = 0; g < NI; ++g) {
-    if (4 * g < nd4) {
-      f4 xv[4], cv[4];
+  for (int s = 0; s < KS; ++s) {
+    KmQuad xv[4], cv[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        xv[j] = *reinterpret_cast<const f4 *>(xr + 16 * g + 4 * j);
-        cv[j] = *reinterpret_cast<const f4 *>(cr + 16 * g + 4 * j);
+    for (int j = 0; j < 4; ++j)
+      if (16 * s + 4 * j + 4 <= D) {
+        xv[j] = *reinterpret_cast<const KmQuad *>(xr + 16 * s + 4 * j);
+        cv[j] = *reinterpret_cast<const KmQuad *>(cr + 16 * s + 4 * j);
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (4 * g + j < nd4) {
+    for (int j = 0; j < 4; ++j)
+      if (16 * s + 4 * j + 4 <= D) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) dist = exact_step<FUSED>(dist, xv[j][e], cv[j][e]);
-        }
-    }
+        for (int e = 0; e < 4; ++e) dist = exact_step<FUSED>(dist, xv[j].v[e], cv[j].v[e]);
+      }
   }
+  for (int d = D & ~3; d < D; ++d) dist = exact_step<FUSED>(dist, xr[d], cr[d]);
   return dist;
 }
 
-// 128 centroids per pass over up to 32 dims: at most 128 VGPRs (4 waves per
-// SIMD, two 8-wave workgroups per CU; without the bound the 32-dim tile took
-// 129 and ran one workgroup per CU: 32 x 256 on 2^24 rows 3.81 -> 3.14 ms).
-// The other tiles fit without it (bounding them measured slower), and the
-// 33..64-dim ones would spill.
-template <int NI, int NT, bool FUSED>
-__global__ __launch_bounds__(64 * kKmWaves, (NT == 8 && NI <= 2) ? 4 : 1) void k_kmeans_assign(KmParams p) {
-  constexpr int DP = 16 * NI + 4;  // LDS row stride (floats), 16-byte multiple
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef float f16v __attribute__((ext_vector_type(16)));
+
+// hi / lo bf16 terms of 8 floats (round to nearest; the residual is exact)
+__device__ __forceinline__ void split8(const float (&v)[8], b8 &hi, b8 &lo) {
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    const b2 h = __builtin_convertvector(f2{v[j], v[j + 1]}, b2);
+    hi[j] = h[0];
+    hi[j + 1] = h[1];
+    const b2 l = __builtin_convertvector(f2{v[j] - (float)h[0], v[j + 1] - (float)h[1]}, b2);
+    lo[j] = l[0];
+    lo[j + 1] = l[1];
+  }
+}
+
+// Squared norms at or above kKmNormMax (and NaN) take a centroid out of the
+// screen; rows that could still choose it (|x|^2 or the best screened
+// distance not below kKmRowMax) are refined over every centroid.
+constexpr float kKmNormMax = 1e37f;
+constexpr float kKmRowMax = 1e36f;
+// screen value of an excluded or padding centroid
+constexpr float kKmExcluded = -1e38f;
+
+// KS = k-steps of 16 dims, MULTI = the centroids take several LDS chunks,
+// VEC = dims a multiple of 4.
+template <int KS, bool MULTI, bool VEC, bool FUSED>
+__global__ __launch_bounds__(64 * kKmWaves, 4) void k_kmeans_screen(KmParams p) {
+  constexpr int NQ = KS * 2;  // 1 KB DMA loads per row tile (at most)
   extern __shared__ f4 km_lds4[];
-  float *lds = reinterpret_cast<float *>(km_lds4);
-  float *cs = lds;                   // KC x DP centroids of the current chunk
-  float *cn = cs + p.KC * DP;        // their squared norms
-  float *cmx = cn + p.KC;            // the largest norm of the chunk (4 floats)
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  float *xs = cmx + 4 + w * 16 * DP;  // this wave's 16 rows
+  char *lds = reinterpret_cast<char *>(km_lds4);
+  b8 *cf = reinterpret_cast<b8 *>(lds);                                 // centroid fragments
+  float *nrm = reinterpret_cast<float *>(lds + (size_t)p.KC * KS * 64); // -|c|^2 / 2
+  // max as a median with infinity (in a register the compiler does not see
+  // through), without the canonicalising moves fmaxf needs for unknown
+  // inputs; a result that a NaN could have entered is never used
+  float inf;
+  asm("s_mov_b32 %0, 0x7f800000" : "=s"(inf));
+  auto vmax = [&](float a, float b) { return __builtin_amdgcn_fmed3f(a, b, inf); };
   const int lane = threadIdx.x & 63;
-  const int q = lane >> 4, r = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int D = p.D, K = p.K;
-  const int nd4 = (D + 3) >> 2;
-  const int nchunks = (K + p.KC - 1) / p.KC;
-  // margin per centroid: tau S_k (see the screen below); per row and chunk
-  // the bound tau2 (|x| + max |c|)^2 >= tau S_k is used for every centroid
-  const float tau = 4.0f * (float)(D + 4) * 0x1p-24f;
-  const float tau2 = 2.0f * tau * (1.0f + 0x1p-10f);
+  float *xs = nrm + p.KC + w * p.xfloats;  // this wave's row tile
+  const int h = lane >> 5, r = lane & 31;
+  const int nchunks = MULTI ? (K + p.KC - 1) / p.KC : 1;
+  // margin factor, see the error terms at the top of the file
+  const float tau = (float)(4 * D + 96 * KS + 256) * 0x1p-24f * (1.0f + 0x1p-8f);
 
-  auto stage = [&](int c0) {
+  // Stages centroids c0 .. c0 + KC - 1 (zeros past K) and returns the
+  // largest norm among those in the screen.  Lanes l and l ^ 32 hold the two
+  // halves of a centroid's dims, in the fragment layout itself: (tile of 32,
+  // k-step, hi / lo, lane, 8 dims).
+  auto stage = [&](int c0) -> float {
     __syncthreads();  // every wave is done with the previous chunk
-    for (int idx = threadIdx.x; idx < p.KC * DP; idx += blockDim.x) {
-      const int k = idx / DP, d = idx - k * DP;
-      cs[idx] = (c0 + k < K && d < D) ? p.ctrds[(int64_t)(c0 + k) * D + d] : 0.f;
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < p.KC; k += blockDim.x) {
-      float s = 0.f;
-      for (int d = 0; d < D; ++d) s = __builtin_fmaf(cs[k * DP + d], cs[k * DP + d], s);
-      cn[k] = s;
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-      // largest squared norm (the zero padding adds nothing; a NaN norm is
-      // skipped: that centroid's screen is NaN, which always passes)
-      float mx = 0.f;
-      for (int k = threadIdx.x; k < p.KC; k += 64) mx = __builtin_fmaxf(mx, cn[k]);
+    for (int i = threadIdx.x; i < p.KC * 2; i += 64 * kKmWaves) {
+      const int t = i >> 6, k = 32 * t + r;
+      const float *c = p.ctrds + (int64_t)(c0 + k) * D + 8 * h;
+      float v[KS][8], s2 = 0.f;
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, off));
-      if (threadIdx.x == 0) cmx[0] = __builtin_sqrtf(mx);
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          v[s][j] = c0 + k < K && 16 * s + 8 * h + j < D ? c[16 * s + j] : 0.f;
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s2 = __builtin_fmaf(v[s][j], v[s][j], s2);
+      s2 += __shfl_xor(s2, 32);
+      const bool in = c0 + k < K && s2 < kKmNormMax;
+      if (h == 0) nrm[k] = in ? -0.5f * s2 : kKmExcluded;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (!in) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[s][j] = 0.f;
+        }
+        b8 hi, lo;
+        split8(v[s], hi, lo);
+        cf[(t * KS + s) * 128 + lane] = hi;
+        cf[(t * KS + s) * 128 + 64 + lane] = lo;
+      }
     }
     __syncthreads();
+    float mx = 0.f;
+    for (int k = lane; k < p.KC; k += 64) {
+      const float n2 = nrm[k];
+      mx = n2 > 0.5f * kKmExcluded ? __builtin_fmaxf(mx, -2.0f * n2) : mx;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, off));
+    return __builtin_sqrtf(mx);
   };
-  if (nchunks == 1) stage(0);
 
-  // rows of step st's tile (zeros for a tile past the end); the next step's
-  // rows are loaded while this step's are screened
-  auto load_rows = [&](int64_t st, f4 (&dst)[NI]) {
-    const int64_t row0 = ((st * gridDim.x + blockIdx.x) * kKmWaves + w) * 16;
-    if (row0 >= p.nrows) {
+  // The wave's 32 rows are one contiguous block of memory, DMAed flat
+  // into the wave's LDS tile.  With D a multiple of 4, row x's 16-byte chunk
+  // c goes to chunk x nc + (c + x nc / 16) % nc (nc = D / 4), which spreads
+  // 8 consecutive rows' reads of one chunk over distinct banks; otherwise
+  // the block is stored as it is and read float by float.
+  const int nc = D >> 2;
+  const int nchunk16 = 8 * D;  // 16-byte chunks of the tile
+  uint32_t aoff[NQ];
 #pragma unroll
-      for (int i = 0; i < NI; ++i) dst[i] = f4{0.f, 0.f, 0.f, 0.f};
-      return;
+  for (int q = 0; q < NQ; ++q) {
+    const int pos = 64 * q + lane;
+    int src = pos;
+    if (VEC) {
+      const int x = pos / nc, sl = pos - x * nc;
+      int c = sl - ((x * nc) >> 4) % nc;
+      if (c < 0) c += nc;
+      src = x * nc + c;
     }
-    const int64_t left = (p.nrows - row0) * D * 4;
-    const __amdgpu_buffer_rsrc_t rs =
-        make_rsrc(p.rows + row0 * D, left < kRsrcMax ? (int32_t)left : kRsrcMax);
+    aoff[q] = pos < nchunk16 ? (uint32_t)src * 16u : kOOB;
+  }
+  // LDS offsets (floats) of this lane's chunks: dims 16 s + 8 h + 4 j .. +3
+  // of row r
+  int xo[VEC ? 2 * KS : 1];
+  if (VEC) {
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int d0 = 16 * i + 4 * q;
-      const bool rin = row0 + r < p.nrows;
-      const uint32_t o = (uint32_t)((r * D + d0) * 4);
-      if (d0 + 4 <= D) {
-        dst[i] = buf_load4<kBufNT>(rs, rin ? o : kOOB, 0);
-      } else {
-        // a group that crosses the end of the row, element by element
-        // (its tail belongs to the next row, or lies past the array)
+    for (int i = 0; i < 2 * KS; ++i) {
+      int c = 4 * (i >> 1) + 2 * h + (i & 1);
+      if (c >= nc) c = 0;  // past the row: masked
+      xo[i] = 4 * (r * nc + (c + ((r * nc) >> 4)) % nc);
+    }
+  } else {
+    xo[0] = r * D + 8 * h;
+  }
+
+  const int64_t wstep = (int64_t)gridDim.x * kKmWaves;
+  int64_t tile = (int64_t)blockIdx.x * kKmWaves + w;
+  // rows of a tile into the wave's LDS area (its earlier reads are done)
+  auto load_rows = [&](int64_t tl) {
+    const int64_t row0 = tl * 32;
+    if (row0 >= p.nrows) return;
+    const float *base = p.rows + row0 * D;
+    if (row0 + 32 <= p.nrows) {
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, 32 * D * 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          dst[i][e] = buf_load1(rs, rin && d0 + e < D ? o + 4 * e : kOOB, 0);
+      for (int q = 0; q < NQ; ++q)
+        if (64 * q < nchunk16) buf_load_lds16<kBufNT>(rs, xs + 256 * q, aoff[q], 0);
+    } else {
+      const int n = (int)(p.nrows - row0) * D;
+      for (int i = lane; i < n; i += 64) {
+        int o = i;
+        if (VEC) {
+          const int x = i / D, d = i - x * D;
+          o = 4 * (x * nc + ((d >> 2) + ((x * nc) >> 4)) % nc) + (d & 3);
+        }
+        xs[o] = base[i];
       }
     }
   };
-  f4 xnext[NI];
-  load_rows(0, xnext);
 
-  for (int64_t st = 0; st < p.steps; ++st) {
-    const int64_t tile = (st * gridDim.x + blockIdx.x) * kKmWaves + w;
-    const int64_t row0 = tile * 16;
+  load_rows(tile);
+  float cmax = 0.f;
+  if (!MULTI) cmax = stage(0);
+
+  for (int64_t st = 0; st < p.steps; ++st, tile += wstep) {
+    const int64_t row0 = tile * 32;
     const bool live = row0 < p.nrows;  // wave-uniform
-    if (nchunks == 1 && !live) break;  // later steps only go further
+    if (!MULTI && !live) break;        // later steps only go further
 
-    f4 xv[NI];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) xv[i] = xnext[i];
-    if (st + 1 < p.steps) load_rows(st + 1, xnext);
-    float xx = 0.f, xr = 0.f;
-    if (live) {
-      wave_lds_sync();  // the previous tile's refinement reads are done
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        *reinterpret_cast<f4 *>(xs + r * DP + 16 * i + 4 * q) = xv[i];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) xx = __builtin_fmaf(xv[i][e], xv[i][e], xx);
-      }
-      xx += __shfl_xor(xx, 16);
-      xx += __shfl_xor(xx, 32);
-      xr = __builtin_sqrtf(xx);
+    b8 xh[KS], xl[KS];
+    float xx = 0.f;
+    if (!MULTI || live) {
+      __builtin_amdgcn_s_waitcnt(kWaitAll);  // the tile is in LDS
+      __builtin_amdgcn_sched_barrier(0);
       wave_lds_sync();
+      float v[KS][8];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (VEC) {
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const f4 q = *reinterpret_cast<const f4 *>(xs + xo[2 * s + j]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[s][4 * j + e] = q[e];
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[s][j] = xs[xo[0] + 16 * s + j];
+        }
+      }
+      wave_lds_sync();
+      __builtin_amdgcn_s_waitcnt(kWaitLgkm0);  // the reads above are done
+      __builtin_amdgcn_sched_barrier(0);
+      load_rows(tile + wstep);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (s == KS - 1) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[s][j] = 16 * s + 8 * h + j < D ? v[s][j] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) xx = __builtin_fmaf(v[s][j], v[s][j], xx);
+        split8(v[s], xh[s], xl[s]);
+      }
+      xx += __shfl_xor(xx, 32);
     }
 
-    float rbd = FLT_MAX;
-    uint32_t rbk = kNone;
-    float thi = __builtin_inff();  // min of s_j + M over the centroids screened so far
+    // lane (h, r), entry i: x.c - |c|^2 / 2 for row r and centroid
+    // 32 tl + 8 (i / 4) + 4 h + i % 4 of the chunk
+    auto screen_tile = [&](int tl) -> f16v {
+      f16v acc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f4 q = *reinterpret_cast<const f4 *>(nrm + 32 * tl + 8 * i + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[4 * i + e] = q[e];
+      }
+      const b8 *f = cf + tl * KS * 128 + lane;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const b8 ch = f[s * 128], cl = f[s * 128 + 64];
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cl, xh[s], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xl[s], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xh[s], acc, 0, 0, 0);
+      }
+      return acc;
+    };
+
+    // The two largest screen values of each lane's even (g = 0) and odd
+    // centroid tiles.  The entry's index in its tile sits in the low 4 bits
+    // of the value; bk holds the first centroid of the largest's tile.
+    float m1[2], m2[2];
+    int bk[2] = {0, 0};
+#pragma unroll
+    for (int g = 0; g < 2; ++g) m1[g] = m2[g] = 2.f * kKmExcluded;
     for (int c = 0; c < nchunks; ++c) {
-      if (nchunks > 1) stage(c * p.KC);
-      if (!live) continue;
-      const int kc = min(p.KC, K - c * p.KC);
-      const float xc = xr + cmx[0];
-      const float M = tau2 * (xc * xc);
-      for (int pb = 0; pb < kc; pb += 16 * NT) {
-        f4 acc[NT];
+      if (MULTI) {
+        const float cm = stage(c * p.KC);
+        cmax = __builtin_fmaxf(cmax, cm);
+        if (!live) continue;
+      }
+      const int k0 = c * p.KC;
+      const int ntl = (min(p.KC, K - k0) + 31) >> 5;
+      for (int tl = 0; tl < ntl; tl += 2) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int g = 0; g < 2; ++g) {
+          if (tl + g >= ntl) break;  // wave-uniform
+          const f16v acc = screen_tile(tl + g);
+          const float was = m1[g];
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            const f4 cf = *reinterpret_cast<const f4 *>(cs + (pb + 16 * t + r) * DP + 16 * i + 4 * q);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[t] = mfma4(cf[e], xv[i][e], acc[t]);
+          for (int i = 0; i < 16; ++i) {
+            const float v = __uint_as_float((__float_as_uint(acc[i]) & ~15u) | (uint32_t)i);
+            m2[g] = __builtin_amdgcn_fmed3f(m1[g], m2[g], v);
+            m1[g] = vmax(m1[g], v);
           }
-        }
-        // Screen.  s_k = |c_k|^2 - 2 x.c_k.  The reference's float distance
-        // and |x|^2 + s_k are both within (2D+4) 2^-24 S_k of the exact
-        // distance, S_k = (|x| + |c_k|)^2 + |s_k|, so only centroids with
-        // s_k - m_k <= s_j + m_j for every j, m_k = tau S_k, can be the
-        // reference's argmin.  |s_k| <= (|x| + |c_k|)^2 gives
-        // m_k <= M = tau2 (|x| + max |c|)^2, hence the test
-        // s_k <= min_j (s_j + M) + M, with j over every centroid screened
-        // so far (earlier passes and chunks included).  A NaN s_k, or a NaN
-        // or infinite M, passes.
-        f4 sv[NT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const f4 nrm = *reinterpret_cast<const f4 *>(cn + pb + 16 * t + 4 * q);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sv[t][i] = __builtin_fmaf(-2.f, acc[t][i], nrm[i]);
-        }
-        // the lane's entries 4t + i, centroid pb + 16t + 4q + i, that lie in
-        // the chunk (every one but in a chunk's last, partial pass)
-        uint32_t valid = NT == 8 ? 0xffffffffu : (1u << (4 * NT)) - 1u;
-        if (pb + 16 * NT > kc) {  // wave-uniform
-          valid = 0;
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            const int n = min(max(kc - pb - 16 * t - 4 * q, 0), 4);
-            valid |= ((1u << n) - 1u) << (4 * t);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (i >= n) sv[t][i] = __builtin_inff();  // out of the minimum
-          }
-        }
-        float smin = __builtin_inff();
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) smin = sv[t][i] < smin ? sv[t][i] : smin;
-        {
-          const float o16 = __shfl_xor(smin, 16);
-          smin = o16 < smin ? o16 : smin;
-          const float o32 = __shfl_xor(smin, 32);
-          smin = o32 < smin ? o32 : smin;
-        }
-        const float th = smin + M;
-        thi = th < thi ? th : thi;
-        const float lim = thi + M;
-        uint32_t cand = 0;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) cand |= sv[t][i] > lim ? 0u : 1u << (4 * t + i);
-        cand &= valid;
-        // exact refinement, ascending k within the lane
-        float bd = FLT_MAX;
-        uint32_t bk = kNone;
-        while (cand) {
-          const int b = __builtin_ctz(cand);
-          cand &= cand - 1;
-          const int kl = pb + 16 * (b >> 2) + 4 * q + (b & 3);
-          const float dist = exact_dist<FUSED, NI>(xs + r * DP, cs + kl * DP, nd4);
-          if (dist < bd) {
-            bd = dist;
-            bk = (uint32_t)(c * p.KC + kl);
-          }
-        }
-#pragma unroll
-        for (int off = 16; off < 64; off <<= 1) {
-          const float obd = __shfl_xor(bd, off);
-          const uint32_t obk = (uint32_t)__shfl_xor((int)bk, off);
-          if (obd < bd || (obd == bd && obk < bk)) {
-            bd = obd;
-            bk = obk;
-          }
-        }
-        if (bd < rbd) {  // earlier passes hold smaller k: they keep ties
-          rbd = bd;
-          rbk = bk;
+          bk[g] = m1[g] != was ? k0 + 32 * (tl + g) : bk[g];
         }
       }
     }
-    if (live && q == 0 && row0 + r < p.nrows)
-      p.assign[row0 + r] = rbk == kNone ? (uint32_t)K : rbk;
+
+    // The row's unique candidate, or refinement of the largest value of each
+    // tracker (need) or of every centroid above the limit (full).
+    float lim = 0.f;
+    uint32_t ans = 0;
+    int kc[2] = {0, 0};
+    bool need = false, full = false;
+    if (!MULTI || live) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int id = (int)(__float_as_uint(m1[g]) & 15u);
+        kc[g] = bk[g] + 8 * (id >> 2) + (id & 3) + 4 * h;
+      }
+      const bool odd = m1[1] > m1[0];
+      const float a1 = odd ? m1[1] : m1[0];  // this lane's largest, its other tracker's
+      const float a2 = odd ? m1[0] : m1[1];
+      const float rest = vmax(m2[0], m2[1]);
+      const int k = odd ? kc[1] : kc[0];
+      const float o1 = __shfl_xor(a1, 32), o2 = __shfl_xor(a2, 32), orest = __shfl_xor(rest, 32);
+      const int ok = __shfl_xor(k, 32);
+      const float s1 = vmax(a1, o1);
+      const float unnamed = vmax(rest, orest);  // every value that no tracker names is below
+      const float s2 = vmax(vmax(unnamed, o1 < a1 ? o1 : a1), vmax(a2, o2));
+      const float xc = __builtin_sqrtf(xx) + cmax;
+      const float M = __builtin_fmaf(tau, xc * xc, 0x1p-100f);
+      // small enough that no distance overflows and excluded centroids are
+      // farther (false for NaN)
+      const bool range = xx < kKmRowMax && xx - 2.f * s1 < kKmRowMax;
+      ans = (uint32_t)(o1 > a1 ? ok : k);
+      need = row0 + r < p.nrows && !(range && s1 - s2 > M);
+      full = need && !(range && s1 - unnamed > M);
+      lim = range ? s1 - M : -__builtin_inff();
+    }
+    const bool any_need = __any(need), any_full = __any(full);
+
+    // Reference distances of the candidates, the two lanes of a row their
+    // own; equal distances go to the smaller index (the reference's first
+    // strict minimum).
+    float bd = FLT_MAX;
+    uint32_t bi = kNone;
+    auto refine = [&](int k) {
+      const float dist = exact_dist<FUSED, KS>(p.rows + (row0 + r) * D, p.ctrds + (int64_t)k * D, D);
+      if (dist < bd || (dist == bd && bi != kNone && (uint32_t)k < bi)) {
+        bd = dist;
+        bi = (uint32_t)k;
+      }
+    };
+    if (any_need) {
+      uint32_t cand = need && !full ? (m1[0] >= lim ? 1u : 0u) | (m1[1] >= lim ? 2u : 0u) : 0u;
+      while (cand) {
+        const bool g0 = cand & 1u;
+        cand &= cand - 1;
+        refine(g0 ? kc[0] : kc[1]);
+      }
+    }
+    if (MULTI ? (bool)__syncthreads_or(any_full) : any_full) {
+#pragma unroll 1
+      for (int c = 0; c < nchunks; ++c) {
+        if (MULTI) {
+          stage(c * p.KC);
+          if (!any_full) continue;
+        }
+        const int k0 = c * p.KC;
+        const int ntl = (min(p.KC, K - k0) + 31) >> 5;
+#pragma unroll 1
+        for (int tl = 0; tl < ntl; ++tl) {
+          const f16v acc = screen_tile(tl);
+          uint32_t cand = 0;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) cand |= full && !(acc[i] < lim) ? 1u << i : 0u;
+          while (cand) {
+            const int b = __builtin_ctz(cand);
+            cand &= cand - 1;
+            const int k = k0 + 32 * tl + 8 * (b >> 2) + 4 * h + (b & 3);
+            if (k < K) refine(k);
+          }
+        }
+      }
+    }
+    if (any_need) {
+      const float od = __shfl_xor(bd, 32);
+      const uint32_t oi = (uint32_t)__shfl_xor((int)bi, 32);
+      if (od < bd || (od == bd && oi < bi)) bi = oi;
+      if (need) ans = bi == kNone ? (uint32_t)K : bi;
+    }
+    if ((!MULTI || live) && h == 0 && row0 + r < p.nrows) p.assign[row0 + r] = ans;
   }
 }
 
@@ -439,27 +593,18 @@ KmKernel kmd_kernel(int d, bool fused) {
   return kmd_find(d, fused, std::make_integer_sequence<int, kKmDirectMaxDims>{});
 }
 
-template <int NI, int NT>
-KmKernel km_pick(bool fused) {
-  return fused ? k_kmeans_assign<NI, NT, true> : k_kmeans_assign<NI, NT, false>;
+template <int KS, bool FUSED>
+KmKernel kms_pick(bool multi, bool vec) {
+  if (multi) return vec ? k_kmeans_screen<KS, true, true, FUSED> : k_kmeans_screen<KS, true, false, FUSED>;
+  return vec ? k_kmeans_screen<KS, false, true, FUSED> : k_kmeans_screen<KS, false, false, FUSED>;
 }
 
-template <int NI>
-KmKernel km_pick_nt(int nt, bool fused) {
-  switch (nt) {
-    case 1: return km_pick<NI, 1>(fused);
-    case 2: return km_pick<NI, 2>(fused);
-    case 4: return km_pick<NI, 4>(fused);
-    default: return km_pick<NI, 8>(fused);
-  }
-}
-
-KmKernel km_kernel(int ni, int nt, bool fused) {
-  switch (ni) {
-    case 1: return km_pick_nt<1>(nt, fused);
-    case 2: return km_pick_nt<2>(nt, fused);
-    case 3: return km_pick_nt<3>(nt, fused);
-    default: return km_pick_nt<4>(nt, fused);
+KmKernel kms_kernel(int ks, bool multi, bool vec, bool fused) {
+  switch (ks) {
+    case 1: return fused ? kms_pick<1, true>(multi, vec) : kms_pick<1, false>(multi, vec);
+    case 2: return fused ? kms_pick<2, true>(multi, vec) : kms_pick<2, false>(multi, vec);
+    case 3: return fused ? kms_pick<3, true>(multi, vec) : kms_pick<3, false>(multi, vec);
+    default: return fused ? kms_pick<4, true>(multi, vec) : kms_pick<4, false>(multi, vec);
   }
 }
 
@@ -475,12 +620,16 @@ int cu_count() {
 
 KmeansPlan plan_kmeans(int64_t nrows, int D, int K, int mode) {
   KmeansPlan pl;
-  // measured on MI355X (2^24 rows, dims 4..32 x clusters 4..1024): the
-  // direct kernel wins up to 8 dims at any cluster count and below
-  // clusters x dims = 1024 up to 32 dims (by up to 9x at few clusters);
-  // the screened kernel wins above
+  // The direct kernel's time grows with dims x clusters from the row stream
+  // up, the screened one's starts at the cost of splitting the rows and
+  // barely grows.  Measured on MI355X over 2^21 rows, dims 2..32 x clusters
+  // 2..128 (screened / direct, us): 5 x 32 32.5 / 33.7, 8 x 24 31.9 / 29.4,
+  // 8 x 32 32.1 / 36.8, 16 x 12 32.5 / 35.3, 24 x 8 44.8 / 38.2, 24 x 12
+  // 44.9 / 45.6, 32 x 8 49.8 / 47.7, 32 x 12 50.2 / 57.8; 4 x 8 30.6 / 11.8
+  // and 16 x 128 58.7 / 219 far from the line.  They cross between 180 and
+  // 290 for every row length.
   pl.direct = (mode == 2 && D <= kKmDirectMaxDims) ||
-              (mode == 0 && D <= kKmDirectMaxDims && (D <= 8 || (int64_t)K * D < 1024));
+              (mode == 0 && D <= kKmDirectMaxDims && (int64_t)K * D < kKmDirectWork);
   if (pl.direct) {
     // one row per lane; centroids in chunks of at most kKmDirectLdsBytes,
     // plus each wave's 64-row area
@@ -495,20 +644,16 @@ KmeansPlan plan_kmeans(int64_t nrows, int D, int K, int mode) {
     return pl;
   }
   pl.ni = (D + 15) / 16;
-  pl.nt = K <= 16 ? 1 : K <= 32 ? 2 : K <= 64 ? 4 : 8;
-  const int dp = 16 * pl.ni + 4;
-  const int pass = 16 * pl.nt;
-  // LDS: centroid chunk (KC x dp) + squared norms (KC) + the chunk's
-  // largest norm (4 floats, keeping 16-byte alignment) + 16 rows per wave,
-  // at most kKmLdsBytes.
-  const int64_t rows_f = (int64_t)kKmWaves * 16 * dp;
-  const int64_t room = kKmLdsBytes / 4 - rows_f - 4;
-  int64_t kc = room / (dp + 1) / pass * pass;
-  const int64_t kpad = ((int64_t)K + pass - 1) / pass * pass;
-  if (kc > kpad) kc = kpad;
-  pl.KC = (int)kc;
-  pl.lds = (size_t)(kc * (dp + 1) + 4 + rows_f) * 4;
-  pl.tiles = (nrows + 15) / 16;
+  const int64_t kpad = ((int64_t)K + 31) / 32 * 32;
+  // LDS: per centroid 64 ni bytes of bf16 terms and its norm, each wave's
+  // row tile in whole 1 KB loads, 256 bytes that reads past the last tile's
+  // last row may touch, and 256 for the workgroup vote
+  pl.xfloats = (D + 7) / 8 * 256;
+  const int64_t rows_b = (int64_t)kKmWaves * pl.xfloats * 4 + 256;
+  const int64_t room = (int64_t)kKmLdsBytes - 256 - rows_b;
+  pl.KC = (int)std::min<int64_t>(kpad, room / (64 * pl.ni + 4) / 32 * 32);
+  pl.lds = (size_t)(pl.KC * (64 * pl.ni + 4) + rows_b);
+  pl.tiles = (nrows + 31) / 32;
   return pl;
 }
 
@@ -516,8 +661,9 @@ hipError_t launch_kmeans_assign(const KmeansPlan &pl, uint32_t *assign, const fl
                                 int64_t nrows, int D, const float *ctrds, int K, bool fused,
                                 hipStream_t st) {
   if (nrows <= 0) return hipSuccess;
-  if (pl.direct ? pl.KC < 1 : pl.KC < 16 * pl.nt) return hipErrorInvalidValue;
-  KmKernel fn = pl.direct ? kmd_kernel(pl.ni, fused) : km_kernel(pl.ni, pl.nt, fused);
+  if (pl.direct ? pl.KC < 1 : pl.KC < 32) return hipErrorInvalidValue;
+  KmKernel fn = pl.direct ? kmd_kernel(pl.ni, fused)
+                          : kms_kernel(pl.ni, pl.KC < K, D % 4 == 0, fused);
   if (!fn) return hipErrorInvalidValue;
   const int waves = pl.direct ? kKmDirectWaves : kKmWaves;
   hipError_t e;
@@ -543,6 +689,7 @@ hipError_t launch_kmeans_assign(const KmeansPlan &pl, uint32_t *assign, const fl
   p.D = D;
   p.K = K;
   p.KC = pl.KC;
+  p.xfloats = pl.xfloats;
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(64 * waves), pl.lds, st, p);
   return hipGetLastError();
 }

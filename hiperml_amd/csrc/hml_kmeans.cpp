@@ -33,7 +33,7 @@ extern "C" hmlStatus hmlKmeansAssign(uint32_t *assign, const float *rows, int64_
     return fail(HML_STATUS_UNSUPPORTED, "kmeans assign: the direct kernel takes at most %d dims",
                 kKmDirectMaxDims);
   const KmeansPlan pl = plan_kmeans(numRows, numDims, numClusts, mode);
-  if (pl.direct ? pl.KC < 1 : pl.KC < 16 * pl.nt)
+  if (pl.direct ? pl.KC < 1 : pl.KC < 32)
     return fail(HML_STATUS_UNSUPPORTED, "kmeans assign: no LDS chunk for %d dims", numDims);
   hipError_t e = launch_kmeans_assign(pl, assign, rows, numRows, numDims, ctrds, numClusts,
                                       !(flags & HML_KMEANS_SEPARATE_ROUNDING),

@@ -167,3 +167,34 @@ def test_centroid_scales(hml):
             for kern in kernels(D):
                 np.testing.assert_array_equal(run(hml, rows, ctrds, kernel=kern), want,
                                               err_msg="inf/nan %s kernel=%s" % (make.__name__, kern))
+
+
+def integer_grid(rng, n, D, K):
+    """Small whole numbers: many rows equidistant from several centroids."""
+    ctrds = rng.integers(-2, 3, (K, D)).astype(np.float32)
+    return rng.integers(-2, 3, (n, D)).astype(np.float32), ctrds
+
+
+@pytest.mark.parametrize("D", [2, 15, 16, 18, 33, 47, 60, 64])
+@pytest.mark.parametrize("K", [1, 31, 32, 33, 64, 65, 97])
+def test_screen_edges(hml, D, K):
+    """The screened kernel at the edges of its 32-row and 32-centroid tiles
+    and 16-dim steps, where the screen decides alone (clustered rows), where
+    trackers or a second screening decide (near ties, whole-number grids),
+    and at scales where squares overflow, underflow or leave the screen's
+    range, with centroids padded by FLT_MAX / 2."""
+    rng = np.random.default_rng(100 * D + K)
+    for n in (1, 31, 32, 33, 8 * 32 + 5):
+        for make in (clustered, near_ties, integer_grid):
+            rows, ctrds = make(rng, n, D, K)
+            want = oracle.kmeans_assign(rows, ctrds)
+            got = run(hml, rows, ctrds, kernel="screened", offset=n % 3)
+            np.testing.assert_array_equal(got, want, err_msg="%s n=%d" % (make.__name__, n))
+    rows, ctrds = clustered(rng, 70, D, K)
+    pad = np.full((5, D), 3.4028235e38 / 2, np.float32)
+    for scale in (1e-30, 1e-19, 1e15, 3e17, 2e18, 1e19, 1e30):
+        r, c = (rows * np.float32(scale)), (ctrds * np.float32(scale))
+        for cc in (c, np.concatenate([c, pad])):
+            want = oracle.kmeans_assign(r, cc)
+            got = run(hml, r, cc, kernel="screened")
+            np.testing.assert_array_equal(got, want, err_msg="scale %g" % scale)
