@@ -436,7 +436,7 @@ hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
     p.kchunk = pl.kchunk; p.kgroups = pl.ksplit;
     p.nct_pad = pl.nct_pad;
     p.alpha = alpha; p.beta = beta; p.read_c = read_c;
-    e = launch_skinny_axpy(v.rt, v.ct, g.M % 4 == 0, g.sBk == 1 || g.K == 1, pl.kw, p, st);
+    e = launch_skinny_axpy(v.rt, v.ct, g.sBk == 1 || g.K == 1, pl.kw, p, st);
   }
   if (e != hipSuccess) return from_hip(e, "skinny kernel launch");
   if (pl.ksplit > 1) {

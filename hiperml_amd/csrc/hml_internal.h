@@ -84,10 +84,10 @@ hipError_t launch_gemv_multi(int lpr, int rb, int nv, bool bvec, int wpb, const 
 // AXPY-form skinny SGEMM (hml_k_skinny.hip, k_skinny_axpy): B read in
 // place, K split over the kw waves of a workgroup and summed there; kgroups
 // > 1 splits K further over workgroups (partials in P, summed by
-// launch_reduce with R = kgroups).  vec: M % 4 == 0; bvec: sBk == 1.
+// launch_reduce with R = kgroups).  bvec: sBk == 1.
 // Returns hipErrorInvalidValue when (rt, ct, kw) has no instantiation.
-hipError_t launch_skinny_axpy(int rt, int ct, bool vec, bool bvec, int kw,
-                              const SkinnyParams &p, hipStream_t st);
+hipError_t launch_skinny_axpy(int rt, int ct, bool bvec, int kw, const SkinnyParams &p,
+                              hipStream_t st);
 bool skinny_axpy_runnable(int rt, int ct, int kw);
 bool skinny_has_variant(int form, int rt, int ct);
 

@@ -519,8 +519,13 @@ __global__ __launch_bounds__(64 * kGroupWaveWpb, 2) void k_grouped_dot(const Gro
 // A lane offset of kOOB returns zero without touching memory: rows past M,
 // columns past N and k past the chunk end.  Steps past the chunk load
 // through a descriptor of size 0, so the pipeline needs no guarded drain.
-// VEC (M % 4 == 0): a lane's 4 rows are all in range or all out, one 16-byte
-// load; otherwise 4 scalar loads, each row checked on its own.
+// VEC: a lane's 4 rows are one 16-byte load (any 4-byte alignment).  With M
+// not a multiple of 4 the lane that crosses row M reads on into the next
+// column (sAk >= 4), and what it finds feeds only rows past M, which are not
+// stored; the step that holds the last column, where that would leave A,
+// takes the element loads of a partial step.  With four scalar loads for every
+// lane, odd M was bound by load instructions: A^T B of 5003 x 24 x 9001 106
+// us, now 49; 8191 x 64 x 8191 130, now 84; 3001 x 100 x 20000 323, now 160.
 // ---------------------------------------------------------------------------
 // register stages of loads in flight, and workgroup size limit, per shape
 __host__ __device__ constexpr int axpy_stages(int rt, int ct) {
@@ -545,7 +550,7 @@ __device__ __forceinline__ void store_out(const SkinnyParams &p, int64_t row,
   }
 }
 
-template <int RT, int CT, bool VEC, bool BVEC>
+template <int RT, int CT, bool VEC, bool BVEC, int APOL>
 __global__ __launch_bounds__(64 * axpy_max_waves(RT, CT)) void k_skinny_axpy(SkinnyParams p) {
   constexpr int PS = axpy_stages(RT, CT);
   extern __shared__ f4 axpy_lds[];
@@ -563,7 +568,9 @@ __global__ __launch_bounds__(64 * axpy_max_waves(RT, CT)) void k_skinny_axpy(Ski
   const int64_t kb = ((int64_t)kgi * kw + w) * p.kchunk;
   int64_t ke = kb + p.kchunk;
   if (ke > p.K) ke = p.K;
-  const int64_t nfull = ke > kb ? (ke - kb) / kAxpyKStep : 0;
+  const bool ragged = VEC && (p.M & 3);
+  // (the step that holds column K - 1 is not a full one when ragged)
+  const int64_t nfull = ke > kb ? (ke - kb - (ragged && ke == p.K ? 1 : 0)) / kAxpyKStep : 0;
 
   // lane offsets (bytes) from a step's descriptor bases
   uint32_t aoff[RT][VEC ? 1 : 4];
@@ -603,10 +610,10 @@ __global__ __launch_bounds__(64 * axpy_max_waves(RT, CT)) void k_skinny_axpy(Ski
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
         if (VEC) {
-          a[j][t][u] = buf_load4<kBufNT>(ra, aoff[t][0], so);
+          a[j][t][u] = buf_load4<APOL>(ra, aoff[t][0], so);
         } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) a[j][t][u][e] = buf_load1<kBufNT>(ra, aoff[t][e], so);
+          for (int e = 0; e < 4; ++e) a[j][t][u][e] = buf_load1<APOL>(ra, aoff[t][e], so);
         }
       }
     }
@@ -656,12 +663,15 @@ __global__ __launch_bounds__(64 * axpy_max_waves(RT, CT)) void k_skinny_axpy(Ski
       const int32_t so = (int32_t)(u * p.sAk * 4);
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
-        if (VEC) {
-          a[0][t][u] = buf_load4<kBufNT>(ra, kin ? aoff[t][0] : kOOB, so);
+        if (VEC && !ragged) {
+          a[0][t][u] = buf_load4<APOL>(ra, kin ? aoff[t][0] : kOOB, so);
         } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            a[0][t][u][e] = buf_load1<kBufNT>(ra, kin ? aoff[t][e] : kOOB, so);
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t o = !VEC ? aoff[t][e]
+                               : m0 + 64 * t + 4 * r + e < p.M ? aoff[t][0] + 4 * e : kOOB;
+            a[0][t][u][e] = buf_load1<APOL>(ra, kin ? o : kOOB, so);
+          }
         }
       }
 #pragma unroll
@@ -1151,27 +1161,35 @@ int resident_blocks(const void *fn, size_t lds, int threads = 256) {
   return std::max(1, nb) * prop.multiProcessorCount;
 }
 
-template <int RT, int CT, bool VEC, bool BVEC>
+template <int RT, int CT, bool VEC, bool BVEC, int APOL>
 hipError_t run_axpy(int kw, const SkinnyParams &p, hipStream_t st) {
   const int64_t rows = (int64_t)kAxpyRowsPerTile * RT;
   const int64_t nblk = ((p.M + rows - 1) / rows) * p.kgroups;
   const int64_t ncb = p.nct_pad / CT;
   if (nblk > 0x7fffffff || ncb > 65535) return hipErrorInvalidConfiguration;
   const size_t lds = kw > 1 ? (size_t)kw * kAxpyRedGroups * 64 * sizeof(f4) : 0;
-  hipLaunchKernelGGL((k_skinny_axpy<RT, CT, VEC, BVEC>), dim3((unsigned)nblk, (unsigned)ncb),
+  hipLaunchKernelGGL((k_skinny_axpy<RT, CT, VEC, BVEC, APOL>), dim3((unsigned)nblk, (unsigned)ncb),
                      dim3(64 * kw), lds, st, p);
   return hipGetLastError();
 }
 
 typedef hipError_t (*RunFn)(int, const SkinnyParams &, hipStream_t);
 
-template <int RT, int CT>
-constexpr RunFn axpy_fn(bool vec, bool bvec) {
-  return vec ? (bvec ? run_axpy<RT, CT, true, true> : run_axpy<RT, CT, true, false>)
-             : (bvec ? run_axpy<RT, CT, false, true> : run_axpy<RT, CT, false, false>);
+// vec 0: element loads of A; 1: 16-byte loads, non-temporal; 2: 16-byte
+// loads, cached
+template <int RT, int CT, bool BVEC>
+constexpr RunFn axpy_fn(int vec) {
+  return vec == 0   ? run_axpy<RT, CT, false, BVEC, 0>
+         : vec == 1 ? run_axpy<RT, CT, true, BVEC, kBufNT>
+                    : run_axpy<RT, CT, true, BVEC, 0>;
 }
 
-RunFn find_axpy(int rt, int ct, bool vec, bool bvec) {
+template <int RT, int CT>
+constexpr RunFn axpy_fn(int vec, bool bvec) {
+  return bvec ? axpy_fn<RT, CT, true>(vec) : axpy_fn<RT, CT, false>(vec);
+}
+
+RunFn find_axpy(int rt, int ct, int vec, bool bvec) {
   // 2 x 64 rows x 128 columns would spill: no (2, 8) tile
   switch (rt * 16 + ct) {
     case 17: return axpy_fn<1, 1>(vec, bvec);
@@ -1189,7 +1207,7 @@ RunFn find_axpy(int rt, int ct, bool vec, bool bvec) {
 
 bool skinny_has_variant(int form, int rt, int ct) {
   if (form == kFormDot) return find_dot(rt, ct, true) != nullptr;
-  return find_axpy(rt, ct, true, true) != nullptr;
+  return find_axpy(rt, ct, 1, true) != nullptr;
 }
 
 size_t skinny_dot_lds_bytes(int rt, int ct, int kw) {
@@ -1244,15 +1262,22 @@ hipError_t launch_skinny_dotb(int rt, int ct, bool bvec, const DotParams &p, hip
 }
 
 bool skinny_axpy_runnable(int rt, int ct, int kw) {
-  return find_axpy(rt, ct, true, true) != nullptr && kw >= 1 && kw <= axpy_max_waves(rt, ct) &&
+  return find_axpy(rt, ct, 1, true) != nullptr && kw >= 1 && kw <= axpy_max_waves(rt, ct) &&
          (kw & (kw - 1)) == 0;
 }
 
-hipError_t launch_skinny_axpy(int rt, int ct, bool vec, bool bvec, int kw,
-                              const SkinnyParams &p, hipStream_t st) {
+hipError_t launch_skinny_axpy(int rt, int ct, bool bvec, int kw, const SkinnyParams &p,
+                              hipStream_t st) {
   if (!skinny_axpy_runnable(rt, ct, kw) || p.nct_pad % ct != 0 || p.kgroups < 1 ||
       p.kchunk % kAxpyKStep != 0)
     return hipErrorInvalidValue;
+  // Element loads only where a lane that crosses row M could reach past the
+  // next column (M <= 3).  Columns that do not start on 128-byte lines share
+  // a line between neighbouring row tiles, so they are read through the
+  // caches (20001 x 100 x 3000: 149 us, non-temporally 160); aligned ones
+  // stream better non-temporally (8192 x 2 x 8192: 65 against 71 us).
+  const bool aligned = (uintptr_t)p.A % 128 == 0 && (p.sAk * 4) % 128 == 0;
+  const int vec = p.M % 4 != 0 && p.sAk < 4 ? 0 : aligned ? 1 : 2;
   return find_axpy(rt, ct, vec, bvec)(kw, p, st);
 }
 

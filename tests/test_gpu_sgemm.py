@@ -477,3 +477,28 @@ def test_axpy_large_stride_offsets(hml):
         dA.free()
         dB.free()
         dC.free()
+
+
+@pytest.mark.parametrize("M", [2, 3, 5, 6, 7, 63, 65, 66, 67, 127, 129, 254])
+@pytest.mark.parametrize("K", [2, 15, 16, 17, 32, 48, 100, 321])
+def test_axpy_ragged_rows(hml, M, K):
+    """A contiguous along M with M not a multiple of 4: the lanes that cross
+    row M read the gap between columns (NaN here), which must not reach C,
+    for leading dimensions equal to M and larger, whole and partial last
+    steps, one and several waves and K groups."""
+    rng = np.random.default_rng(1000 * M + K)
+    for pad, N in ((0, 1), (1, 2), (3, 17), (8, 33)):
+        if N > M:
+            continue
+        A, B, C0 = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
+        As = np.full((K, M + pad), np.nan, np.float32)
+        As[:, :M] = A.T
+        tail = np.full(64, np.nan, np.float32)  # past the last column
+        dA = hml.DeviceBuffer.from_numpy(np.concatenate([As.ravel(), tail]))
+        dB = hml.DeviceBuffer.from_numpy(B)
+        R = exact_product(A, B, 2.0, -1.0, C0)
+        for v in ((2, 1, 1, 1, 1), (2, 1, 2, 1, 1), (2, 2, 1, 4, 4), (2, 1, 4, 8, 2)):
+            dC = hml.DeviceBuffer.from_numpy(C0)
+            hml.sgemm_ex(M, N, K, dA, dB, dC, 2.0, -1.0, transA=True, lda=M + pad, variant=v)
+            hml.synchronize()
+            np.testing.assert_array_equal(dC.to_numpy((M, N)), R, err_msg="N=%d %r" % (N, v))
