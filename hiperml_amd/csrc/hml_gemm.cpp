@@ -365,7 +365,7 @@ hmlStatus run_dense_fallback(const GemmCanon &g, const GemmKey &k, float alpha, 
 }
 
 hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
-                    const hmlSgemmVariant &v, float alpha, float beta,
+                    const hmlSgemmVariant &v, bool chosen, float alpha, float beta,
                     int read_c, void *ws, size_t ws_bytes, hipStream_t st) {
   const size_t need = workspace_bytes(k, v);
   void *const caller_ws = ws;
@@ -378,6 +378,21 @@ hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
   } else if (need > ws_bytes) {
     return fail(HML_STATUS_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes",
                 ws_bytes, need);
+  }
+  // A chosen (not named) DOT-form variant gives way to the row-streaming
+  // kernel where that one is better.
+  if (chosen && k.form == kFormDot &&
+      (v.family == HML_SGEMM_FAMILY_DOT || v.family == HML_SGEMM_FAMILY_DOTB ||
+       v.family == HML_SGEMM_FAMILY_GEMVN) &&
+      skinny_rows_better(g.M, g.N, g.K, g.sAm)) {
+    DotParams p{};
+    p.A = g.A; p.sAm = g.sAm;
+    p.B = g.B; p.sBk = g.sBk; p.sBn = g.sBn;
+    p.C = g.C; p.sCm = g.sCm; p.sCn = g.sCn;
+    p.M = g.M; p.N = g.N; p.K = g.K;
+    p.kgroups = 1;
+    p.alpha = alpha; p.beta = beta; p.read_c = read_c;
+    return from_hip(launch_skinny_rows(p, st), "row-streaming kernel launch");
   }
   if (v.family == HML_SGEMM_FAMILY_GEMV)
     return run_gemv_family(g, k, v, alpha, beta, read_c, ws, st);
@@ -502,7 +517,7 @@ hmlStatus sgemm_impl(hmlOrder order, hmlOp ta, hmlOp tb, int64_t M, int64_t N,
     select_sgemm(key, &v, &src);
   }
   if (used) *used = v;
-  return run_sgemm(g, key, v, alpha, beta, read_c, ws, ws_bytes, st);
+  return run_sgemm(g, key, v, !forced, alpha, beta, read_c, ws, ws_bytes, st);
 }
 
 // Host-pointer compatibility path (src/hml_sgemm.cu:39-113,120-211).

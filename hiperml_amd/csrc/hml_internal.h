@@ -145,6 +145,15 @@ hipError_t launch_skinny_dotb(int rt, int ct, bool bvec, const DotParams &p, hip
 hipError_t launch_skinny_dot(int rt, int ct, bool bvec, int kw, const DotParams &p,
                              hipStream_t st);
 
+// k_skinny_rows: unsplit products of few k and many rows, rows streamed by
+// persistent waves.  `better` is the rule that sends a problem there.
+constexpr int kRowsWaves = 8;  // most waves per workgroup
+constexpr int kRowsMaxK = 128, kRowsMaxN = 128;
+constexpr int64_t kRowsMaxLda = 1 << 23;  // 16 rows within 31-bit offsets
+constexpr int64_t kRowsMinM = 1 << 16;
+bool skinny_rows_better(int64_t M, int64_t N, int64_t K, int64_t lda);
+hipError_t launch_skinny_rows(const DotParams &p, hipStream_t st);
+
 // out(m,n) = alpha * sum_r P[r*total + m*ninner + n] + beta * out(m,n)
 hipError_t launch_reduce(const float *P, int R, int64_t total, int64_t ninner,
                          float *C, int64_t sCm, int64_t sCn, float alpha,

@@ -424,6 +424,170 @@ __global__ __launch_bounds__(64 * dot_max_waves(RT, CT)) void k_skinny_dot(DotPa
 }
 
 // ---------------------------------------------------------------------------
+// Short rows: k_skinny_rows, for DOT-form problems with few k and many rows,
+// where k_skinny_dot's one or two stages per wave leave nothing to pipeline:
+// a wave loaded a tile, waited, loaded B, waited, and stored 4-byte elements.
+//
+// Persistent waves stream tiles of 16 rows.  A tile is one contiguous block
+// of memory when lda == K and goes flat into the wave's LDS area by LDS DMA,
+// the next tile's load in flight while this one is multiplied; with VEC (K a
+// multiple of 4) any lda works, and row x's 16-byte chunk c sits at chunk x
+// nc + (c + x nc / 16) % nc (nc = K / 4), which spreads the operand reads of
+// 8 consecutive rows over distinct banks.  All of B lives in LDS in operand
+// order (one conflict-free 16-byte read per lane for 16 k of a column tile),
+// staged once per workgroup.  The MFMA takes B as its first operand, so a
+// lane ends with 4 consecutive columns of one row: 16-byte stores where C's
+// columns are contiguous.  The k order within and across MFMAs is that of
+// an unsplit k_skinny_dot: both give the same bits.
+//
+// Bound by the streams of A and C.  Measured on 10^6 rows, N x K (us, before
+// -> now): 16 x 31 77 -> 35, 32 x 48 112 -> 60 (5.3 TB/s), 64 x 64 168 -> 112,
+// 96 x 96 482 -> 269.  32-row tiles were no faster at any of them.
+// ---------------------------------------------------------------------------
+constexpr int kWaitAll = 0x0070;            // vmcnt(0) lgkmcnt(0)
+constexpr int kRowsQ = kRowsMaxK / 16;      // 1 KB loads of a tile at the largest K
+struct __attribute__((packed, aligned(4))) RowQuad {
+  float v[4];
+};
+
+template <int CT, bool VEC>
+__global__ __launch_bounds__(64 * kRowsWaves, 4) void k_skinny_rows(DotParams p) {
+  extern __shared__ f4 rows_lds[];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kw = blockDim.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int K = (int)p.K, N = (int)p.N;
+  const int nks = (K + 15) >> 4, nct = (N + 15) >> 4;
+  const int nc = K >> 2;                // VEC: 16-byte chunks per row
+  const int nchunk = 4 * K;             // 16-byte chunks of a tile
+  const int nq = (nchunk + 63) >> 6;    // 1 KB loads of a tile
+  f4 *bf = rows_lds;                    // B: (16 k, column tile, lane, 4 k)
+  float *xs = reinterpret_cast<float *>(bf + (size_t)nks * nct * 64) + (size_t)w * nq * 256;
+
+  const int64_t tiles = (p.M + 15) / 16;
+  const int64_t wstep = (int64_t)gridDim.x * kw;
+  int64_t tile = (int64_t)blockIdx.x * kw + w;
+  uint32_t aoff[kRowsQ];  // lane offsets of the tile's loads
+#pragma unroll
+  for (int q = 0; q < kRowsQ; ++q) {
+    const int pos = 64 * q + lane;
+    uint32_t o = (uint32_t)pos * 16u;
+    if (VEC) {
+      const int x = pos / nc, sl = pos - x * nc;
+      int c = sl - ((x * nc) >> 4) % nc;
+      if (c < 0) c += nc;
+      o = (uint32_t)((x * p.sAm + 4 * c) * 4);
+    }
+    aoff[q] = pos < nchunk ? o : kOOB;
+  }
+  auto load_rows = [&](int64_t tl) {
+    const int64_t row0 = tl * 16;
+    if (row0 >= p.M) return;
+    const float *base = p.A + row0 * p.sAm;
+    if (row0 + 16 <= p.M) {
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(base, (int32_t)((15 * p.sAm + K) * 4));
+#pragma unroll
+      for (int q = 0; q < kRowsQ; ++q)
+        if (q < nq) buf_load_lds16<kBufNT>(rs, xs + 256 * q, aoff[q], 0);
+    } else {
+      // the last, partial tile: element by element
+      const int n = (int)(p.M - row0) * K;
+      for (int i = lane; i < n; i += 64) {
+        const int x = i / K, k = i - x * K;
+        const int o = VEC ? 4 * (x * nc + ((k >> 2) + ((x * nc) >> 4)) % nc) + (k & 3) : i;
+        xs[o] = base[x * p.sAm + k];
+      }
+    }
+  };
+  auto wave_sync = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  load_rows(tile);
+
+  for (int i = threadIdx.x; i < nks * nct * 64; i += blockDim.x) {
+    const int l = i & 63, t = i >> 6, c = t % nct, j = t / nct;
+    const int n = 16 * c + (l & 15), k = 16 * j + 4 * (l >> 4);
+    f4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[e] = n < N && k + e < K ? p.B[(k + e) * p.sBk + n * p.sBn] : 0.f;
+    bf[i] = v;
+  }
+  __syncthreads();
+
+  const int xb = r * nc, xr = VEC ? (xb >> 4) % nc : 0;  // row r: first chunk, rotation
+  for (; tile < tiles; tile += wstep) {
+    const int64_t row = tile * 16 + r;
+    __builtin_amdgcn_s_waitcnt(kWaitAll);  // the tile is in LDS
+    __builtin_amdgcn_sched_barrier(0);
+    wave_sync();
+    for (int c0 = 0; c0 < nct; c0 += CT) {
+      f4 acc[CT];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[c] = f4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < nks; ++j) {
+        // lane (g, r): row r, k = 16 j + 4 g .. +3 (zero past K)
+        f4 a, b[CT];
+        if (VEC) {
+          const int c = 4 * j + g;
+          int o = xr + (c < nc ? c : 0);
+          o = o >= nc ? o - nc : o;
+          a = *reinterpret_cast<const f4 *>(xs + 4 * (xb + o));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a[e] = xs[r * K + 16 * j + 4 * g + e];
+        }
+        if (j + 1 == nks) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a[e] = 16 * j + 4 * g + e < K ? a[e] : 0.f;
+        }
+#pragma unroll
+        for (int c = 0; c < CT; ++c) b[c] = bf[(j * nct + (c0 + c < nct ? c0 + c : c0)) * 64 + lane];
+        if (j + 1 == nks && c0 + CT >= nct) {
+          // the tile's last reads: its area takes the next one
+          wave_sync();
+          __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+          __builtin_amdgcn_sched_barrier(0);
+          load_rows(tile + wstep);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int c = 0; c < CT; ++c) acc[c] = mfma4(b[c][e], a[e], acc[c]);
+      }
+      // lane (g, r): row r, columns 16 (c0 + c) + 4 g .. +3
+      if (row < p.M) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          const int n = 16 * (c0 + c) + 4 * g;
+          float *cp = p.C + row * p.sCm + n * p.sCn;
+          if (p.sCn == 1 && n + 3 < N) {
+            RowQuad o;
+            if (p.read_c) o = *reinterpret_cast<const RowQuad *>(cp);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              o.v[e] = p.read_c ? p.alpha * acc[c][e] + p.beta * o.v[e] : p.alpha * acc[c][e];
+            *reinterpret_cast<RowQuad *>(cp) = o;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (n + e < N) {
+                float v = p.alpha * acc[c][e];
+                if (p.read_c) v = p.alpha * acc[c][e] + p.beta * cp[e * p.sCn];
+                cp[e * p.sCn] = v;
+              }
+          }
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Persistent grouped SGEMM: hundreds of independent skinny problems in one
 // graph launch.  The host sorts the problems into tile classes by N (1, 2
 // or 4 column tiles of 16 per pass), builds one descriptor per problem and,
@@ -1148,6 +1312,17 @@ DotbFn find_dotb(int rt, int ct, bool bv) {
   }
 }
 
+// Compute units of the current device (256 if unknown).
+int device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  return n > 0 ? n : 256;
+}
+
 // Workgroups (256 threads, dynamic LDS `lds`) of kernel `fn` the current
 // device holds at once, from the occupancy calculator; 0 if unknown.
 int resident_blocks(const void *fn, size_t lds, int threads = 256) {
@@ -1259,6 +1434,64 @@ hipError_t launch_skinny_dotb(int rt, int ct, bool bvec, const DotParams &p, hip
   if (!skinny_dotb_runnable(rt, ct) || p.kgroups < 1 || p.kchunk % kDotStageK != 0)
     return hipErrorInvalidValue;
   return find_dotb(rt, ct, bvec)(p, st);
+}
+
+namespace {
+// B fragments and w row tiles; element reads of a tile may run 64 bytes on
+size_t rows_lds_bytes(int w, int64_t N, int64_t K) {
+  const int64_t nks = (K + 15) / 16, nct = (N + 15) / 16;
+  return (size_t)(nks * nct + w * nks) * 1024 + (K % 4 == 0 ? 0 : 64);
+}
+
+template <bool VEC>
+const void *rows_fn(int ct) {
+  switch (ct) {
+    case 1: return (const void *)k_skinny_rows<1, VEC>;
+    case 2: return (const void *)k_skinny_rows<2, VEC>;
+    case 3: return (const void *)k_skinny_rows<3, VEC>;
+    default: return (const void *)k_skinny_rows<4, VEC>;
+  }
+}
+}  // namespace
+
+// Few k, many rows.  Below about 2^16 rows there is one tile per wave or
+// none, and staging B per workgroup costs more than it saves (us, k_skinny_dot
+// / this; 30000 rows: 16 x 48 5.6 / 6.5, 64 x 64 9.1 / 8.9; 70000: 16 x 48
+// 8.4 / 7.7, 64 x 64 18.2 / 16.4).  With few column tiles and whole 64-k
+// stages k_skinny_dot pipelines as well (16 x 128: 12.8 / 15.3 at 10^5 rows,
+// 100 / 105 at 10^6; 32 x 128 15.7 / 16.7 at 70000, 131 / 128 at 10^6; 16 x
+// 64: 10.2 / 11.1 at 10^5, 23.3 / 21.1 at 3 10^5).
+bool skinny_rows_better(int64_t M, int64_t N, int64_t K, int64_t lda) {
+  if (K < 1 || K > kRowsMaxK || N < 1 || N > kRowsMaxN || M < kRowsMinM) return false;
+  if (lda > kRowsMaxLda || (lda != K && K % 4 != 0)) return false;
+  return !(K == 128 && N <= 32) && !(K == 64 && N <= 16 && M < 4 * kRowsMinM);
+}
+
+hipError_t launch_skinny_rows(const DotParams &p, hipStream_t st) {
+  if (!skinny_rows_better(p.M, p.N, p.K, p.sAm)) return hipErrorInvalidValue;
+  // passes of at most 4 column tiles, the tiles spread evenly
+  const int nct = (int)((p.N + 15) / 16), passes = (nct + 3) / 4, ct = (nct + passes - 1) / passes;
+  const void *fn = p.K % 4 == 0 ? rows_fn<true>(ct) : rows_fn<false>(ct);
+  // the workgroup size that keeps most waves (at most 16) on a CU by LDS
+  int w = 4, per_cu = 1;
+  for (const int ww : {8, 6, 4}) {
+    const int n = std::min<int>(16 / ww, (int)(kDotMaxLds / rows_lds_bytes(ww, p.N, p.K)));
+    if (n * ww > w * per_cu) {
+      w = ww;
+      per_cu = n;
+    }
+  }
+  const size_t lds = rows_lds_bytes(w, p.N, p.K);
+  if (lds > 65536) {
+    const hipError_t e =
+        hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  const int64_t tiles = (p.M + 15) / 16;
+  const int64_t nblk = std::min<int64_t>((tiles + w - 1) / w, (int64_t)device_cus() * per_cu);
+  DotParams q = p;
+  void *args[] = {&q};
+  return hipLaunchKernel(fn, dim3((unsigned)nblk), dim3(64 * w), args, lds, st);
 }
 
 bool skinny_axpy_runnable(int rt, int ct, int kw) {

@@ -170,7 +170,10 @@ size_t hmlSgemmWorkspaceSize(hmlOrder order, hmlOp transA, hmlOp transB,
 
 /* The variant hmlSgemmEx would run for these arguments, and which selector
  * produced it (0 built-in heuristic, 1 config table, 2 learned MLP; the
- * order is given with hmlSelectorInstall). */
+ * order is given with hmlSelectorInstall).  Where a DOT-form variant is selected
+ * for many rows of few k (K <= 128, M >= 65536), hmlSgemmEx runs a
+ * row-streaming kernel in its place, with the results of an unsplit DOT
+ * variant; hmlSgemmExVariant runs the variant it is given. */
 hmlStatus hmlSgemmSelect(hmlOrder order, hmlOp transA, hmlOp transB,
                          int64_t M, int64_t N, int64_t K, float beta,
                          hmlSgemmVariant *variant, int32_t *source);

@@ -502,3 +502,36 @@ def test_axpy_ragged_rows(hml, M, K):
             hml.sgemm_ex(M, N, K, dA, dB, dC, 2.0, -1.0, transA=True, lda=M + pad, variant=v)
             hml.synchronize()
             np.testing.assert_array_equal(dC.to_numpy((M, N)), R, err_msg="N=%d %r" % (N, v))
+
+
+@pytest.mark.parametrize("N", [2, 16, 17, 33, 65, 113, 128])
+@pytest.mark.parametrize("K", [1, 4, 15, 17, 64, 100, 127, 128])
+def test_row_streaming(hml, N, K):
+    """Many rows of few k (the row-streaming kernel): whole and partial row
+    tiles, the k and column remainders of its tiles, B and C in either
+    layout, a leading dimension past K, beta, and the same bits as the
+    unsplit DOT variant."""
+    rng = np.random.default_rng(1000 * N + K)
+    M = 65536 + (1, 16, 9)[K % 3]
+    A, B, C0 = uniform(rng, (M, K)), uniform(rng, (K, N)), uniform(rng, (M, N))
+    Ai, Bi, Ci = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
+    variant = (1, 1, 1 if N <= 16 else 2, 1, 1)
+    for tb in (False, True):
+        got = run_gemm(hml, A, B, C0, 1.0, 0.0, tb=tb)
+        want = run_gemm(hml, A, B, C0, 1.0, 0.0, tb=tb, variant=variant)
+        np.testing.assert_array_equal(got, want)
+        np.testing.assert_array_equal(run_gemm(hml, Ai, Bi, Ci, 2.0, -1.0, tb=tb),
+                                      exact_product(Ai, Bi, 2.0, -1.0, Ci))
+    # column-major C = A B with A stored row-major (transposed)
+    np.testing.assert_array_equal(run_gemm(hml, Ai, Bi, Ci, 1.0, 3.0, order="col", ta=True),
+                                  exact_product(Ai, Bi, 1.0, 3.0, Ci))
+    # A and C as panels of wider matrices (NaN around A, kept values around C)
+    Aw = np.full((M, K + 5), np.nan, np.float32)
+    Aw[:, :K] = Ai
+    Cw = np.full((M, N + 3), 7.0, np.float32)
+    dA, dB, dC = (hml.DeviceBuffer.from_numpy(x) for x in (Aw, Bi, Cw))
+    hml.sgemm_ex(M, N, K, dA, dB, dC, 1.0, 0.0, lda=K + 5, ldc=N + 3)
+    hml.synchronize()
+    out = dC.to_numpy((M, N + 3))
+    np.testing.assert_array_equal(out[:, :N], exact_product(Ai, Bi))
+    assert (out[:, N:] == 7.0).all()
