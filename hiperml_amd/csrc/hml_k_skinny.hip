@@ -65,12 +65,14 @@ __device__ __forceinline__ f4 mfma4(float a, float b, f4 c) {
 // private to the wave, so only the wave's own LDS ordering is needed, not a
 // barrier.
 //
-// B(k, n) is read in place with its own strides: lane
-// (g, r) of column tile c needs B(k0 + 16v + 4g + j, 16c + r), j = 0..3 --
-// one 16-byte load when B is K-contiguous and aligned (BVEC), four scalar
-// loads otherwise.  Columns past N read column N - 1: they feed only output
-// columns that are never stored.  K past the chunk end reads as zero (A and
-// B), so no NaN from memory outside the operands can reach a sum.
+// B(k, n) is read in place.  K-contiguous B (BVEC): lane (g, r) of column
+// tile c takes column 16c + r, one 16-byte load for its 4 k.  N-contiguous
+// B: lane (g, r) takes CT consecutive columns, one per column tile, so that
+// one load per k fetches them (16 loads of 4 CT bytes per 64-k stage instead
+// of 16 CT element loads) and C leaves in CT-float stores; the lane that
+// crosses column N takes the CT columns before it (dot_cols).  The sums of an
+// element are the same in either assignment.  K past the chunk end reads as
+// zero (A and B), so no NaN from memory outside the operands can reach a sum.
 //
 // The A and B loads of a stage are issued together, PS stages ahead, into
 // PS register sets: all vector loads retire through one in-order counter,
@@ -148,6 +150,101 @@ __device__ __forceinline__ void dot_store(const DotParams &p, int64_t row,
   }
 }
 
+// Columns of lane r in a tile of CT column tiles that starts at column n0.
+// K-contiguous B (BVEC): column n0 + 16 c + r in tile c.  N-contiguous B: the
+// CT consecutive columns base .. base + CT - 1, one per tile, so that one
+// load fetches them (and one store writes them); base is n0 + CT r, or, for
+// the lane that would cross column N, N - CT: its first `skip` columns are
+// the previous lane's and are not stored.  base < 0: no column.
+struct DotCols {
+  int64_t base;
+  int skip;
+};
+template <int CT>
+__device__ __forceinline__ DotCols dot_cols(int64_t n0, int r, int64_t N) {
+  const int64_t first = n0 + CT * r;
+  if (first >= N) return DotCols{-1, 0};
+  if (first + CT <= N) return DotCols{first, 0};
+  return DotCols{N - CT, (int)(first + CT - N)};
+}
+
+// Stores v[c], c < CT, at C(row, columns of the lane) (see dot_cols; with
+// BVEC at columns n0 + 16 c + r) of a matrix with strides (sCm, sCn).
+template <int N>
+struct __attribute__((packed, aligned(4))) DotVec {
+  float v[N];
+};
+template <int CT, bool BVEC>
+__device__ __forceinline__ void dot_store_cols(float *C, int64_t sCm, int64_t sCn, int64_t M,
+                                               int64_t N, float alpha, float beta, bool read_c,
+                                               int64_t row, int64_t n0, int r, DotCols dc,
+                                               const float (&v)[CT]) {
+  if (row >= M) return;
+  float *cr = C + row * sCm;
+  if (BVEC) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int64_t col = n0 + 16 * c + r;
+      if (col < N) {
+        float o = alpha * v[c];
+        if (read_c) o = alpha * v[c] + beta * cr[col * sCn];
+        cr[col * sCn] = o;
+      }
+    }
+    return;
+  }
+  if (dc.base < 0) return;
+  if (CT > 1 && sCn == 1 && dc.skip == 0) {
+    DotVec<CT> o;
+    if (read_c) o = *reinterpret_cast<const DotVec<CT> *>(cr + dc.base);
+#pragma unroll
+    for (int c = 0; c < CT; ++c) o.v[c] = read_c ? alpha * v[c] + beta * o.v[c] : alpha * v[c];
+    *reinterpret_cast<DotVec<CT> *>(cr + dc.base) = o;
+    return;
+  }
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+    if (c >= dc.skip) {
+      float *cp = cr + (dc.base + c) * sCn;
+      float o = alpha * v[c];
+      if (read_c) o = alpha * v[c] + beta * (*cp);
+      *cp = o;
+    }
+}
+// The same into C or, with several K groups, the partials of group kgi.
+template <int CT, bool BVEC>
+__device__ __forceinline__ void dot_store_row(const DotParams &p, int64_t row, int64_t n0, int r,
+                                              DotCols dc, int kgi, const float (&v)[CT]) {
+  if (p.kgroups == 1)
+    dot_store_cols<CT, BVEC>(p.C, p.sCm, p.sCn, p.M, p.N, p.alpha, p.beta, p.read_c != 0, row, n0,
+                             r, dc, v);
+  else
+    dot_store_cols<CT, BVEC>(p.P + (int64_t)kgi * p.M * p.N, p.N, 1, p.M, p.N, 1.f, 0.f, false,
+                             row, n0, r, dc, v);
+}
+
+// CT consecutive floats at any 4-byte-aligned offset.
+template <int CT>
+__device__ __forceinline__ void buf_load_n(__amdgpu_buffer_rsrc_t rs, uint32_t voff, int32_t soff,
+                                           float (&o)[CT]) {
+  if constexpr (CT == 1) {
+    o[0] = buf_load1(rs, voff, soff);
+  } else if constexpr (CT == 2) {
+    const f2 x = buf_load2(rs, voff, soff);
+    o[0] = x[0];
+    o[1] = x[1];
+  } else if constexpr (CT == 3) {
+    typedef float f3 __attribute__((ext_vector_type(3)));
+    const f3 x = __builtin_bit_cast(f3, __builtin_amdgcn_raw_buffer_load_b96(rs, voff, soff, 0));
+#pragma unroll
+    for (int c = 0; c < 3; ++c) o[c] = x[c];
+  } else {
+    const f4 x = buf_load4<0>(rs, voff, soff);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] = x[c];
+  }
+}
+
 // One wave: rows [row0, row0 + 16 RT) x columns [ct0*16, ct0*16 + 16 CT)
 // over k in [kb, ke) (kb a multiple of the 64-k stage), accumulated into
 // acc.  T is the wave's private LDS: one A tile (16 RT x 64 floats) when the
@@ -161,7 +258,8 @@ __device__ __forceinline__ void dot_store(const DotParams &p, int64_t row,
 // compiler does not order these LDS writes against the tile's reads, so the
 // waits are explicit: before a stage's reads, vmcnt(NQ) (only the NQ loads
 // of the stage issued last may still be in flight: the loads of the stage
-// being read and its B came earlier), and before a tile is refilled,
+// being read and its B came earlier; SPREAD: also the second half of the
+// stage's own 16 loads of B, issued in between), and before a tile is refilled,
 // lgkmcnt(0) (its reads are done).
 template <int RT, int CT, bool BVEC, bool DMA, int APOL = kBufNT>
 __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_t sAm,
@@ -186,7 +284,7 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
   // guarantees every in-range offset of a wave is below 2^31.
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(A + row0 * sAm + kb, kRsrcMax);
   const __amdgpu_buffer_rsrc_t rbs =
-      make_rsrc(B + kb * sBk + (int64_t)ct0 * 16 * sBn, kRsrcMax);
+      make_rsrc(B + kb * sBk + (BVEC ? (int64_t)ct0 * 16 * sBn : 0), kRsrcMax);
   const __amdgpu_buffer_rsrc_t rnull = make_rsrc(A, 0);
   uint32_t aoff[NQ];  // row row0 + 4q + g, k = kb + 4r (DMA: 4 (r ^ row % 16))
 #pragma unroll
@@ -195,11 +293,16 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
     const int kc = DMA ? (r ^ (x & 15)) : r;
     aoff[q] = row0 + x < M ? (uint32_t)((x * sAm + 4 * kc) * 4) : kOOB;
   }
-  uint32_t boff[CT];  // column ct0*16 + 16c + r, k = kb + 4g
+  uint32_t boff[BVEC ? CT : 1];  // the lane's columns, k = kb + 4g
+  if constexpr (BVEC) {
 #pragma unroll
-  for (int c = 0; c < CT; ++c)
-    boff[c] = (int64_t)(ct0 + c) * 16 + r < N
-                  ? (uint32_t)((4 * g * sBk + (16 * c + r) * sBn) * 4) : kOOB;
+    for (int c = 0; c < CT; ++c)
+      boff[c] = (int64_t)(ct0 + c) * 16 + r < N
+                    ? (uint32_t)((4 * g * sBk + (16 * c + r) * sBn) * 4) : kOOB;
+  } else {
+    const DotCols dc = dot_cols<CT>((int64_t)ct0 * 16, r, N);
+    boff[0] = dc.base >= 0 ? (uint32_t)((4 * g * sBk + dc.base) * 4) : kOOB;
+  }
 
 #pragma unroll
   for (int t = 0; t < RT; ++t)
@@ -223,20 +326,21 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
   auto loadBu = [&](int u, int64_t s) {
     const __amdgpu_buffer_rsrc_t rs = s < nst ? rbs : rnull;
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int v = 0; v < 2; ++v) {
+      const int64_t ko = s * kDotStageK + 32 * u + 16 * v;
+      if constexpr (BVEC) {
 #pragma unroll
-      for (int v = 0; v < 2; ++v) {
-        const int64_t ko = s * kDotStageK + 32 * u + 16 * v;
-        f4 x;
-        if (BVEC) {
-          x = buf_load4<0>(rs, boff[c], (int32_t)(ko * 4));
-        } else {
+        for (int c = 0; c < CT; ++c) b[c][u][v] = buf_load4<0>(rs, boff[c], (int32_t)(ko * 4));
+      } else {
 #pragma unroll
-          for (int jj = 0; jj < 4; ++jj)
-            x[jj] = buf_load1(rs, boff[c], (int32_t)((ko + jj) * sBk * 4));
+        for (int jj = 0; jj < 4; ++jj) {
+          float x[CT];
+          buf_load_n<CT>(rs, boff[0], (int32_t)((ko + jj) * sBk * 4), x);
+#pragma unroll
+          for (int c = 0; c < CT; ++c) b[c][u][v][jj] = x[c];
         }
-        b[c][u][v] = x;
       }
+    }
   };
   // wave-local LDS ordering (the tile is private to the wave)
   auto wave_sync = [&]() {
@@ -248,6 +352,45 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
       *reinterpret_cast<f4 *>(Tj + dot_tile_off(4 * q + g, r)) = a[j][q];
+    wave_sync();
+  };
+  // The DMA tiles with N-contiguous B: each B register is refilled right
+  // behind the MFMAs that read it, and the tile is read one half k-step
+  // ahead, a scheduling barrier per MFMA group keeping the loads spread over
+  // the stage.  Left to the scheduler they gather at the stage's end and the
+  // next stage waits for them.  8192 x 64 x 8192 (K split 4): 94 us with
+  // element loads of B in one burst, 91 with CT-column loads, 83 spread;
+  // 8192 x 128 x 8192 153 / 144 / 138.  K-contiguous B and fewer column tiles
+  // load little enough that the plain order is as good or better.
+  constexpr bool SPREAD = DMA && !BVEC;
+  auto compute_spread = [&](const float *Tj, int64_t s_next) {
+    const __amdgpu_buffer_rsrc_t rs = s_next < nst ? rbs : rnull;
+    f4 x[2][RT];
+    auto read = [&](int h) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+        x[h & 1][t] = *reinterpret_cast<const f4 *>(Tj + dot_tile_off(16 * t + r, 4 * h + g));
+    };
+    read(0);
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {  // k-step u = h / 2, half v = h % 2
+      if (h < 3) read(h + 1);
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const int32_t so = (int32_t)((s_next * kDotStageK + 16 * h + jj) * sBk * 4);
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int c = 0; c < CT; ++c)
+            acc[t][c] = mfma4(x[h & 1][t][jj], b[c][h >> 1][h & 1][jj], acc[t][c]);
+        float y[CT];
+        buf_load_n<CT>(rs, boff[0], so, y);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) b[c][h >> 1][h & 1][jj] = y[c];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // the tile may be overwritten only after these reads
     wave_sync();
   };
   // MFMAs of the stage in tile Tj and b; each k-step's B registers are
@@ -287,10 +430,11 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
 #pragma unroll
       for (int j = 0; j < PS; ++j) {
         if (s + j < nst) {
-          __builtin_amdgcn_s_waitcnt(waitcnt_vm(NQ));
+          __builtin_amdgcn_s_waitcnt(waitcnt_vm(SPREAD ? NQ + 8 : NQ));
           __builtin_amdgcn_sched_barrier(0);
           wave_sync();
-          compute(T + j * TF, s + j + 1);
+          if constexpr (SPREAD) compute_spread(T + j * TF, s + j + 1);
+          else compute(T + j * TF, s + j + 1);
         }
         __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
         __builtin_amdgcn_sched_barrier(0);
@@ -353,8 +497,9 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {
             const int64_t ko = nst * kDotStageK + 32 * u + 16 * v + jj;
-            const uint32_t vo = (boff[c] == kOOB || kb + ko + 4 * g >= ke) ? kOOB
-                                : boff[c] + (uint32_t)(ko * sBk * 4);
+            const uint32_t bo = BVEC ? boff[BVEC ? c : 0] : boff[0];
+            const uint32_t vo = (bo == kOOB || kb + ko + 4 * g >= ke) ? kOOB
+                                : bo + (uint32_t)((ko * sBk + (BVEC ? 0 : c)) * 4);
             x[jj] = buf_load1(rbs, vo, 0);
           }
           b[c][u][v] = x;
@@ -363,7 +508,9 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
     for (int q = 0; q < NQ; ++q)
       *reinterpret_cast<f4 *>(T + dot_tile_off(4 * q + g, r)) = ap[q];
     wave_sync();
-    compute(T, nst + 1);  // nothing left to load: the refills read zeros, no traffic
+    // nothing left to load: the refills read zeros, no traffic
+    if constexpr (SPREAD) compute_spread(T, nst + 1);
+    else compute(T, nst + 1);
   }
 }
 
@@ -392,34 +539,44 @@ __global__ __launch_bounds__(64 * dot_max_waves(RT, CT)) void k_skinny_dot(DotPa
                                                    row0, ct0, kb, ke,
                                                    reinterpret_cast<float *>(dot_lds) + w * WF, acc);
 
+  // Lane (g, r) holds rows 16 t + 4 g + i of its CT columns.
+  const int64_t n0 = (int64_t)ct0 * 16;
+  const DotCols dc = dot_cols<CT>(n0, r, p.N);
   if (kw == 1) {
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
-      for (int c = 0; c < CT; ++c)
+      for (int i = 0; i < 4; ++i) {
+        float v[CT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          dot_store(p, row0 + 16 * t + 4 * g + i, (int64_t)(ct0 + c) * 16 + r, kgi, acc[t][c][i]);
+        for (int c = 0; c < CT; ++c) v[c] = acc[t][c][i];
+        dot_store_row<CT, BVEC>(p, row0 + 16 * t + 4 * g + i, n0, r, dc, kgi, v);
+      }
     return;
   }
-  // sum over the waves of the workgroup, in wave order (the tiles are done)
+  // sum over the waves of the workgroup, in wave order (the tiles are done):
+  // row group q = 4 t + i, CT floats per lane
   __syncthreads();
-  constexpr int NT = RT * CT;
+  constexpr int NT = RT * 4;
+  DotVec<CT> *sums = reinterpret_cast<DotVec<CT> *>(dot_lds);
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int c = 0; c < CT; ++c) dot_lds[(w * NT + t * CT + c) * 64 + lane] = acc[t][c];
+    for (int i = 0; i < 4; ++i) {
+      DotVec<CT> v;
+#pragma unroll
+      for (int c = 0; c < CT; ++c) v.v[c] = acc[t][c][i];
+      sums[(w * NT + 4 * t + i) * 64 + lane] = v;
+    }
   __syncthreads();
   for (int q = w; q < NT; q += kw) {
-    f4 sum = dot_lds[q * 64 + lane];
+    DotVec<CT> sum = sums[q * 64 + lane];
     for (int ww = 1; ww < kw; ++ww) {
-      const f4 x = dot_lds[(ww * NT + q) * 64 + lane];
-      sum[0] += x[0]; sum[1] += x[1]; sum[2] += x[2]; sum[3] += x[3];
-    }
-    const int t = q / CT, c = q - t * CT;
+      const DotVec<CT> x = sums[(ww * NT + q) * 64 + lane];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      dot_store(p, row0 + 16 * t + 4 * g + i, (int64_t)(ct0 + c) * 16 + r, kgi, sum[i]);
+      for (int c = 0; c < CT; ++c) sum.v[c] += x.v[c];
+    }
+    dot_store_row<CT, BVEC>(p, row0 + 16 * (q >> 2) + 4 * g + (q & 3), n0, r, dc, kgi, sum.v);
   }
 }
 
@@ -608,7 +765,9 @@ __global__ __launch_bounds__(64 * kRowsWaves, 4) void k_skinny_rows(DotParams p)
 // as the compiler knows the C stores may alias the descriptor array, so
 // fields read through the reference inside the loop were reloaded from
 // memory after every store, one dependent round trip per element.
-template <int RT, int CT>
+// ROWS: the lane's CT columns are consecutive (dot_cols), as k_grouped_dot's
+// tiles leave them; otherwise column 16 c + r.
+template <int RT, int CT, bool ROWS>
 __device__ __forceinline__ void grouped_store(const GroupProblem &gp, int64_t row0, int ct0,
                                               const f4 (&acc)[RT][CT]) {
   float *const C = gp.C;
@@ -617,21 +776,18 @@ __device__ __forceinline__ void grouped_store(const GroupProblem &gp, int64_t ro
   const bool read_c = gp.read_c != 0;
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
+  const int64_t n0 = (int64_t)ct0 * 16;
+  const DotCols dc = dot_cols<CT>(n0, r, N);
 #pragma unroll
-  for (int tt = 0; tt < RT; ++tt)
+  for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int i = 0; i < 4; ++i) {
+      float v[CT];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t row = row0 + 16 * tt + 4 * g + i;
-        const int64_t col = (int64_t)(ct0 + c) * 16 + r;
-        if (row < M && col < N) {
-          float *cp = C + row * ldc + col;
-          float v = alpha * acc[tt][c][i];
-          if (read_c) v = alpha * acc[tt][c][i] + beta * (*cp);
-          *cp = v;
-        }
-      }
+      for (int c = 0; c < CT; ++c) v[c] = acc[t][c][i];
+      dot_store_cols<CT, !ROWS>(C, ldc, 1, M, N, alpha, beta, read_c, row0 + 16 * t + 4 * g + i,
+                                n0, r, dc, v);
+    }
 }
 
 template <int RT, int CT>
@@ -655,7 +811,7 @@ __global__ __launch_bounds__(64 * kGroupWaveWpb, 2) void k_grouped_dot(const Gro
       f4 acc[RT][CT];
       dot_tile_lds<RT, CT, false, dot_dma(RT, CT), 0>(gp.A, gp.lda, gp.B, gp.ldb, 1, gp.M, gp.N,
                                                      row0, ct0, 0, gp.K, T, acc);
-      grouped_store<RT, CT>(gp, row0, ct0, acc);
+      grouped_store<RT, CT, true>(gp, row0, ct0, acc);
     }
   }
 }
@@ -1225,7 +1381,7 @@ __global__ __launch_bounds__(64 * kDotbWaves, 2) void k_grouped_dotb(const Group
       f4 acc[RT][CT];
       dotb_block<RT, CT, false, 0>(gp.A, gp.lda, gp.B, gp.ldb, 1, gp.M, gp.N, row0, ct0, 0,
                                    gp.K, lds, acc);
-      grouped_store<RT, CT>(gp, row0, ct0, acc);
+      grouped_store<RT, CT, false>(gp, row0, ct0, acc);
       // the next block's first stage overwrites the LDS other waves may
       // still be reading
       __syncthreads();
@@ -1422,6 +1578,9 @@ hipError_t launch_skinny_dot(int rt, int ct, bool bvec, int kw, const DotParams 
                              hipStream_t st) {
   if (!skinny_dot_runnable(rt, ct, kw) || p.kgroups < 1 || p.kchunk % kDotStageK != 0)
     return hipErrorInvalidValue;
+  // N-contiguous B is read CT columns at a time; fewer columns take the
+  // one-tile kernel (the sums are the same)
+  if (!bvec && p.N < ct) ct = 1;
   const int64_t ncb = ((p.N + 15) / 16 + ct - 1) / ct;
   DotFn fn = find_dot(rt, ct, bvec, a_loads_cached(p.A, p.sAm, ncb));
   return fn(kw, p, st);

@@ -535,3 +535,31 @@ def test_row_streaming(hml, N, K):
     out = dC.to_numpy((M, N + 3))
     np.testing.assert_array_equal(out[:, :N], exact_product(Ai, Bi))
     assert (out[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("N", [2, 3, 4, 5, 17, 18, 31, 33, 34, 35, 47, 49, 61, 62, 63, 65, 127, 129])
+def test_dot_column_remainders(hml, N):
+    """N-contiguous B read a few columns per lane: column counts around the
+    tiles' and the lanes' edges, B and C as panels (NaN beside B, kept values
+    beside C), B's last row ending its allocation, one and several waves and
+    K groups, whole and partial stages."""
+    rng = np.random.default_rng(N)
+    for M, K in ((70, 64), (33, 129), (130, 200)):
+        A, B, C0 = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
+        R = exact_product(A, B, 2.0, -1.0, C0)
+        for pad in (0, 5):
+            Bw = np.full((K, N + pad), np.nan, np.float32)
+            Bw[:, :N] = B
+            Cw = np.full((M, N + pad), 7.0, np.float32)
+            Cw[:, :N] = C0
+            dA, dB = hml.DeviceBuffer.from_numpy(A), hml.DeviceBuffer.from_numpy(Bw)
+            for v in ((1, 1, 1, 1, 1), (1, 1, 2, 2, 1), (1, 2, 2, 4, 4), (1, 1, 4, 3, 2),
+                      (1, 2, 4, 1, 1), (1, 2, 4, 4, 1), (1, 4, 2, 2, 2)):
+                if N > M:
+                    continue
+                dC = hml.DeviceBuffer.from_numpy(Cw)
+                hml.sgemm_ex(M, N, K, dA, dB, dC, 2.0, -1.0, ldb=N + pad, ldc=N + pad, variant=v)
+                hml.synchronize()
+                out = dC.to_numpy((M, N + pad))
+                np.testing.assert_array_equal(out[:, :N], R, err_msg="%r pad=%d" % (v, pad))
+                assert (out[:, N:] == 7.0).all()
