@@ -364,8 +364,63 @@ hmlStatus run_dense_fallback(const GemmCanon &g, const GemmKey &k, float alpha, 
                    alpha, beta, read_c, dws, dn, st);
 }
 
+// Tile and K split of a chosen DOT variant with more than 32 columns of
+// N-contiguous B, where the kernels are bound by the FP32 matrix cores.  The
+// model, in us: a wave of rt x ct tiles spends 8 rt ct clocks of its SIMD per
+// k; the waves (tiles x K chunks) run in rounds of one per SIMD, where
+// workgroups of 2 or 3 waves leave 2 or 1 of a CU's 4 SIMDs idle; a round's
+// start and end cost 1 (16-row tiles) or 3 (32-row tiles); 16-row tiles take
+// 10% longer per product (B is loaded for fewer rows), one or two column
+// tiles 20%; chunks past one workgroup's waves add a reduction pass.  Fitted
+// on 24 shapes (M 600..60000, N 40..2500, K 300..16384).  Measured / modelled:
+// 8192 x 64 x 8192: 2x4 in 4 chunks 77 / 78, in 8 85 / 86, 1x4 in 4 87 / 85;
+// 60000 x 64 x 1000: 2x4 in 4 104 / 99, 1x4 unsplit 88 / 85; 2500 x 2500 x
+// 1000: 2x4 in 4 165 / 155, 1x4 unsplit 139 / 143.
+double dot_model_us(const GemmKey &k, const hmlSgemmVariant &v) {
+  const SkinnyPlan pl = plan_skinny(k, v);
+  const int64_t nct = ceil_div(k.N, 16), nch = ceil_div(k.K, pl.kchunk);
+  const int64_t tiles = ceil_div(k.M, 16 * v.rt) * ceil_div(nct, v.ct);
+  const int64_t slots = pl.kw == 2 ? 512 : pl.kw == 3 ? 768 : 1024;
+  const double rounds = (double)ceil_div(tiles * nch, slots);
+  double us = 1.12 * rounds * (double)pl.kchunk * 8.0 * v.rt * v.ct / 2200.0;
+  us *= (v.rt == 1 ? 1.1 : 1.0) * (v.ct < 3 ? 1.2 : 1.0);
+  us += rounds * (v.rt == 1 ? 1.0 : 3.0);
+  us = std::max(us, (double)k.M * (double)k.K * 4.0 / 6.0e6) + 7.0;
+  if (pl.ksplit > 1) us += 5.0 + (double)pl.p_floats * 8.0 / 4.0e6;
+  return us;
+}
+
+// Replaces a chosen DOT variant by the model's best geometry where that is
+// 5% or more ahead of it (from 3.5e8 products: below that the model's errors
+// are as large as the differences).  It never needs more partial sums than
+// the variant that was chosen and sums no longer chains (8192 x 64 x 8192 in 4
+// chunks instead of 8 would be 77 us instead of 81, at 1.4 times the error).
+// Unsplit 32-row tiles stay out: single-wave workgroups with 16 KB of LDS
+// each fill the chip unevenly (2500 x 2500 x 1000 169 us, unsplit 16-row tiles
+// 139).
+void dot_geometry(const GemmKey &k, hmlSgemmVariant *v) {
+  if ((double)k.M * (double)k.N * (double)k.K < 3.5e8) return;
+  const SkinnyPlan from = plan_skinny(k, *v);
+  hmlSgemmVariant out = *v;
+  double best = 0.95 * dot_model_us(k, *v);
+  for (int ct = 4; ct >= 3; --ct)
+    for (int rt = 1; rt <= 2; ++rt)
+      for (const int32_t ks : {1, 4, 8, 16, 32, 64, v->ksplit}) {
+        if ((rt == 2 && ks == 1) || ks < 1) continue;
+        const hmlSgemmVariant c{HML_SGEMM_FAMILY_DOT, rt, ct, ks, 4};
+        const SkinnyPlan pl = plan_skinny(k, c);
+        if (pl.p_floats > from.p_floats || pl.kchunk > from.kchunk) continue;
+        const double us = dot_model_us(k, c);
+        if (us < best) {
+          best = us;
+          out = c;
+        }
+      }
+  *v = out;
+}
+
 hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
-                    const hmlSgemmVariant &v, bool chosen, float alpha, float beta,
+                    hmlSgemmVariant v, bool chosen, float alpha, float beta,
                     int read_c, void *ws, size_t ws_bytes, hipStream_t st) {
   const size_t need = workspace_bytes(k, v);
   void *const caller_ws = ws;
@@ -394,6 +449,7 @@ hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
     p.alpha = alpha; p.beta = beta; p.read_c = read_c;
     return from_hip(launch_skinny_rows(p, st), "row-streaming kernel launch");
   }
+  if (chosen && v.family == HML_SGEMM_FAMILY_DOT && k.N > 32 && g.sBk != 1) dot_geometry(k, &v);
   if (v.family == HML_SGEMM_FAMILY_GEMV)
     return run_gemv_family(g, k, v, alpha, beta, read_c, ws, st);
   if (v.family == HML_SGEMM_FAMILY_GEMVN) {

@@ -65,12 +65,12 @@ __device__ __forceinline__ f4 mfma4(float a, float b, f4 c) {
 // private to the wave, so only the wave's own LDS ordering is needed, not a
 // barrier.
 //
-// B(k, n) is read in place.  K-contiguous B (BVEC): lane (g, r) of column
-// tile c takes column 16c + r, one 16-byte load for its 4 k.  N-contiguous
-// B: lane (g, r) takes CT consecutive columns, one per column tile, so that
-// one load per k fetches them (16 loads of 4 CT bytes per 64-k stage instead
-// of 16 CT element loads) and C leaves in CT-float stores; the lane that
-// crosses column N takes the CT columns before it (dot_cols).  The sums of an
+// B(k, n) is read in place.  Lane (g, r) of column tile c takes column
+// 16c + r: one 16-byte load for its 4 k when B is K-contiguous (BVEC), four
+// element loads otherwise.  N-contiguous B and 3 or 4 column tiles (BROW):
+// lane (g, r) takes CT consecutive columns, one per column tile, so that one
+// load per k fetches them (16 loads of 4 CT bytes per 64-k stage instead of
+// 16 CT element loads) and C leaves in CT-float stores; the lane that crosses column N takes the CT columns before it (dot_cols).  The sums of an
 // element are the same in either assignment.  K past the chunk end reads as
 // zero (A and B), so no NaN from memory outside the operands can reach a sum.
 //
@@ -150,12 +150,16 @@ __device__ __forceinline__ void dot_store(const DotParams &p, int64_t row,
   }
 }
 
-// Columns of lane r in a tile of CT column tiles that starts at column n0.
-// K-contiguous B (BVEC): column n0 + 16 c + r in tile c.  N-contiguous B: the
+// Columns of lane r in a tile of CT column tiles that starts at column n0:
+// n0 + 16 c + r in tile c or, for N-contiguous B and 3 or 4 tiles (BROW), the
 // CT consecutive columns base .. base + CT - 1, one per tile, so that one
 // load fetches them (and one store writes them); base is n0 + CT r, or, for
 // the lane that would cross column N, N - CT: its first `skip` columns are
 // the previous lane's and are not stored.  base < 0: no column.
+// Only for 3 and 4 column tiles: with two, the pairs measured slower than
+// element loads (5000 x 64 x 700 14.6 against 13.5 us, 1000 x 900 x 300 14.2
+// against 12.3).
+__host__ __device__ constexpr bool dot_brow(int ct, bool bvec) { return !bvec && ct >= 3; }
 struct DotCols {
   int64_t base;
   int skip;
@@ -168,20 +172,20 @@ __device__ __forceinline__ DotCols dot_cols(int64_t n0, int r, int64_t N) {
   return DotCols{N - CT, (int)(first + CT - N)};
 }
 
-// Stores v[c], c < CT, at C(row, columns of the lane) (see dot_cols; with
-// BVEC at columns n0 + 16 c + r) of a matrix with strides (sCm, sCn).
+// Stores v[c], c < CT, at C(row, columns of the lane) (see dot_cols; without
+// BROW at columns n0 + 16 c + r) of a matrix with strides (sCm, sCn).
 template <int N>
 struct __attribute__((packed, aligned(4))) DotVec {
   float v[N];
 };
-template <int CT, bool BVEC>
+template <int CT, bool BROW>
 __device__ __forceinline__ void dot_store_cols(float *C, int64_t sCm, int64_t sCn, int64_t M,
                                                int64_t N, float alpha, float beta, bool read_c,
                                                int64_t row, int64_t n0, int r, DotCols dc,
                                                const float (&v)[CT]) {
   if (row >= M) return;
   float *cr = C + row * sCm;
-  if (BVEC) {
+  if (!BROW) {
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
       const int64_t col = n0 + 16 * c + r;
@@ -212,14 +216,14 @@ __device__ __forceinline__ void dot_store_cols(float *C, int64_t sCm, int64_t sC
     }
 }
 // The same into C or, with several K groups, the partials of group kgi.
-template <int CT, bool BVEC>
+template <int CT, bool BROW>
 __device__ __forceinline__ void dot_store_row(const DotParams &p, int64_t row, int64_t n0, int r,
                                               DotCols dc, int kgi, const float (&v)[CT]) {
   if (p.kgroups == 1)
-    dot_store_cols<CT, BVEC>(p.C, p.sCm, p.sCn, p.M, p.N, p.alpha, p.beta, p.read_c != 0, row, n0,
+    dot_store_cols<CT, BROW>(p.C, p.sCm, p.sCn, p.M, p.N, p.alpha, p.beta, p.read_c != 0, row, n0,
                              r, dc, v);
   else
-    dot_store_cols<CT, BVEC>(p.P + (int64_t)kgi * p.M * p.N, p.N, 1, p.M, p.N, 1.f, 0.f, false,
+    dot_store_cols<CT, BROW>(p.P + (int64_t)kgi * p.M * p.N, p.N, 1, p.M, p.N, 1.f, 0.f, false,
                              row, n0, r, dc, v);
 }
 
@@ -270,6 +274,7 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
   constexpr int PS = dot_stages(RT, CT);
   constexpr int NQ = 4 * RT;  // A load instructions per stage
   constexpr int TF = dot_tile_floats(RT);
+  constexpr bool BROW = dot_brow(CT, BVEC);
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
   const int64_t nst = ke > kb ? (ke - kb) / kDotStageK : 0;
@@ -284,7 +289,7 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
   // guarantees every in-range offset of a wave is below 2^31.
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(A + row0 * sAm + kb, kRsrcMax);
   const __amdgpu_buffer_rsrc_t rbs =
-      make_rsrc(B + kb * sBk + (BVEC ? (int64_t)ct0 * 16 * sBn : 0), kRsrcMax);
+      make_rsrc(B + kb * sBk + (BROW ? 0 : (int64_t)ct0 * 16 * sBn), kRsrcMax);
   const __amdgpu_buffer_rsrc_t rnull = make_rsrc(A, 0);
   uint32_t aoff[NQ];  // row row0 + 4q + g, k = kb + 4r (DMA: 4 (r ^ row % 16))
 #pragma unroll
@@ -293,8 +298,8 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
     const int kc = DMA ? (r ^ (x & 15)) : r;
     aoff[q] = row0 + x < M ? (uint32_t)((x * sAm + 4 * kc) * 4) : kOOB;
   }
-  uint32_t boff[BVEC ? CT : 1];  // the lane's columns, k = kb + 4g
-  if constexpr (BVEC) {
+  uint32_t boff[BROW ? 1 : CT];  // the lane's columns, k = kb + 4g
+  if constexpr (!BROW) {
 #pragma unroll
     for (int c = 0; c < CT; ++c)
       boff[c] = (int64_t)(ct0 + c) * 16 + r < N
@@ -331,6 +336,12 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
       if constexpr (BVEC) {
 #pragma unroll
         for (int c = 0; c < CT; ++c) b[c][u][v] = buf_load4<0>(rs, boff[c], (int32_t)(ko * 4));
+      } else if constexpr (!BROW) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj)
+            b[c][u][v][jj] = buf_load1(rs, boff[c], (int32_t)((ko + jj) * sBk * 4));
       } else {
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
@@ -362,7 +373,7 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
   // element loads of B in one burst, 91 with CT-column loads, 83 spread;
   // 8192 x 128 x 8192 153 / 144 / 138.  K-contiguous B and fewer column tiles
   // load little enough that the plain order is as good or better.
-  constexpr bool SPREAD = DMA && !BVEC;
+  constexpr bool SPREAD = DMA && BROW;
   auto compute_spread = [&](const float *Tj, int64_t s_next) {
     const __amdgpu_buffer_rsrc_t rs = s_next < nst ? rbs : rnull;
     f4 x[2][RT];
@@ -497,9 +508,9 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {
             const int64_t ko = nst * kDotStageK + 32 * u + 16 * v + jj;
-            const uint32_t bo = BVEC ? boff[BVEC ? c : 0] : boff[0];
+            const uint32_t bo = boff[BROW ? 0 : c];
             const uint32_t vo = (bo == kOOB || kb + ko + 4 * g >= ke) ? kOOB
-                                : bo + (uint32_t)((ko * sBk + (BVEC ? 0 : c)) * 4);
+                                : bo + (uint32_t)((ko * sBk + (BROW ? c : 0)) * 4);
             x[jj] = buf_load1(rbs, vo, 0);
           }
           b[c][u][v] = x;
@@ -550,7 +561,7 @@ __global__ __launch_bounds__(64 * dot_max_waves(RT, CT)) void k_skinny_dot(DotPa
         float v[CT];
 #pragma unroll
         for (int c = 0; c < CT; ++c) v[c] = acc[t][c][i];
-        dot_store_row<CT, BVEC>(p, row0 + 16 * t + 4 * g + i, n0, r, dc, kgi, v);
+        dot_store_row<CT, dot_brow(CT, BVEC)>(p, row0 + 16 * t + 4 * g + i, n0, r, dc, kgi, v);
       }
     return;
   }
@@ -576,7 +587,7 @@ __global__ __launch_bounds__(64 * dot_max_waves(RT, CT)) void k_skinny_dot(DotPa
 #pragma unroll
       for (int c = 0; c < CT; ++c) sum.v[c] += x.v[c];
     }
-    dot_store_row<CT, BVEC>(p, row0 + 16 * (q >> 2) + 4 * g + (q & 3), n0, r, dc, kgi, sum.v);
+    dot_store_row<CT, dot_brow(CT, BVEC)>(p, row0 + 16 * (q >> 2) + 4 * g + (q & 3), n0, r, dc, kgi, sum.v);
   }
 }
 
@@ -765,9 +776,7 @@ __global__ __launch_bounds__(64 * kRowsWaves, 4) void k_skinny_rows(DotParams p)
 // as the compiler knows the C stores may alias the descriptor array, so
 // fields read through the reference inside the loop were reloaded from
 // memory after every store, one dependent round trip per element.
-// ROWS: the lane's CT columns are consecutive (dot_cols), as k_grouped_dot's
-// tiles leave them; otherwise column 16 c + r.
-template <int RT, int CT, bool ROWS>
+template <int RT, int CT, bool BROW>
 __device__ __forceinline__ void grouped_store(const GroupProblem &gp, int64_t row0, int ct0,
                                               const f4 (&acc)[RT][CT]) {
   float *const C = gp.C;
@@ -785,7 +794,7 @@ __device__ __forceinline__ void grouped_store(const GroupProblem &gp, int64_t ro
       float v[CT];
 #pragma unroll
       for (int c = 0; c < CT; ++c) v[c] = acc[t][c][i];
-      dot_store_cols<CT, !ROWS>(C, ldc, 1, M, N, alpha, beta, read_c, row0 + 16 * t + 4 * g + i,
+      dot_store_cols<CT, BROW>(C, ldc, 1, M, N, alpha, beta, read_c, row0 + 16 * t + 4 * g + i,
                                 n0, r, dc, v);
     }
 }
@@ -811,7 +820,7 @@ __global__ __launch_bounds__(64 * kGroupWaveWpb, 2) void k_grouped_dot(const Gro
       f4 acc[RT][CT];
       dot_tile_lds<RT, CT, false, dot_dma(RT, CT), 0>(gp.A, gp.lda, gp.B, gp.ldb, 1, gp.M, gp.N,
                                                      row0, ct0, 0, gp.K, T, acc);
-      grouped_store<RT, CT, true>(gp, row0, ct0, acc);
+      grouped_store<RT, CT, dot_brow(CT, false)>(gp, row0, ct0, acc);
     }
   }
 }
@@ -1416,6 +1425,13 @@ DotFn dot_fn(bool bv, bool cached) {
                 : (bv ? run_dot<RT, CT, true, kBufNT> : run_dot<RT, CT, false, kBufNT>);
 }
 
+// Tiles of 3 column tiles, N-contiguous B: run by dot_geometry's choice only.
+DotFn find_dot3(int rt, bool cached) {
+  return rt == 1   ? (cached ? run_dot<1, 3, false, 0> : run_dot<1, 3, false, kBufNT>)
+         : rt == 2 ? (cached ? run_dot<2, 3, false, 0> : run_dot<2, 3, false, kBufNT>)
+                   : nullptr;
+}
+
 // instantiated (rt, ct): ct <= 4, rt * ct <= 8
 DotFn find_dot(int rt, int ct, bool bv, bool cached = false) {
   switch (rt * 16 + ct) {
@@ -1576,11 +1592,15 @@ bool skinny_dot_runnable(int rt, int ct, int kw) {
 
 hipError_t launch_skinny_dot(int rt, int ct, bool bvec, int kw, const DotParams &p,
                              hipStream_t st) {
-  if (!skinny_dot_runnable(rt, ct, kw) || p.kgroups < 1 || p.kchunk % kDotStageK != 0)
-    return hipErrorInvalidValue;
-  // N-contiguous B is read CT columns at a time; fewer columns take the
+  if (p.kgroups < 1 || p.kchunk % kDotStageK != 0) return hipErrorInvalidValue;
+  if (ct == 3) {
+    if (bvec || rt > 2 || p.N < 3 || kw < 1 || kw > 4) return hipErrorInvalidValue;
+    return find_dot3(rt, a_loads_cached(p.A, p.sAm, ((p.N + 15) / 16 + 2) / 3))(kw, p, st);
+  }
+  if (!skinny_dot_runnable(rt, ct, kw)) return hipErrorInvalidValue;
+  // CT columns of N-contiguous B are read at a time; fewer columns take the
   // one-tile kernel (the sums are the same)
-  if (!bvec && p.N < ct) ct = 1;
+  if (dot_brow(ct, bvec) && p.N < ct) ct = 1;
   const int64_t ncb = ((p.N + 15) / 16 + ct - 1) / ct;
   DotFn fn = find_dot(rt, ct, bvec, a_loads_cached(p.A, p.sAm, ncb));
   return fn(kw, p, st);

@@ -563,3 +563,23 @@ def test_dot_column_remainders(hml, N):
                 out = dC.to_numpy((M, N + pad))
                 np.testing.assert_array_equal(out[:, :N], R, err_msg="%r pad=%d" % (v, pad))
                 assert (out[:, N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("shape", [(3000, 33, 4000), (3001, 48, 4001), (2500, 72, 2100), (1000, 96, 9000),
+                                   (1300, 100, 2700), (700, 49, 16390), (20011, 81, 257), (600, 600, 1200)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_chosen_geometry(hml, shape):
+    """Products whose tile and K split the dispatch chooses by its model (3
+    and 4 column tiles, one and several K groups): exact on whole numbers,
+    with beta, in the workspace that hmlSgemmWorkspaceSize names and in none."""
+    M, N, K = shape
+    rng = np.random.default_rng(M + N)
+    A, B, C0 = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
+    R = exact_product(A, B, 2.0, -1.0, C0)
+    np.testing.assert_array_equal(run_gemm(hml, A, B, C0, 2.0, -1.0), R)
+    ws = hml.lib.hmlSgemmWorkspaceSize(0, 0, 0, M, N, K, None)
+    dA, dB, dC = (hml.DeviceBuffer.from_numpy(x) for x in (A, B, C0))
+    W = hml.DeviceBuffer(max(ws, 4))
+    hml.sgemm_ex(M, N, K, dA, dB, dC, 2.0, -1.0, workspace=W, ws_bytes=ws)
+    hml.synchronize()
+    np.testing.assert_array_equal(dC.to_numpy((M, N)), R)
