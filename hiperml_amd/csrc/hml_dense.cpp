@@ -67,20 +67,23 @@ hmlStatus run_dense(int prec, const float *A, int64_t sAm, int64_t sAk,
   void *Ap = ws;
   void *Bp = (char *)ws + d.a_bytes;
   uint32_t *rmA = nullptr, *rmB = nullptr;
-  hipError_t e;
+  hipError_t e = hipSuccess;
   if (prec == 3) {
-    // scaled fp16 split: zero the row maxima (a fill kernel, so the sequence
-    // can be captured), gather them, then split with the row scales
     rmA = (uint32_t *)((char *)ws + d.a_bytes + d.b_bytes);
     rmB = rmA + d.Mp;
-    e = launch_fill((float *)rmA, (size_t)(d.Mp + d.Np), 0.f, st);
-    if (e == hipSuccess) e = launch_rowmax(A, sAm, sAk, M, K, rmA, st);
-    if (e == hipSuccess) e = launch_rowmax(B, sBn, sBk, N, K, rmB, st);
-    if (e == hipSuccess) e = launch_split_f16(A, sAm, sAk, M, K, d.Mp, d.Kp, rmA, Ap, st);
-    if (e == hipSuccess) e = launch_split_f16(B, sBn, sBk, N, K, d.Np, d.Kp, rmB, Bp, st);
+  }
+  const SplitSource sa{A, sAm, sAk, M, d.Mp, Ap, rmA}, sb{B, sBn, sBk, N, d.Np, Bp, rmB};
+  if (S == 0) {
+    e = launch_pack(sa, K, d.Kp, st);
+    if (e == hipSuccess) e = launch_pack(sb, K, d.Kp, st);
   } else {
-    e = launch_split(A, sAm, sAk, M, K, d.Mp, d.Kp, S, Ap, st);
-    if (e == hipSuccess) e = launch_split(B, sBn, sBk, N, K, d.Np, d.Kp, S, Bp, st);
+    if (prec == 3) {
+      // scaled fp16 split: zero the row maxima (a fill kernel, so the sequence
+      // can be captured), gather them, then split with the row scales
+      e = launch_fill((float *)rmA, (size_t)(d.Mp + d.Np), 0.f, st);
+      if (e == hipSuccess) e = launch_rowmax(sa, sb, K, st);
+    }
+    if (e == hipSuccess) e = launch_split(prec == 3 ? 4 : S, sa, sb, K, d.Kp, st);
   }
   if (e != hipSuccess) return from_hip(e, "split/pack pass");
   DenseParams p{};

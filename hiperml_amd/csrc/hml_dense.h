@@ -32,18 +32,22 @@ struct DenseParams {
   const uint32_t *rmaxB;
 };
 
-// S: 0 = FP32 copy, 2 = hi/lo bf16, 3 = hi/mid/lo bf16.
-hipError_t launch_split(const float *src, int64_t sR, int64_t sK, int64_t rows,
-                        int64_t K, int64_t rowsP, int64_t Kp, int S, void *dst,
+// One operand X(r, k) = src[r*sR + k*sK] of a product: its planes (dst, rowsP
+// padded rows) and, for the scaled fp16 split, its row maxima.
+struct SplitSource {
+  const float *src;
+  int64_t sR, sK, rows, rowsP;
+  void *dst;
+  uint32_t *rowmax;
+};
+// FP32 copy of one operand.
+hipError_t launch_pack(const SplitSource &x, int64_t K, int64_t Kp, hipStream_t st);
+// Planes of both operands: S = 2 hi/lo bf16, 3 hi/mid/lo bf16, 4 scaled fp16
+// hi/lo from the row maxima.
+hipError_t launch_split(int S, const SplitSource &a, const SplitSource &b, int64_t K, int64_t Kp,
                         hipStream_t st);
+// rowmax[r] = max_k |X(r,k)| as FP32 bits, both operands; zero on entry.
+hipError_t launch_rowmax(const SplitSource &a, const SplitSource &b, int64_t K, hipStream_t st);
 // S: 0 FP32, 2 bf16x3, 3 bf16x6, 4 scaled f16x3.
 hipError_t launch_dense(int S, const DenseParams &p, hipStream_t st);
-// rowmax[r] = max_k |X(r,k)| as FP32 bits; rowmax must be zero on entry.
-hipError_t launch_rowmax(const float *src, int64_t sR, int64_t sK, int64_t rows,
-                         int64_t K, uint32_t *rowmax, hipStream_t st);
-// Scaled fp16 hi / lo planes (k-blocked, 2 planes) from the row maxima.
-hipError_t launch_split_f16(const float *src, int64_t sR, int64_t sK, int64_t rows,
-                            int64_t K, int64_t rowsP, int64_t Kp, const uint32_t *rowmax,
-                            void *dst, hipStream_t st);
-
 }  // namespace hml

@@ -111,14 +111,31 @@ constexpr int kLmK = 0, kLmR = 1, kLmAny = 2;
 constexpr int kSplitRows = 64;
 constexpr int kLdsStride = 33;
 
+// One operand of a row-maxima or split pass.  Both operands of a product go
+// through one launch of each pass, A's workgroups first: the passes are short
+// (bound by launches and the last wave of workgroups) until the operands are
+// tens of MB.  Whole calls, two launches -> one: f16x3 1024 x 1024 x 256
+// 28.6 -> 24.5 us, 5001 x 3003 x 1001 126 -> 121, 4096^3 415 -> 404; bf16x3
+// 2048^3 90.4 -> 88.0, 8192 x 8192 x 256 149 -> 146; equal at f16x3 8192^3.
+struct SplitOperand {
+  const float *src;
+  int64_t sR, sK, rows, K, rowsP;
+  int lm, vec;        // load mode; 16-byte loads are aligned
+  int kpb;            // row maxima: k-blocks per workgroup
+  int64_t nblk;       // workgroups of the pass
+  uint32_t *rowmax;
+  void *dst;
+};
+
 // X(r0 + i, k0 + j), i < 64, j < 32, into lt[i * 33 + j]; zero outside the
-// operand.  vec: 16-byte loads are aligned (host-checked).
-template <int LM>
-__device__ __forceinline__ void load_split_tile(const float *__restrict__ src, int64_t sR,
-                                                int64_t sK, int64_t rows, int64_t K,
-                                                int64_t r0, int64_t k0, int vec, float *lt) {
+// operand.  The load mode is the same for a whole workgroup.
+__device__ __forceinline__ void load_split_tile(const SplitOperand &o, int64_t r0, int64_t k0,
+                                                float *lt) {
   const int t = threadIdx.x;
-  if constexpr (LM == kLmK) {
+  const float *__restrict__ src = o.src;
+  const int64_t sR = o.sR, sK = o.sK, rows = o.rows, K = o.K;
+  const int vec = o.vec;
+  if (o.lm == kLmK) {
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
       const int i = (t >> 3) + 32 * it, j = (t & 7) * 4;
@@ -136,7 +153,7 @@ __device__ __forceinline__ void load_split_tile(const float *__restrict__ src, i
 #pragma unroll
       for (int e = 0; e < 4; ++e) lt[i * kLdsStride + j + e] = v[e];
     }
-  } else if constexpr (LM == kLmR) {
+  } else if (o.lm == kLmR) {
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
       const int j = (t >> 4) + 16 * it, i = (t & 15) * 4;
@@ -169,19 +186,19 @@ __device__ __forceinline__ void load_split_tile(const float *__restrict__ src, i
 // above Inf).  rowmax must be zero on entry.  Block b covers rows
 // 64 (b % nrb) .. +63 and k-blocks kpb (b / nrb) .. +kpb-1 (nrb row
 // blocks); one atomic per row and block.
-template <int LM>
-__global__ __launch_bounds__(256) void k_rowmax(const float *__restrict__ src, int64_t sR,
-                                                int64_t sK, int64_t rows, int64_t K, int vec,
-                                                int kpb, uint32_t *__restrict__ rowmax) {
+__global__ __launch_bounds__(256) void k_rowmax(SplitOperand a, SplitOperand b) {
   __shared__ float lt[kSplitRows * kLdsStride];
   const int t = threadIdx.x, i = t >> 2, q = t & 3;
-  const int64_t nrb = (rows + kSplitRows - 1) / kSplitRows;
-  const int64_t r0 = ((int64_t)blockIdx.x % nrb) * kSplitRows;
-  const int64_t kt0 = ((int64_t)blockIdx.x / nrb) * kpb;
-  const int64_t nkt = (K + kSplitKBlock - 1) / kSplitKBlock;
+  const bool second = (int64_t)blockIdx.x >= a.nblk;
+  const SplitOperand o = second ? b : a;
+  const int64_t blk = (int64_t)blockIdx.x - (second ? a.nblk : 0);
+  const int64_t nrb = (o.rows + kSplitRows - 1) / kSplitRows;
+  const int64_t r0 = (blk % nrb) * kSplitRows;
+  const int64_t kt0 = (blk / nrb) * o.kpb;
+  const int64_t nkt = (o.K + kSplitKBlock - 1) / kSplitKBlock;
   uint32_t m = 0;
-  for (int64_t kt = kt0; kt < kt0 + kpb && kt < nkt; ++kt) {
-    load_split_tile<LM>(src, sR, sK, rows, K, r0, kt * kSplitKBlock, vec, lt);
+  for (int64_t kt = kt0; kt < kt0 + o.kpb && kt < nkt; ++kt) {
+    load_split_tile(o, r0, kt * kSplitKBlock, lt);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -191,7 +208,7 @@ __global__ __launch_bounds__(256) void k_rowmax(const float *__restrict__ src, i
   // the 4 threads of a row are adjacent lanes
   m = max(m, (uint32_t)__shfl_xor((int)m, 1, 64));
   m = max(m, (uint32_t)__shfl_xor((int)m, 2, 64));
-  if (q == 0 && m && r0 + i < rows) atomicMax(rowmax + r0 + i, m);
+  if (q == 0 && m && r0 + i < o.rows) atomicMax(o.rowmax + r0 + i, m);
 }
 
 // Exponent e with max * 2^e in [2^14, 2^15) (0 for a zero, Inf or NaN max).
@@ -205,20 +222,22 @@ __device__ __forceinline__ int split_exponent(uint32_t maxbits) {
 // FP32, rounding to nearest even) or, F16, scaled fp16 hi / lo planes
 // (row r times 2^e_r from rowmax, then hi = fp16(x), lo = fp16(x - hi)),
 // in the k-blocked layout dst[s][Kp/32][rowsP][32].
-template <int S, bool F16, int LM>
-__global__ __launch_bounds__(256) void k_split_tiled(const float *__restrict__ src, int64_t sR,
-                                                     int64_t sK, int64_t rows, int64_t K,
-                                                     int64_t rowsP, int64_t Kp, int vec,
-                                                     const uint32_t *__restrict__ rowmax,
-                                                     void *__restrict__ dst) {
+template <int S, bool F16>
+__global__ __launch_bounds__(256) void k_split_tiled(SplitOperand oa, SplitOperand ob, int64_t Kp) {
   __shared__ float lt[kSplitRows * kLdsStride];
   const int t = threadIdx.x, i = t >> 2, q = t & 3;
-  // block b: row block b % nrb of k-block b / nrb, so consecutive blocks
+  const bool second = (int64_t)blockIdx.x >= oa.nblk;
+  const SplitOperand o = second ? ob : oa;
+  const int64_t blk = (int64_t)blockIdx.x - (second ? oa.nblk : 0);
+  const int64_t rows = o.rows, rowsP = o.rowsP;
+  const uint32_t *__restrict__ rowmax = o.rowmax;
+  void *__restrict__ dst = o.dst;
+  // block: row block blk % nrb of k-block blk / nrb, so consecutive blocks
   // write consecutive 4 KB pieces of each plane
   const int64_t nrb = rowsP / kSplitRows;
-  const int64_t r0 = ((int64_t)blockIdx.x % nrb) * kSplitRows;
-  const int64_t kt = (int64_t)blockIdx.x / nrb;
-  load_split_tile<LM>(src, sR, sK, rows, K, r0, kt * kSplitKBlock, vec, lt);
+  const int64_t r0 = (blk % nrb) * kSplitRows;
+  const int64_t kt = blk / nrb;
+  load_split_tile(o, r0, kt * kSplitKBlock, lt);
   __syncthreads();
   float v[8];
 #pragma unroll
@@ -537,78 +556,80 @@ int split_load_mode(const float *src, int64_t sR, int64_t sK, int64_t rows, int6
   return kLmAny;
 }
 
-template <int S, bool F16>
-hipError_t launch_split_mode(int lm, dim3 grid, hipStream_t st, const float *src, int64_t sR,
-                             int64_t sK, int64_t rows, int64_t K, int64_t rowsP, int64_t Kp,
-                             int vec, const uint32_t *rowmax, void *dst) {
-  switch (lm) {
-    case kLmK: hipLaunchKernelGGL((k_split_tiled<S, F16, kLmK>), grid, dim3(256), 0, st, src, sR, sK, rows, K, rowsP, Kp, vec, rowmax, dst); break;
-    case kLmR: hipLaunchKernelGGL((k_split_tiled<S, F16, kLmR>), grid, dim3(256), 0, st, src, sR, sK, rows, K, rowsP, Kp, vec, rowmax, dst); break;
-    default: hipLaunchKernelGGL((k_split_tiled<S, F16, kLmAny>), grid, dim3(256), 0, st, src, sR, sK, rows, K, rowsP, Kp, vec, rowmax, dst); break;
+SplitOperand split_operand(const SplitSource &x, int64_t K) {
+  SplitOperand o{};
+  o.src = x.src;
+  o.sR = x.sR;
+  o.sK = x.sK;
+  o.rows = x.rows;
+  o.K = K;
+  o.rowsP = x.rowsP;
+  o.lm = split_load_mode(x.src, x.sR, x.sK, x.rows, K, &o.vec);
+  o.rowmax = x.rowmax;
+  o.dst = x.dst;
+  return o;
+}
+
+// One launch for both operands, or one each where the sum would pass the
+// 2^32 work-items of a grid.
+template <typename Launch>
+hipError_t launch_both(const SplitOperand (&o)[2], hipStream_t st, Launch launch) {
+  if (o[0].nblk > 0x7fffffff || o[1].nblk > 0x7fffffff) return hipErrorInvalidValue;
+  if (o[0].nblk + o[1].nblk < (int64_t)1 << 24) {
+    launch(dim3((unsigned)(o[0].nblk + o[1].nblk)), st, o[0], o[1]);
+    return hipGetLastError();
   }
-  return hipGetLastError();
+  for (const SplitOperand &x : o) {
+    launch(dim3((unsigned)x.nblk), st, x, x);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace
 
-hipError_t launch_split(const float *src, int64_t sR, int64_t sK, int64_t rows,
-                        int64_t K, int64_t rowsP, int64_t Kp, int S, void *dst,
-                        hipStream_t st) {
-  if (rowsP <= 0 || Kp <= 0) return hipSuccess;
-  if (S == 0) {
-    const int64_t total = rowsP * (Kp / 8);
-    const int kfast = sK == 1 ? 1 : 0;
-    const dim3 grid((unsigned)((total + 255) / 256));
-    hipLaunchKernelGGL(k_pack_f32, grid, dim3(256), 0, st, src, sR, sK, rows, K, rowsP, Kp,
-                       (float *)dst, kfast);
-    return hipGetLastError();
-  }
-  const int64_t nblk = (rowsP / kSplitRows) * (Kp / kSplitKBlock);
-  if (rowsP % kSplitRows != 0 || Kp % kSplitKBlock != 0 || nblk > 0x7fffffff)
-    return hipErrorInvalidValue;
-  int vec = 0;
-  const int lm = split_load_mode(src, sR, sK, rows, K, &vec);
-  const dim3 grid((unsigned)nblk);
-  switch (S) {
-    case 2: return launch_split_mode<2, false>(lm, grid, st, src, sR, sK, rows, K, rowsP, Kp, vec, nullptr, dst);
-    case 3: return launch_split_mode<3, false>(lm, grid, st, src, sR, sK, rows, K, rowsP, Kp, vec, nullptr, dst);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch_rowmax(const float *src, int64_t sR, int64_t sK, int64_t rows,
-                         int64_t K, uint32_t *rowmax, hipStream_t st) {
-  if (rows <= 0 || K <= 0) return hipSuccess;
-  int vec = 0;
-  const int lm = split_load_mode(src, sR, sK, rows, K, &vec);
-  const int64_t nkt = (K + kSplitKBlock - 1) / kSplitKBlock;
-  const int64_t nrb = (rows + kSplitRows - 1) / kSplitRows;
-  // k-blocks per workgroup: up to 8 (fewer atomics), but enough workgroups
-  // (about 4096) to fill the device when the operand is small
-  const int kpb = (int)std::max<int64_t>(1, std::min<int64_t>(8, nrb * nkt / 4096));
-  const int64_t nblk = nrb * ((nkt + kpb - 1) / kpb);
-  if (nblk > 0x7fffffff) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)nblk);
-  switch (lm) {
-    case kLmK: hipLaunchKernelGGL(k_rowmax<kLmK>, grid, dim3(256), 0, st, src, sR, sK, rows, K, vec, kpb, rowmax); break;
-    case kLmR: hipLaunchKernelGGL(k_rowmax<kLmR>, grid, dim3(256), 0, st, src, sR, sK, rows, K, vec, kpb, rowmax); break;
-    default: hipLaunchKernelGGL(k_rowmax<kLmAny>, grid, dim3(256), 0, st, src, sR, sK, rows, K, vec, kpb, rowmax); break;
-  }
+hipError_t launch_pack(const SplitSource &x, int64_t K, int64_t Kp, hipStream_t st) {
+  if (x.rowsP <= 0 || Kp <= 0) return hipSuccess;
+  const int64_t total = x.rowsP * (Kp / 8);
+  const dim3 grid((unsigned)((total + 255) / 256));
+  hipLaunchKernelGGL(k_pack_f32, grid, dim3(256), 0, st, x.src, x.sR, x.sK, x.rows, K, x.rowsP, Kp,
+                     (float *)x.dst, x.sK == 1 ? 1 : 0);
   return hipGetLastError();
 }
 
-hipError_t launch_split_f16(const float *src, int64_t sR, int64_t sK, int64_t rows,
-                            int64_t K, int64_t rowsP, int64_t Kp, const uint32_t *rowmax,
-                            void *dst, hipStream_t st) {
-  if (rowsP <= 0 || Kp <= 0) return hipSuccess;
-  const int64_t nblk = (rowsP / kSplitRows) * (Kp / kSplitKBlock);
-  if (rowsP % kSplitRows != 0 || Kp % kSplitKBlock != 0 || nblk > 0x7fffffff)
+hipError_t launch_rowmax(const SplitSource &a, const SplitSource &b, int64_t K, hipStream_t st) {
+  if (a.rows <= 0 || b.rows <= 0 || K <= 0) return hipSuccess;
+  const int64_t nkt = (K + kSplitKBlock - 1) / kSplitKBlock;
+  SplitOperand o[2] = {split_operand(a, K), split_operand(b, K)};
+  for (SplitOperand &x : o) {
+    const int64_t nrb = (x.rows + kSplitRows - 1) / kSplitRows;
+    // k-blocks per workgroup: up to 8 (fewer atomics), but enough workgroups
+    // (about 4096) to fill the device when the operand is small
+    x.kpb = (int)std::max<int64_t>(1, std::min<int64_t>(8, nrb * nkt / 4096));
+    x.nblk = nrb * ((nkt + x.kpb - 1) / x.kpb);
+  }
+  return launch_both(o, st, [](dim3 grid, hipStream_t s, const SplitOperand &p, const SplitOperand &q) {
+    hipLaunchKernelGGL(k_rowmax, grid, dim3(256), 0, s, p, q);
+  });
+}
+
+hipError_t launch_split(int S, const SplitSource &a, const SplitSource &b, int64_t K, int64_t Kp,
+                        hipStream_t st) {
+  if (a.rowsP <= 0 || b.rowsP <= 0 || Kp <= 0) return hipSuccess;
+  if (S < 2 || S > 4 || a.rowsP % kSplitRows != 0 || b.rowsP % kSplitRows != 0 ||
+      Kp % kSplitKBlock != 0)
     return hipErrorInvalidValue;
-  int vec = 0;
-  const int lm = split_load_mode(src, sR, sK, rows, K, &vec);
-  const dim3 grid((unsigned)nblk);
-  return launch_split_mode<2, true>(lm, grid, st, src, sR, sK, rows, K, rowsP, Kp, vec, rowmax,
-                                    dst);
+  SplitOperand o[2] = {split_operand(a, K), split_operand(b, K)};
+  for (SplitOperand &x : o) x.nblk = (x.rowsP / kSplitRows) * (Kp / kSplitKBlock);
+  return launch_both(o, st, [=](dim3 grid, hipStream_t s, const SplitOperand &p, const SplitOperand &q) {
+    if (S == 2)
+      hipLaunchKernelGGL((k_split_tiled<2, false>), grid, dim3(256), 0, s, p, q, Kp);
+    else if (S == 3)
+      hipLaunchKernelGGL((k_split_tiled<3, false>), grid, dim3(256), 0, s, p, q, Kp);
+    else
+      hipLaunchKernelGGL((k_split_tiled<2, true>), grid, dim3(256), 0, s, p, q, Kp);
+  });
 }
 
 // Block height of the two-plane kernels (bf16x3, f16x3): 128-row tiles

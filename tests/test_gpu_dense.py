@@ -70,6 +70,21 @@ def test_small_integers_exact(hml, precision, layout):
         np.testing.assert_array_equal(C, want)
 
 
+@pytest.mark.parametrize("precision", ["bf16x3", "bf16x6", "f16x3"])
+@pytest.mark.parametrize("M,N,K", [(1, 700, 33), (700, 1, 1), (65, 2049, 31), (1025, 129, 64)])
+def test_unequal_operands_exact(hml, precision, M, N, K):
+    """Both operands go through one pass of row maxima and one split: extents
+    that put the line between them at either end of the grid, with the load
+    of each operand in either direction (exact on small integers)."""
+    rng = np.random.default_rng(M + N + K)
+    A, B = int_matrix(rng, (M, K), -8, 8), int_matrix(rng, (K, N), -8, 8)
+    want = (A.astype(np.int64) @ B.astype(np.int64)).astype(np.float32)
+    for ta in (False, True):
+        for tb in (False, True):
+            C = run_dense(hml, A, B, np.zeros((M, N), np.float32), 1.0, 0.0, precision, "row", ta, tb)
+            np.testing.assert_array_equal(C, want)
+
+
 @pytest.mark.parametrize("precision,terms", [("bf16x3", 2), ("bf16x6", 3)])
 def test_split_product_sets_exact(hml, precision, terms):
     """12-bit integers: hi has 8 significant bits and the remainder fits the
