@@ -73,18 +73,13 @@ hmlStatus run_dense(int prec, const float *A, int64_t sAm, int64_t sAk,
     rmB = rmA + d.Mp;
   }
   const SplitSource sa{A, sAm, sAk, M, d.Mp, Ap, rmA}, sb{B, sBn, sBk, N, d.Np, Bp, rmB};
-  if (S == 0) {
-    e = launch_pack(sa, K, d.Kp, st);
-    if (e == hipSuccess) e = launch_pack(sb, K, d.Kp, st);
-  } else {
-    if (prec == 3) {
-      // scaled fp16 split: zero the row maxima (a fill kernel, so the sequence
-      // can be captured), gather them, then split with the row scales
-      e = launch_fill((float *)rmA, (size_t)(d.Mp + d.Np), 0.f, st);
-      if (e == hipSuccess) e = launch_rowmax(sa, sb, K, st);
-    }
-    if (e == hipSuccess) e = launch_split(prec == 3 ? 4 : S, sa, sb, K, d.Kp, st);
+  if (prec == 3) {
+    // scaled fp16 split: zero the row maxima (a fill kernel, so the sequence
+    // can be captured), gather them, then split with the row scales
+    e = launch_fill((float *)rmA, (size_t)(d.Mp + d.Np), 0.f, st);
+    if (e == hipSuccess) e = launch_rowmax(sa, sb, K, st);
   }
+  if (e == hipSuccess) e = launch_split(prec == 3 ? 4 : S ? S : 1, sa, sb, K, d.Kp, st);
   if (e != hipSuccess) return from_hip(e, "split/pack pass");
   DenseParams p{};
   p.Ap = Ap; p.Bp = Bp; p.C = C; p.sCm = sCm; p.sCn = sCn;

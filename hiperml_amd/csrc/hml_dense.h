@@ -17,8 +17,8 @@ constexpr int kSplitKBlock = 32;  // k-block of the bf16 plane layout
 constexpr int64_t kDenseShortK = 1024;
 
 struct DenseParams {
-  // S == 0: FP32 [Mp][Kp] / [Np][Kp] (B transposed, K contiguous);
-  // S > 0:  bf16 planes, k-blocked [S][Kp/32][Mp][32] / [S][Kp/32][Np][32]
+  // S == 0: FP32, k-blocked [Kp/16][Mp][16] / [Kp/16][Np][16] (B transposed);
+  // S > 0:  16-bit planes, k-blocked [S][Kp/32][Mp][32] / [S][Kp/32][Np][32]
   const void *Ap;
   const void *Bp;
   float *C;
@@ -40,10 +40,8 @@ struct SplitSource {
   void *dst;
   uint32_t *rowmax;
 };
-// FP32 copy of one operand.
-hipError_t launch_pack(const SplitSource &x, int64_t K, int64_t Kp, hipStream_t st);
-// Planes of both operands: S = 2 hi/lo bf16, 3 hi/mid/lo bf16, 4 scaled fp16
-// hi/lo from the row maxima.
+// Planes of both operands: S = 1 an FP32 copy, 2 hi/lo bf16, 3 hi/mid/lo
+// bf16, 4 scaled fp16 hi/lo from the row maxima.
 hipError_t launch_split(int S, const SplitSource &a, const SplitSource &b, int64_t K, int64_t Kp,
                         hipStream_t st);
 // rowmax[r] = max_k |X(r,k)| as FP32 bits, both operands; zero on entry.

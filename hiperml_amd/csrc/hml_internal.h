@@ -145,6 +145,9 @@ hipError_t launch_skinny_dotb(int rt, int ct, bool bvec, const DotParams &p, hip
 hipError_t launch_skinny_dot(int rt, int ct, bool bvec, int kw, const DotParams &p,
                              hipStream_t st);
 
+// Compute units of the current device (256 if unknown).
+int device_cus();
+
 // k_skinny_rows: unsplit products of few k and many rows, rows streamed by
 // persistent waves.  `better` is the rule that sends a problem there.
 constexpr int kRowsWaves = 8;  // most waves per workgroup

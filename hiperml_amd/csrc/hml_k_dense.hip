@@ -36,8 +36,8 @@
 // while step t computes, LDS rows unpadded with the 16-byte chunk index
 // XOR-swizzled by the row (conflict-free row-contiguous writes and operand
 // reads), and an XCD-aware block order (blocks that share A/B panels run on
-// the same L2).  The plain FP32 kernel keeps K-contiguous FP32 copies and
-// 128 x 128 tiles.
+// the same L2).  The plain FP32 kernel does the same on FP32 copies with
+// 16-wide k-steps and 128 x 128 or 64 x 128 tiles.
 #include <algorithm>
 
 #include "hml_internal.h"
@@ -51,10 +51,9 @@ typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-constexpr int BM = kDenseTileM, BN = kDenseTileN;  // FP32 kernel tile
+constexpr int BN = kDenseTileN;                     // FP32 kernel tile width
 constexpr int BNH = kSplitTileN;                    // 16-bit kernels' tile width
 constexpr int BKF = 16;        // k per step, FP32 kernel
-constexpr int PADF = 4;        // float elements of LDS row padding
 
 // Round-to-nearest-even FP32 -> bf16 bits (finite inputs; NaN kept quiet).
 __device__ __forceinline__ uint32_t bf16_bits(float x) {
@@ -65,36 +64,6 @@ __device__ __forceinline__ uint32_t bf16_bits(float x) {
 }
 __device__ __forceinline__ float bf16_to_float(uint32_t b) {
   return __uint_as_float(b << 16);
-}
-
-// ---- FP32 pack pass -----------------------------------------------------------
-// K-contiguous FP32 copy [rowsP][Kp] of a rows x K operand X(r,k) =
-// src[r*sR + k*sK], zero-padded, for the plain FP32 kernel.  One thread per
-// 8 consecutive k of one row; the thread index runs fastest along whichever
-// of r / k is contiguous in src, so the reads coalesce.
-__global__ void k_pack_f32(const float *__restrict__ src, int64_t sR, int64_t sK,
-                           int64_t rows, int64_t K, int64_t rowsP, int64_t Kp,
-                           float *__restrict__ dst, int kfast) {
-  const int64_t kc_n = Kp / 8;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= rowsP * kc_n) return;
-  int64_t r, kc;
-  if (kfast) {
-    r = idx / kc_n;
-    kc = idx - r * kc_n;
-  } else {
-    kc = idx / rowsP;
-    r = idx - kc * rowsP;
-  }
-  float v[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int64_t k = kc * 8 + j;
-    v[j] = (r < rows && k < K) ? src[r * sR + k * sK] : 0.f;
-  }
-  float *d = dst + r * Kp + kc * 8;
-  *reinterpret_cast<f4 *>(d) = f4{v[0], v[1], v[2], v[3]};
-  *reinterpret_cast<f4 *>(d + 4) = f4{v[4], v[5], v[6], v[7]};
 }
 
 // ---- tiled split passes ------------------------------------------------------
@@ -221,7 +190,8 @@ __device__ __forceinline__ int split_exponent(uint32_t maxbits) {
 // bf16 planes (S = 2: hi, lo; S = 3: hi, mid, lo; each residual exact in
 // FP32, rounding to nearest even) or, F16, scaled fp16 hi / lo planes
 // (row r times 2^e_r from rowmax, then hi = fp16(x), lo = fp16(x - hi)),
-// in the k-blocked layout dst[s][Kp/32][rowsP][32].
+// in the k-blocked layout dst[s][Kp/32][rowsP][32].  S = 1: an FP32 copy in
+// 16-wide k-blocks, dst[Kp/16][rowsP][16].
 template <int S, bool F16>
 __global__ __launch_bounds__(256) void k_split_tiled(SplitOperand oa, SplitOperand ob, int64_t Kp) {
   __shared__ float lt[kSplitRows * kLdsStride];
@@ -242,6 +212,12 @@ __global__ __launch_bounds__(256) void k_split_tiled(SplitOperand oa, SplitOpera
   float v[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) v[j] = lt[i * kLdsStride + q * 8 + j];
+  if constexpr (S == 1) {
+    float *d = (float *)dst + ((2 * kt + (q >> 1)) * rowsP + r0 + i) * BKF + (q & 1) * 8;
+    *reinterpret_cast<f4 *>(d) = f4{v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<f4 *>(d + 4) = f4{v[4], v[5], v[6], v[7]};
+    return;
+  }
   const int64_t plane = rowsP * Kp;
   const int64_t off = (kt * rowsP + r0 + i) * kSplitKBlock + q * 8;
   if constexpr (F16) {
@@ -470,68 +446,104 @@ __global__ __launch_bounds__(128 * WM, 2) void k_dense_bf16(DenseParams p) {
 }
 
 // ---- plain FP32 GEMM on v_mfma_f32_16x16x4f32 ------------------------------
-__global__ __launch_bounds__(256) void k_dense_f32(DenseParams p) {
-  __shared__ __attribute__((aligned(16))) float As[2][BM][BKF + PADF];
-  __shared__ __attribute__((aligned(16))) float Bs[2][BN][BKF + PADF];
+// Float offset of 16-byte chunk kq (0..3) of LDS tile row x (16 floats = 64
+// bytes per row); the swizzle of sw_off.
+__device__ __forceinline__ int sw_off32(int x, int kq) {
+  return x * BKF + 4 * (kq ^ (((x >> 1) ^ (x >> 2)) & 3));
+}
+
+// Bound by the matrix cores (157 TF/s; the best library product of 8192^3
+// here reaches 154).  4 waves, 2 x 2, of 16 RT x 64 outputs; operands come
+// as FP32 copies in 16-wide k-blocks, so a step's panel is 4 or 8 KB of
+// contiguous memory (rows a whole K apart met in the same memory channels).
+// One barrier per 16-k step: a wave reads the next step's fragments while it
+// multiplies this one's, so the products wait for neither LDS nor loads, and
+// the LDS rows carry no padding (32 or 24 KB, up to 4 workgroups per CU).
+// Same products in the same order as before, us: 8192^3 9070 -> 8040
+// (137 TF/s), 4096^3 1205 -> 1039, 8192 x 8192 x 256 335 -> 288,
+// 3001 x 2047 x 2500 378 -> 284, 1000 x 1000 x 300 35.7 -> 20.0.  Left to the
+// compiler's schedule and capped at 168 registers (three waves per SIMD) for
+// RT = 4: an explicit MFMA / LDS / load interleave took 8620 us at 8192^3,
+// raised wave priority around the products 8650, fragments read at the start
+// of their own step 8300.
+template <int RT>
+__global__ __launch_bounds__(256, RT == 4 ? 3 : 1) void k_dense_f32(DenseParams p) {
+  constexpr int TM = 32 * RT, NA = TM / 64, NB = BN / 64;
+  __shared__ __attribute__((aligned(16))) float As[2][TM * BKF];
+  __shared__ __attribute__((aligned(16))) float Bs[2][BN * BKF];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wr = wave >> 1, wc = wave & 1;
   int64_t bm, bn;
-  block_coords(p.Mp / BM, p.Np / BN, &bm, &bn);
-  const float *Ag = (const float *)p.Ap + bm * BM * p.Kp;
-  const float *Bg = (const float *)p.Bp + bn * BN * p.Kp;
-  f4 ra[2], rb[2];
-  auto gload = [&](int64_t k0) {
+  block_coords((p.M + TM - 1) / TM, p.Np / BN, &bm, &bn);
+  const float *Ag = (const float *)p.Ap + bm * TM * BKF + 4 * tid;
+  const float *Bg = (const float *)p.Bp + bn * BN * BKF + 4 * tid;
+  const int64_t sA = p.Mp * BKF, sB = p.Np * BKF;
+  const int64_t nsteps = p.Kp / BKF;  // even: Kp is a multiple of 32
+  f4 ra[NA], rb[NB];
+  auto gload = [&](int64_t t) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int c = tid + 256 * i, row = c >> 2, kq = c & 3;
-      ra[i] = *reinterpret_cast<const f4 *>(Ag + row * p.Kp + k0 + 4 * kq);
-      rb[i] = *reinterpret_cast<const f4 *>(Bg + row * p.Kp + k0 + 4 * kq);
-    }
+    for (int i = 0; i < NA; ++i) ra[i] = *reinterpret_cast<const f4 *>(Ag + t * sA + 1024 * i);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) rb[i] = *reinterpret_cast<const f4 *>(Bg + t * sB + 1024 * i);
   };
+  const int wo = sw_off32(tid >> 2, tid & 3);  // the swizzle repeats every 16 rows
   auto lstore = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int c = tid + 256 * i, row = c >> 2, kq = c & 3;
-      *reinterpret_cast<f4 *>(&As[buf][row][4 * kq]) = ra[i];
-      *reinterpret_cast<f4 *>(&Bs[buf][row][4 * kq]) = rb[i];
-    }
-  };
-  f4 acc[4][4];
+    for (int i = 0; i < NA; ++i) *reinterpret_cast<f4 *>(&As[buf][wo + 1024 * i]) = ra[i];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NB; ++i) *reinterpret_cast<f4 *>(&Bs[buf][wo + 1024 * i]) = rb[i];
+  };
+  const int r16 = lane & 15, g = lane >> 4;
+  const int ro = sw_off32(r16, g);
+  const int ao = wr * RT * 16 * BKF + ro, bo = wc * 64 * BKF + ro;
+  struct Frag { f4 a[RT], b[4]; };
+  auto lread = [&](Frag &f, int buf) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) f.a[i] = *reinterpret_cast<const f4 *>(&As[buf][ao + i * 16 * BKF]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f.b[j] = *reinterpret_cast<const f4 *>(&Bs[buf][bo + j * 16 * BKF]);
+  };
+  f4 acc[RT][4];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-  const int r16 = lane & 15, g = lane >> 4;
-  const int64_t nsteps = p.Kp / BKF;
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  for (int64_t t = 0; t < nsteps; ++t) {
-    const int buf = (int)(t & 1);
-    if (t + 1 < nsteps) gload((t + 1) * BKF);
-    f4 fa[4], fb[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      fa[i] = *reinterpret_cast<const f4 *>(&As[buf][wr * 64 + i * 16 + r16][4 * g]);
-      fb[i] = *reinterpret_cast<const f4 *>(&Bs[buf][wc * 64 + i * 16 + r16][4 * g]);
-    }
+  // step t: load tile t + 2, read the fragments of t + 1 (stored in step
+  // t - 1), the products of t, then store tile t + 2 over tile t (its
+  // fragments were read in step t - 1).  The last two steps load the last
+  // tile again; it is not used.
+  auto step = [&](int64_t t, const Frag &cur, Frag &nxt, int buf) {
+    gload(t + 2 < nsteps ? t + 2 : nsteps - 1);
+    lread(nxt, buf ^ 1);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][e], fb[j][e], acc[i][j], 0, 0, 0);
-    if (t + 1 < nsteps) lstore(buf ^ 1);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.a[i][e], cur.b[j][e], acc[i][j], 0, 0, 0);
+    lstore(buf);
     __syncthreads();
+  };
+  Frag f0, f1;
+  gload(0);
+  lstore(0);
+  gload(1);
+  lstore(1);
+  __syncthreads();
+  lread(f0, 0);
+  __syncthreads();
+  for (int64_t t = 0; t < nsteps; t += 2) {
+    step(t, f0, f1, 0);
+    step(t + 1, f1, f0, 1);
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        store_c(p, bm * BM + wr * 64 + i * 16 + 4 * g + e,
+        store_c(p, bm * TM + (wr * RT + i) * 16 + 4 * g + e,
                 bn * BN + wc * 64 + j * 16 + r16, acc[i][j][e]);
 }
 
@@ -589,15 +601,6 @@ hipError_t launch_both(const SplitOperand (&o)[2], hipStream_t st, Launch launch
 
 }  // namespace
 
-hipError_t launch_pack(const SplitSource &x, int64_t K, int64_t Kp, hipStream_t st) {
-  if (x.rowsP <= 0 || Kp <= 0) return hipSuccess;
-  const int64_t total = x.rowsP * (Kp / 8);
-  const dim3 grid((unsigned)((total + 255) / 256));
-  hipLaunchKernelGGL(k_pack_f32, grid, dim3(256), 0, st, x.src, x.sR, x.sK, x.rows, K, x.rowsP, Kp,
-                     (float *)x.dst, x.sK == 1 ? 1 : 0);
-  return hipGetLastError();
-}
-
 hipError_t launch_rowmax(const SplitSource &a, const SplitSource &b, int64_t K, hipStream_t st) {
   if (a.rows <= 0 || b.rows <= 0 || K <= 0) return hipSuccess;
   const int64_t nkt = (K + kSplitKBlock - 1) / kSplitKBlock;
@@ -617,13 +620,15 @@ hipError_t launch_rowmax(const SplitSource &a, const SplitSource &b, int64_t K, 
 hipError_t launch_split(int S, const SplitSource &a, const SplitSource &b, int64_t K, int64_t Kp,
                         hipStream_t st) {
   if (a.rowsP <= 0 || b.rowsP <= 0 || Kp <= 0) return hipSuccess;
-  if (S < 2 || S > 4 || a.rowsP % kSplitRows != 0 || b.rowsP % kSplitRows != 0 ||
+  if (S < 1 || S > 4 || a.rowsP % kSplitRows != 0 || b.rowsP % kSplitRows != 0 ||
       Kp % kSplitKBlock != 0)
     return hipErrorInvalidValue;
   SplitOperand o[2] = {split_operand(a, K), split_operand(b, K)};
   for (SplitOperand &x : o) x.nblk = (x.rowsP / kSplitRows) * (Kp / kSplitKBlock);
   return launch_both(o, st, [=](dim3 grid, hipStream_t s, const SplitOperand &p, const SplitOperand &q) {
-    if (S == 2)
+    if (S == 1)
+      hipLaunchKernelGGL((k_split_tiled<1, false>), grid, dim3(256), 0, s, p, q, Kp);
+    else if (S == 2)
       hipLaunchKernelGGL((k_split_tiled<2, false>), grid, dim3(256), 0, s, p, q, Kp);
     else if (S == 3)
       hipLaunchKernelGGL((k_split_tiled<3, false>), grid, dim3(256), 0, s, p, q, Kp);
@@ -647,16 +652,36 @@ int dense_tile_m(int S, int64_t Kp) {
   return Kp <= kDenseShortK ? 128 : 256;
 }
 
+// Block height of the FP32 kernel.  A CU's time goes with the most rows it
+// is given, ceil(blocks / CUs) times the height, and a 64-row block costs 2 to
+// 5% more per row (more loads per product), so 64 rows where that sum is
+// clearly smaller; and where each CU has at most one 128-row block, so that
+// two waves share a SIMD.  us, 128 / 64 rows: 2048^3 189 / 163,
+// 3001 x 2047 x 2500 355 / 284, 2560 x 4096 x 1000 218 / 193,
+// 3712 x 3584 x 1000 269 / 247, 4608 x 4608 x 1000 393 / 379; the other way
+// 2816 x 4096 x 1000 221 / 226, 4096^3 1039 / 1072, 8192^3 8040 / 8270.
+int f32_tile_m(const DenseParams &p) {
+  const int64_t cus = device_cus(), nbn = p.Np / BN;
+  const int64_t n128 = (p.M + 127) / 128 * nbn, n64 = (p.M + 63) / 64 * nbn;
+  if (n128 <= cus) return 64;
+  const int64_t r128 = (n128 + cus - 1) / cus, r64 = (n64 + cus - 1) / cus;
+  return 105 * r64 < 200 * r128 ? 64 : 128;
+}
+
 hipError_t launch_dense(int S, const DenseParams &p, hipStream_t st) {
   // S: 0 FP32, 2 bf16x3, 3 bf16x6, 4 scaled f16x3
-  const int tm = S == 0 ? BM : dense_tile_m(S, p.Kp);
-  const int64_t nblk = S == 0 ? (p.Mp / BM) * (p.Np / BN) : (p.Mp / tm) * (p.Np / BNH);
+  const int tm = S == 0 ? f32_tile_m(p) : dense_tile_m(S, p.Kp);
+  const int64_t nblk =
+      S == 0 ? (p.M + tm - 1) / tm * (p.Np / BN) : (p.Mp / tm) * (p.Np / BNH);
   if (nblk <= 0) return hipSuccess;
   if (nblk > 0x7fffffff) return hipErrorInvalidConfiguration;
   const dim3 grid((unsigned)nblk);
   const bool t128 = tm == 128;
   switch (S) {
-    case 0: hipLaunchKernelGGL(k_dense_f32, grid, dim3(256), 0, st, p); break;
+    case 0:
+      if (t128) hipLaunchKernelGGL(k_dense_f32<4>, grid, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL(k_dense_f32<2>, grid, dim3(256), 0, st, p);
+      break;
     case 2:
       if (t128) hipLaunchKernelGGL((k_dense_bf16<2, false, 2>), grid, dim3(256), 0, st, p);
       else hipLaunchKernelGGL((k_dense_bf16<2, false, 4>), grid, dim3(512), 0, st, p);

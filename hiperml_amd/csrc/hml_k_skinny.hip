@@ -30,6 +30,17 @@
 #include "hml_kdev.h"
 
 namespace hml {
+
+int device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  return n > 0 ? n : 256;
+}
+
 namespace {
 
 __device__ __forceinline__ f4 mfma4(float a, float b, f4 c) {
@@ -1482,17 +1493,6 @@ DotbFn find_dotb(int rt, int ct, bool bv) {
     case 36: return dotb_fn<2, 4>(bv);
     default: return nullptr;
   }
-}
-
-// Compute units of the current device (256 if unknown).
-int device_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-    (void)hipGetLastError();
-    return 256;
-  }
-  return n > 0 ? n : 256;
 }
 
 // Workgroups (256 threads, dynamic LDS `lds`) of kernel `fn` the current

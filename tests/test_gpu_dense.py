@@ -85,6 +85,21 @@ def test_unequal_operands_exact(hml, precision, M, N, K):
             np.testing.assert_array_equal(C, want)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (64, 128, 16), (65, 129, 17), (2049, 2049, 33),
+                                   (2112, 2000, 40), (4100, 1030, 64), (3000, 4000, 48)])
+def test_fp32_block_heights_exact(hml, M, N, K):
+    """Both block heights of the plain FP32 kernel (64 rows where the last
+    round of 128-row blocks would leave CUs idle: the first six; 128 rows:
+    the last), remainders of a block, of a k-step and of the k padding."""
+    rng = np.random.default_rng(M + N + K)
+    A, B = int_matrix(rng, (M, K), -8, 8), int_matrix(rng, (K, N), -8, 8)
+    C0 = int_matrix(rng, (M, N), -8, 8)
+    want = (A.astype(np.float64) @ B.astype(np.float64) - C0).astype(np.float32)
+    for order, ta, tb in (("row", False, False), ("col", True, False), ("row", True, True)):
+        C = run_dense(hml, A, B, C0, 1.0, -1.0, "fp32", order, ta, tb)
+        np.testing.assert_array_equal(C, want)
+
+
 @pytest.mark.parametrize("precision,terms", [("bf16x3", 2), ("bf16x6", 3)])
 def test_split_product_sets_exact(hml, precision, terms):
     """12-bit integers: hi has 8 significant bits and the remainder fits the
