@@ -173,7 +173,9 @@ size_t hmlSgemmWorkspaceSize(hmlOrder order, hmlOp transA, hmlOp transB,
  * order is given with hmlSelectorInstall).  Where a DOT-form variant is selected
  * for many rows of few k (K <= 128, M >= 65536), hmlSgemmEx runs a
  * row-streaming kernel in its place, with the results of an unsplit DOT
- * variant; hmlSgemmExVariant runs the variant it is given. */
+ * variant, and for more than 32 columns of row-major B it may run a DOT
+ * variant in another tile and K split (never more partial sums nor longer
+ * chains); hmlSgemmExVariant runs the variant it is given. */
 hmlStatus hmlSgemmSelect(hmlOrder order, hmlOp transA, hmlOp transB,
                          int64_t M, int64_t N, int64_t K, float beta,
                          hmlSgemmVariant *variant, int32_t *source);
