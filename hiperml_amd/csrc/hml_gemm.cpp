@@ -416,6 +416,27 @@ void dot_geometry(const GemmKey &k, hmlSgemmVariant *v) {
           out = c;
         }
       }
+  // Wide products left on split 2x4 tiles: where they come to an odd number
+  // of workgroups per CU (two share one) the last runs alone, with nothing
+  // to hide its loads.  1x4 in the same split (the same chains and partial
+  // sums) is then ahead where it needs no more half rounds and B, which it
+  // reads twice as often, is small.  us, 2x4 / 1x4: 3333 x 1234 x 2345
+  // 216 / 196, 2759 x 1928 x 2880 298 / 277, 3800 x 600 x 4000 193 / 180,
+  // 5000 x 700 x 2300 169 / 161, 3000 x 2900 x 1600 283 / 262; an even number:
+  // 3001 x 2047 x 2500 274 / 286, 4000 x 1000 x 2200 165 / 179; B of 33 MB:
+  // 2759 x 2047 x 4000 391 / 417.
+  if (out.rt == 2 && out.ct == 4 && out.ksplit > 1 && k.N >= 512 &&
+      k.K * k.N * 4 <= (int64_t)28 << 20) {
+    hmlSgemmVariant c = out;
+    c.rt = 1;
+    const SkinnyPlan p2 = plan_skinny(k, out), p1 = plan_skinny(k, c);
+    const int64_t nb = ceil_div(k.N, 64), nch = ceil_div(k.K, p2.kchunk);
+    const int64_t r2 = ceil_div(ceil_div(k.M, 32) * nb * nch, 1024);
+    const int64_t r1 = ceil_div(ceil_div(k.M, 16) * nb * nch, 1024);
+    if (p1.p_floats <= p2.p_floats && p1.kchunk == p2.kchunk && p1.kw == p2.kw && r2 % 2 == 1 &&
+        r1 <= 2 * r2)
+      out = c;
+  }
   *v = out;
 }
 

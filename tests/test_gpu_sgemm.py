@@ -583,3 +583,12 @@ def test_chosen_geometry(hml, shape):
     hml.sgemm_ex(M, N, K, dA, dB, dC, 2.0, -1.0, workspace=W, ws_bytes=ws)
     hml.synchronize()
     np.testing.assert_array_equal(dC.to_numpy((M, N)), R)
+
+
+@pytest.mark.parametrize("M,N,K", [(2000, 600, 2880), (2001, 515, 2003), (3000, 600, 2880)])
+def test_wide_odd_rounds(hml, M, N, K):
+    """Wide products whose split 2x4 tiles come to an odd number of workgroups
+    per CU (1x4 in the same split) and, the last, to an even one."""
+    rng = np.random.default_rng(M + K)
+    A, B, C0 = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
+    np.testing.assert_array_equal(run_gemm(hml, A, B, C0, 2.0, -1.0), exact_product(A, B, 2.0, -1.0, C0))
