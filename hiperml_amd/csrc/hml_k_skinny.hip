@@ -271,11 +271,12 @@ __device__ __forceinline__ void buf_load_n(__amdgpu_buffer_rsrc_t rs, uint32_t v
 // instruction q loads row 4q + g, chunk r ^ ((4q + g) % 16): the same 4 rows
 // x 256 bytes per instruction, landing in the swizzled tile layout.  The
 // compiler does not order these LDS writes against the tile's reads, so the
-// waits are explicit: before a stage's reads, vmcnt(NQ) (only the NQ loads
-// of the stage issued last may still be in flight: the loads of the stage
-// being read and its B came earlier; SPREAD: also the second half of the
-// stage's own 16 loads of B, issued in between), and before a tile is refilled,
-// lgkmcnt(0) (its reads are done).
+// waits are explicit, and they count on the order in which loads are issued
+// (A and B of stage 0, 1, ...): A0 A1 B0, then in stage s B(s+1) and A(s+2).
+// Scheduling barriers keep it.  Behind the loads of the stage being read
+// there are so the NQ of the next stage's A and at least one stage of B.
+// Before a stage's reads: vmcnt(NQ); SPREAD, with 16 loads of B per stage,
+// vmcnt(NQ + 8).  Before a tile is refilled: lgkmcnt(0) (its reads are done).
 template <int RT, int CT, bool BVEC, bool DMA, int APOL = kBufNT>
 __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_t sAm,
                                              const float *__restrict__ B, int64_t sBk,
@@ -442,9 +443,15 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
   };
 
   if constexpr (DMA) {
-    // Stage t lands in tile t % PS, PS stages ahead; B one stage ahead.
+    // Stage t lands in tile t % PS, PS stages ahead; B one stage ahead.  The
+    // waits below need the first stages in this order, and B behind them:
+    // were B's loads issued first, the first stage's wait would leave its own
+    // tile in flight.
 #pragma unroll
-    for (int j = 0; j < PS; ++j) loadA(j, j);
+    for (int j = 0; j < PS; ++j) {
+      loadA(j, j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     loadBu(0, 0);
     loadBu(1, 0);
     __builtin_amdgcn_sched_barrier(0);
