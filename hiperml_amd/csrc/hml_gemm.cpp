@@ -397,8 +397,9 @@ double dot_model_us(const GemmKey &k, const hmlSgemmVariant &v) {
 // chunks instead of 8 would be 77 us instead of 81, at 1.4 times the error).
 // Unsplit 32-row tiles stay out: single-wave workgroups with 16 KB of LDS
 // each fill the chip unevenly (2500 x 2500 x 1000 169 us, unsplit 16-row tiles
-// 139).
-void dot_geometry(const GemmKey &k, hmlSgemmVariant *v) {
+// 139).  Nor does it take a tile whose rows are too far apart for the skinny
+// kernels' offsets where the chosen variant's are not.
+void dot_geometry(const GemmCanon &g, const GemmKey &k, hmlSgemmVariant *v) {
   if ((double)k.M * (double)k.N * (double)k.K < 3.5e8) return;
   const SkinnyPlan from = plan_skinny(k, *v);
   hmlSgemmVariant out = *v;
@@ -410,6 +411,7 @@ void dot_geometry(const GemmKey &k, hmlSgemmVariant *v) {
         const hmlSgemmVariant c{HML_SGEMM_FAMILY_DOT, rt, ct, ks, 4};
         const SkinnyPlan pl = plan_skinny(k, c);
         if (pl.p_floats > from.p_floats || pl.kchunk > from.kchunk) continue;
+        if (!skinny_offsets_fit(g, c, pl)) continue;
         const double us = dot_model_us(k, c);
         if (us < best) {
           best = us;
@@ -470,7 +472,7 @@ hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
     p.alpha = alpha; p.beta = beta; p.read_c = read_c;
     return from_hip(launch_skinny_rows(p, st), "row-streaming kernel launch");
   }
-  if (chosen && v.family == HML_SGEMM_FAMILY_DOT && k.N > 32 && g.sBk != 1) dot_geometry(k, &v);
+  if (chosen && v.family == HML_SGEMM_FAMILY_DOT && k.N > 32 && g.sBk != 1) dot_geometry(g, k, &v);
   if (v.family == HML_SGEMM_FAMILY_GEMV)
     return run_gemv_family(g, k, v, alpha, beta, read_c, ws, st);
   if (v.family == HML_SGEMM_FAMILY_GEMVN) {

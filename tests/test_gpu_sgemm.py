@@ -592,3 +592,26 @@ def test_wide_odd_rounds(hml, M, N, K):
     rng = np.random.default_rng(M + K)
     A, B, C0 = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
     np.testing.assert_array_equal(run_gemm(hml, A, B, C0, 2.0, -1.0), exact_product(A, B, 2.0, -1.0, C0))
+
+
+def test_chosen_geometry_large_stride(hml):
+    """The dispatch may widen a chosen 16-row tile to 32 rows.  Rows so far
+    apart that 16 of them fit the skinny kernels' 31-bit offsets and 32 do not
+    stay on a tile that fits, in the workspace that hmlSgemmWorkspaceSize
+    names and in none."""
+    M, N, K, lda = 129, 115, 26401, 18 << 20
+    rng = np.random.default_rng(12)
+    A, B = int_matrix(rng, (M, K)), int_matrix(rng, (K, N))
+    dA = hml.DeviceBuffer(4 * ((M - 1) * lda + K))
+    for i in range(M):
+        row = np.ascontiguousarray(A[i])
+        hml.check(hml.lib.hmlMemcpyHtoD(dA.ptr + 4 * i * lda, row.ctypes.data, row.nbytes))
+    dB, dC = hml.DeviceBuffer.from_numpy(B), hml.DeviceBuffer(4 * M * N)
+    ws = hml.lib.hmlSgemmWorkspaceSize(0, 0, 0, M, N, K, None)
+    W = hml.DeviceBuffer(max(ws, 4))
+    for kw in (dict(workspace=W, ws_bytes=ws), {}):
+        hml.check(hml.lib.hmlMemsetD8(dC.ptr, 0, 4 * M * N))
+        hml.sgemm_ex(M, N, K, dA, dB, dC, lda=lda, **kw)
+        hml.synchronize()
+        np.testing.assert_array_equal(dC.to_numpy((M, N)), exact_product(A, B))
+    dA.free()
