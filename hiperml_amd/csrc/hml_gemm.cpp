@@ -457,11 +457,15 @@ hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
     return fail(HML_STATUS_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes",
                 ws_bytes, need);
   }
-  // A chosen (not named) DOT-form variant gives way to the row-streaming
-  // kernel where that one is better.
-  if (chosen && k.form == kFormDot &&
-      (v.family == HML_SGEMM_FAMILY_DOT || v.family == HML_SGEMM_FAMILY_DOTB ||
-       v.family == HML_SGEMM_FAMILY_GEMVN) &&
+  // A chosen (not named) unsplit tile variant gives way to the row-streaming
+  // kernel where that one is better: the sums are the same.  A variant that
+  // splits K, over chunks or over a row's lanes (GEMVN), adds in shorter
+  // chains and stays; but not GEMVN with two columns, the heuristic's choice
+  // for any K: 10^6 x 2 x 127 409 us against 87, 65545 x 2 x 48 20.6 against
+  // 6.9 (relative error 0.77e-7 against 2.0e-7, 0.66e-7 against 1.25e-7).
+  const bool tile = (v.family == HML_SGEMM_FAMILY_DOT || v.family == HML_SGEMM_FAMILY_DOTB) &&
+                    plan_skinny(k, v).kchunk >= k.K;
+  if (chosen && (tile || (v.family == HML_SGEMM_FAMILY_GEMVN && k.N == 2)) &&
       skinny_rows_better(g.M, g.N, g.K, g.sAm)) {
     DotParams p{};
     p.A = g.A; p.sAm = g.sAm;

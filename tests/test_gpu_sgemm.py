@@ -615,3 +615,27 @@ def test_chosen_geometry_large_stride(hml):
         hml.synchronize()
         np.testing.assert_array_equal(dC.to_numpy((M, N)), exact_product(A, B))
     dA.free()
+
+
+@pytest.mark.parametrize("N,K,variant", [(8, 65, (8, 16, 1, 1, 2)), (4, 100, (8, 16, 2, 1, 4)),
+                                         (24, 100, (1, 2, 2, 2, 4)), (48, 127, (7, 1, 4, 2, 4))])
+def test_split_sums_stay_split(hml, N, K, variant):
+    """Many rows of few k where the selected variant splits K over lanes
+    (family 8) or chunks: that kernel runs, not one with longer chains of
+    additions: its very bits, and an error below the unsplit tile's.  The
+    selection comes from a table rule of a neighbouring shape."""
+    M = 65536 + 9
+    rng = np.random.default_rng(K)
+    A, B, C0 = uniform(rng, (M, K)), uniform(rng, (K, N)), uniform(rng, (M, N))
+    near = hml.GemmShape(4 * M, N, K, 0, 0, 0, 1)
+    rule = hml.SgemmVariant(*variant)
+    hml.check(hml.lib.hmlSgemmConfigAddRule(ctypes.byref(near), ctypes.byref(rule)))
+    try:
+        assert hml.sgemm_select(M, N, K)[0].astuple() == variant
+        got = run_gemm(hml, A, B, C0, 1.0, 0.0)
+    finally:
+        hml.config_clear()
+    np.testing.assert_array_equal(got, run_gemm(hml, A, B, C0, 1.0, 0.0, variant=variant))
+    R = f64_ref(A, B)[0]
+    tile = run_gemm(hml, A, B, C0, 1.0, 0.0, variant=(1, 1, 1, 1, 1))
+    assert np.linalg.norm(got - R) < np.linalg.norm(tile - R)
