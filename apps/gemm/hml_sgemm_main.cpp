@@ -86,8 +86,11 @@ static double run_test(float *C, const float *A, const float *B, int M, int N,
   std::vector<double> g;
   for (int t = 0; t < trials; ++t) {
     const double t0 = wall_secs();
-    s = hmlSgemmExVariant(HML_ROW_MAJOR, HML_OP_N, HML_OP_N, M, N, K, alpha, dA, K, dB, N,
-                          beta, dC, N, HML_FLAG_READ_C_ALWAYS, &basic_v, nullptr, 0, nullptr);
+    s = basic ? hmlSgemmExVariant(HML_ROW_MAJOR, HML_OP_N, HML_OP_N, M, N, K, alpha, dA, K, dB,
+                                  N, beta, dC, N, HML_FLAG_READ_C_ALWAYS, &basic_v, nullptr, 0,
+                                  nullptr)
+              : hmlSgemmEx(HML_ROW_MAJOR, HML_OP_N, HML_OP_N, M, N, K, alpha, dA, K, dB, N, beta,
+                           dC, N, HML_FLAG_READ_C_ALWAYS, nullptr, 0, nullptr);
     if (s == HML_STATUS_SUCCESS) s = hmlDeviceSynchronize();
     const double t1 = wall_secs();
     if (s) {

@@ -624,13 +624,15 @@ void sgemm_compat(float *C, const float *A, const float *B, int M, int N,
   GemmKey key = make_key(g, beta, HML_FLAG_READ_C_ALWAYS, HML_ROW_MAJOR,
                          HML_OP_N, HML_OP_N);
   int src = 0;
+  // the basic variant is named; otherwise the call below chooses as
+  // hmlSgemmEx does, and the line printed tells the selector's answer
   if (basic) basic_sgemm(key, &v); else select_sgemm(key, &v, &src);
   if (verbosity() >= 1 && !basic)
     fprintf(stderr, "Info: kernel type = %d, colStops = %d, rowStops = %d\n",
             v.family, v.ct, v.rt);
   s = sgemm_impl(HML_ROW_MAJOR, HML_OP_N, HML_OP_N, M, N, K, alpha, dA,
                  std::max(K, 1), dB, std::max(N, 1), beta, dC, std::max(N, 1),
-                 HML_FLAG_READ_C_ALWAYS, &v, nullptr, 0, nullptr, nullptr);
+                 HML_FLAG_READ_C_ALWAYS, basic ? &v : nullptr, nullptr, 0, nullptr, nullptr);
   if (s != HML_STATUS_SUCCESS) {
     fprintf(stderr, "Run kernel: %s\n", hmlLastError());
     exit(1);

@@ -639,3 +639,15 @@ def test_split_sums_stay_split(hml, N, K, variant):
     R = f64_ref(A, B)[0]
     tile = run_gemm(hml, A, B, C0, 1.0, 0.0, variant=(1, 1, 1, 1, 1))
     assert np.linalg.norm(got - R) < np.linalg.norm(tile - R)
+
+
+@pytest.mark.parametrize("M,N,K", [(1000, 96, 9000), (700, 49, 16390), (1300, 100, 2700), (65545, 2, 127),
+                                   (70000, 40, 31), (3000, 16, 500)])
+def test_host_entry_runs_the_device_entry(hml, M, N, K):
+    """hmlSgemm on host arrays gives the bits that hmlSgemmEx gives on device
+    buffers, also where the dispatch replaces the selected variant."""
+    rng = np.random.default_rng(M + K)
+    A, B, C0 = uniform(rng, (M, K)), uniform(rng, (K, N)), uniform(rng, (M, N))
+    C = C0.copy()
+    hml.sgemm(C, A, B, 1.5, 0.5)
+    np.testing.assert_array_equal(C, run_gemm(hml, A, B, C0, 1.5, 0.5, flags=hml.FLAG_READ_C_ALWAYS))
