@@ -230,7 +230,7 @@ def main():
         if kind == "sgemv":
             vv, src = hml.sgemv_select(shp[0], shp[1], trans=shp[2])
         else:
-            vv, src = hml.sgemm_select(*shp)
+            vv, src = hml.sgemm_resolve(*shp)
         shapes.append({"call": label, "variant": list(vv.astuple()), "selected_by": src,
                        "ms": round(ms, 5), "GB_s": round(gbs, 1),
                        "GFLOP_s": round(gfl, 1),
@@ -412,7 +412,7 @@ def bench_reference_shape(hml, cpu=True, reps=20):
     nbytes = 4.0 * (M * K + K * N + M * N)
     gpu = dC.to_numpy((M, N))
     st = hml.check_f64(M, N, K, dA, dB, dC)
-    v, src = hml.sgemm_select(M, N, K)
+    v, src = hml.sgemm_resolve(M, N, K)
     out = {"workload": "row-major SGEMM C = A B, M = K = 2048, N = 16, uniform[-1,1] (seed 2048)",
            "variant": list(v.astuple()), "gpu_cold_ms": round(cold_ms, 5),
            "gpu_warm_ms": round(warm, 5),

@@ -432,6 +432,21 @@ def sgemm_select(M, N, K, order="row", transA=False, transB=False, beta=0.0):
     return v, src.value
 
 
+def sgemm_resolve(M, N, K, order="row", transA=False, transB=False, beta=0.0, lda=None, ldb=None,
+                  ldc=None, flags=0):
+    """The variant that sgemm_ex runs for these arguments, and its source
+    (sgemm_select: what the selectors answer, before the dispatch's rules)."""
+    o, ta, tb = _order(order), _op(transA), _op(transB)
+    lda = lda or (_ld(o, M, K) if ta == OP_N else _ld(o, K, M))
+    ldb = ldb or (_ld(o, K, N) if tb == OP_N else _ld(o, N, K))
+    ldc = ldc or _ld(o, M, N)
+    v = SgemmVariant()
+    src = ctypes.c_int32()
+    check(lib.hmlSgemmResolve(o, ta, tb, M, N, K, lda, ldb, ldc, beta, flags, ctypes.byref(v),
+                              ctypes.byref(src)))
+    return v, src.value
+
+
 def sgemv_select(M, N, order="row", trans=False, beta=0.0):
     v = SgemvVariant()
     src = ctypes.c_int32()

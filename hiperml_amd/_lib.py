@@ -90,6 +90,9 @@ _SIGS = {
     "hmlSgemmSelect": (c_i32, [c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
                                ctypes.c_float, ctypes.POINTER(SgemmVariant),
                                ctypes.POINTER(c_i32)]),
+    "hmlSgemmResolve": (c_i32, [c_i32, c_i32, c_i32, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64,
+                                ctypes.c_float, c_u32, ctypes.POINTER(SgemmVariant),
+                                ctypes.POINTER(c_i32)]),
     "hmlSgemmDense": (c_i32, [c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
                               ctypes.c_float, c_void_p, c_i64, c_void_p, c_i64,
                               ctypes.c_float, c_void_p, c_i64, c_u32, c_void_p,

@@ -181,6 +181,16 @@ std::vector<hmlSgemmVariant> sgemm_candidates(const GemmKey &k) {
         if (ks <= std::max<int64_t>(1, k.K / 256) && sgemm_variant_runnable(k, v)) push_unique(&out, v);
       }
   }
+  // Tiles of 3 column tiles, and the row-streaming kernel for few k.
+  if (k.N > 32) {
+    for (int rt : {1, 2})
+      for (int ks = 1; ks <= std::max<int64_t>(1, std::min<int64_t>(64, k.K / 128)); ks *= 2) {
+        const hmlSgemmVariant v{HML_SGEMM_FAMILY_DOT, rt, 3, ks, 4};
+        if (sgemm_variant_runnable(k, v)) push_unique(&out, v);
+      }
+  }
+  const hmlSgemmVariant rows{HML_SGEMM_FAMILY_ROWS, 1, 1, 1, 4};
+  if (sgemm_variant_runnable(k, rows)) push_unique(&out, rows);
   if (sgemm_variant_runnable(k, h)) push_unique(&out, h);
   return out;
 }

@@ -98,6 +98,8 @@ GemmKey make_key(const GemmCanon &g, float beta, uint32_t flags, hmlOrder order,
   k.gemv_ok = g.N == 1 && (g.sBk == 1 || g.K == 1) && (g.sCm == 1 || g.M == 1);
   k.cM = g.swapped ? g.N : g.M;
   k.cN = g.swapped ? g.M : g.N;
+  k.b_rows = g.sBk != 1;
+  k.rows_ok = g.form == kFormDot && skinny_rows_fit(g.K, g.sAm);
   return k;
 }
 
@@ -285,7 +287,11 @@ bool sgemm_variant_runnable(const GemmKey &k, const hmlSgemmVariant &v) {
   if (v.family == HML_SGEMM_FAMILY_DOT)
     return k.form == kFormDot && v.ksplit >= 1 && v.ksplit <= 4096 &&
            (v.wpb == 1 || v.wpb == 2 || v.wpb == 4 || v.wpb == 8) &&
-           skinny_dot_runnable(v.rt, v.ct, v.wpb);
+           (v.ct == 3 ? k.b_rows && k.N >= 3 && skinny_dot3_runnable(v.rt, v.wpb)
+                      : skinny_dot_runnable(v.rt, v.ct, v.wpb));
+  if (v.family == HML_SGEMM_FAMILY_ROWS)
+    return k.rows_ok && k.K <= kRowsMaxK && k.N <= kRowsMaxN && v.rt == 1 && v.ct == 1 &&
+           v.ksplit == 1 && v.wpb == 4;
   if (v.family == HML_SGEMM_FAMILY_AXPY)
     return k.form == kFormAxpy && v.ksplit >= 1 && v.ksplit <= 4096 &&
            skinny_axpy_runnable(v.rt, v.ct, v.wpb);
@@ -304,11 +310,13 @@ bool sgemm_variant_runnable(const GemmKey &k, const hmlSgemmVariant &v) {
   return false;
 }
 
-void select_sgemm(const GemmKey &k, hmlSgemmVariant *v, int *source) {
+void select_sgemm(const GemmKey &k, hmlSgemmVariant *v, int *source, bool *exact) {
   // A table rule for this exact shape bucket is the exhaustive autotuner's
   // own measurement: it outranks the learned selector, which generalises
   // from other shapes; a more distant rule ranks below it.
+  if (exact) *exact = true;
   if (config_select_sgemm(k, v, source, true) && sgemm_variant_runnable(k, *v)) return;
+  if (exact) *exact = false;
   if (learned_select_sgemm(k, v) && sgemm_variant_runnable(k, *v)) {
     *source = 2;
     return;
@@ -332,6 +340,7 @@ size_t workspace_bytes(const GemmKey &k, const hmlSgemmVariant &v) {
     const int64_t cols = v.family == HML_SGEMM_FAMILY_GEMVN ? k.N : 1;
     return slots > 1 ? align256((size_t)slots * k.M * cols * sizeof(float)) : 0;
   }
+  if (v.family == HML_SGEMM_FAMILY_ROWS) return 0;
   const SkinnyPlan pl = plan_skinny(k, v);
   return align256(pl.p_floats * sizeof(float));
 }
@@ -442,10 +451,31 @@ void dot_geometry(const GemmCanon &g, const GemmKey &k, hmlSgemmVariant *v) {
   *v = out;
 }
 
-hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
-                    hmlSgemmVariant v, bool chosen, float alpha, float beta,
-                    int read_c, void *ws, size_t ws_bytes, hipStream_t st) {
-  const size_t need = workspace_bytes(k, v);
+// The variant to run in place of v, a selector's choice other than a table
+// rule of the problem's own bucket (which is a measurement of such problems:
+// it runs as it is).  It needs no more workspace.
+//
+// An unsplit tile gives way to the row-streaming kernel where that one is
+// better: the sums are the same.  A variant that splits K, over chunks or over
+// a row's lanes (GEMVN), adds in shorter chains and stays; but not GEMVN with
+// two columns, the heuristic's choice for any K: 10^6 x 2 x 127 409 us against
+// 87, 65545 x 2 x 48 20.6 against 6.9 (relative error 0.77e-7 against 2.0e-7,
+// 0.66e-7 against 1.25e-7).
+void resolve_choice(const GemmCanon &g, const GemmKey &k, hmlSgemmVariant *v) {
+  const bool tile = (v->family == HML_SGEMM_FAMILY_DOT || v->family == HML_SGEMM_FAMILY_DOTB) &&
+                    plan_skinny(k, *v).kchunk >= k.K;
+  const hmlSgemmVariant rows{HML_SGEMM_FAMILY_ROWS, 1, 1, 1, 4};
+  if ((tile || (v->family == HML_SGEMM_FAMILY_GEMVN && k.N == 2)) &&
+      sgemm_variant_runnable(k, rows) && skinny_rows_better(k.M, k.N, k.K))
+    *v = rows;
+  else if (v->family == HML_SGEMM_FAMILY_DOT && k.N > 32 && k.b_rows)
+    dot_geometry(g, k, v);
+}
+
+// `need` bytes of workspace are asked for (v's own or more).
+hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k, const hmlSgemmVariant &v, size_t need,
+                    float alpha, float beta, int read_c, void *ws, size_t ws_bytes,
+                    hipStream_t st) {
   void *const caller_ws = ws;
   WsLease lease;  // held until the kernels below are queued
   if (need > 0 && !ws) {
@@ -457,16 +487,7 @@ hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
     return fail(HML_STATUS_WORKSPACE_TOO_SMALL, "workspace %zu < %zu bytes",
                 ws_bytes, need);
   }
-  // A chosen (not named) unsplit tile variant gives way to the row-streaming
-  // kernel where that one is better: the sums are the same.  A variant that
-  // splits K, over chunks or over a row's lanes (GEMVN), adds in shorter
-  // chains and stays; but not GEMVN with two columns, the heuristic's choice
-  // for any K: 10^6 x 2 x 127 409 us against 87, 65545 x 2 x 48 20.6 against
-  // 6.9 (relative error 0.77e-7 against 2.0e-7, 0.66e-7 against 1.25e-7).
-  const bool tile = (v.family == HML_SGEMM_FAMILY_DOT || v.family == HML_SGEMM_FAMILY_DOTB) &&
-                    plan_skinny(k, v).kchunk >= k.K;
-  if (chosen && (tile || (v.family == HML_SGEMM_FAMILY_GEMVN && k.N == 2)) &&
-      skinny_rows_better(g.M, g.N, g.K, g.sAm)) {
+  if (v.family == HML_SGEMM_FAMILY_ROWS) {
     DotParams p{};
     p.A = g.A; p.sAm = g.sAm;
     p.B = g.B; p.sBk = g.sBk; p.sBn = g.sBn;
@@ -476,7 +497,6 @@ hmlStatus run_sgemm(const GemmCanon &g, const GemmKey &k,
     p.alpha = alpha; p.beta = beta; p.read_c = read_c;
     return from_hip(launch_skinny_rows(p, st), "row-streaming kernel launch");
   }
-  if (chosen && v.family == HML_SGEMM_FAMILY_DOT && k.N > 32 && g.sBk != 1) dot_geometry(g, k, &v);
   if (v.family == HML_SGEMM_FAMILY_GEMV)
     return run_gemv_family(g, k, v, alpha, beta, read_c, ws, st);
   if (v.family == HML_SGEMM_FAMILY_GEMVN) {
@@ -589,18 +609,23 @@ hmlStatus sgemm_impl(hmlOrder order, hmlOp ta, hmlOp tb, int64_t M, int64_t N,
   }
   GemmKey key = make_key(g, beta, flags, order, ta, tb);
   hmlSgemmVariant v;
+  size_t need;
   if (forced) {
     v = *forced;
     if (!sgemm_variant_runnable(key, v))
       return fail(HML_STATUS_NO_KERNEL,
                   "variant family=%d rt=%d ct=%d ksplit=%d wpb=%d cannot run form %d",
                   v.family, v.rt, v.ct, v.ksplit, v.wpb, key.form);
+    need = workspace_bytes(key, v);
   } else {
     int src;
-    select_sgemm(key, &v, &src);
+    bool exact;
+    select_sgemm(key, &v, &src, &exact);
+    need = workspace_bytes(key, v);
+    if (!exact) resolve_choice(g, key, &v);
   }
   if (used) *used = v;
-  return run_sgemm(g, key, v, !forced, alpha, beta, read_c, ws, ws_bytes, st);
+  return run_sgemm(g, key, v, need, alpha, beta, read_c, ws, ws_bytes, st);
 }
 
 // Host-pointer compatibility path (src/hml_sgemm.cu:39-113,120-211).
@@ -683,11 +708,16 @@ size_t hmlSgemmWorkspaceSize(hmlOrder order, hmlOp transA, hmlOp transB,
   GemmCanon g = dense_canon(order, transA, transB, M, N, K);
   // The strides and beta are unknown here: when N == 1 after orientation
   // the call may take either the GEMV or the skinny route, and a selector
-  // may choose differently for beta == 0 and beta != 0.  Return the largest
-  // need over those cases.
+  // may choose differently for beta == 0 and beta != 0, and where a table
+  // names the row-streaming kernel, whether that one runs is a matter of lda.
+  // Return the largest need over those cases.
   size_t need = 0;
-  for (int beta_nz = 0; beta_nz <= 1; ++beta_nz) {
-    GemmKey key = make_key(g, beta_nz ? 1.0f : 0.0f, 0, order, transA, transB);
+  for (int c = 0; c < 4; ++c) {
+    GemmKey key = make_key(g, c & 1 ? 1.0f : 0.0f, 0, order, transA, transB);
+    if (c & 2) {
+      if (!key.rows_ok || K > kRowsMaxK) continue;
+      key.rows_ok = false;
+    }
     for (int gemv = 0; gemv <= (g.N == 1 ? 1 : 0); ++gemv) {
       key.gemv_ok = gemv == 1;
       hmlSgemmVariant v;
@@ -714,6 +744,27 @@ hmlStatus hmlSgemmSelect(hmlOrder order, hmlOp transA, hmlOp transB,
   GemmKey key = make_key(g, beta, 0, order, transA, transB);
   int src = 0;
   select_sgemm(key, variant, &src);
+  if (source) *source = src;
+  return HML_STATUS_SUCCESS;
+}
+
+hmlStatus hmlSgemmResolve(hmlOrder order, hmlOp transA, hmlOp transB, int64_t M, int64_t N,
+                          int64_t K, int64_t lda, int64_t ldb, int64_t ldc, float beta,
+                          uint32_t flags, hmlSgemmVariant *variant, int32_t *source) {
+  if (!variant) return fail(HML_STATUS_INVALID_VALUE, "variant is NULL");
+  if (M <= 0 || N <= 0 || K <= 0)
+    return fail(HML_STATUS_INVALID_VALUE, "dimensions must be positive");
+  // no pointer is read: the check only needs them to be there
+  const float *const some = (const float *)variant;
+  const hmlStatus s = check_gemm_args(order, transA, transB, M, N, K, some, lda, some, ldb, some, ldc);
+  if (s != HML_STATUS_SUCCESS) return s;
+  const GemmCanon g = canonicalize(order, transA, transB, M, N, K, nullptr, lda, nullptr, ldb,
+                                   nullptr, ldc);
+  const GemmKey key = make_key(g, beta, flags, order, transA, transB);
+  int src = 0;
+  bool exact;
+  select_sgemm(key, variant, &src, &exact);
+  if (!exact) resolve_choice(g, key, variant);
   if (source) *source = src;
   return HML_STATUS_SUCCESS;
 }

@@ -112,6 +112,7 @@ struct DotParams {
 };
 // kw = waves per workgroup (each with its own K chunk)
 bool skinny_dot_runnable(int rt, int ct, int kw);
+bool skinny_dot3_runnable(int rt, int kw);  // 3 column tiles: N-contiguous B, N >= 3
 // Load kind of the skinny DOT kernels' A (row-major, leading dimension ld
 // floats).  Rows that do not start on 128-byte lines share a line between
 // the end of one 64-k stage and the start of the next; read
@@ -149,12 +150,14 @@ hipError_t launch_skinny_dot(int rt, int ct, bool bvec, int kw, const DotParams 
 int device_cus();
 
 // k_skinny_rows: unsplit products of few k and many rows, rows streamed by
-// persistent waves.  `better` is the rule that sends a problem there.
+// persistent waves.  `fit`: a leading dimension it can address; `better` is
+// the rule that sends a problem there.
 constexpr int kRowsWaves = 8;  // most waves per workgroup
 constexpr int kRowsMaxK = 128, kRowsMaxN = 128;
 constexpr int64_t kRowsMaxLda = 1 << 23;  // 16 rows within 31-bit offsets
 constexpr int64_t kRowsMinM = 1 << 16;
-bool skinny_rows_better(int64_t M, int64_t N, int64_t K, int64_t lda);
+bool skinny_rows_fit(int64_t K, int64_t lda);
+bool skinny_rows_better(int64_t M, int64_t N, int64_t K);
 hipError_t launch_skinny_rows(const DotParams &p, hipStream_t st);
 
 // out(m,n) = alpha * sum_r P[r*total + m*ninner + n] + beta * out(m,n)

@@ -1443,7 +1443,7 @@ DotFn dot_fn(bool bv, bool cached) {
                 : (bv ? run_dot<RT, CT, true, kBufNT> : run_dot<RT, CT, false, kBufNT>);
 }
 
-// Tiles of 3 column tiles, N-contiguous B: run by dot_geometry's choice only.
+// Tiles of 3 column tiles, N-contiguous B.
 DotFn find_dot3(int rt, bool cached) {
   return rt == 1   ? (cached ? run_dot<1, 3, false, 0> : run_dot<1, 3, false, kBufNT>)
          : rt == 2 ? (cached ? run_dot<2, 3, false, 0> : run_dot<2, 3, false, kBufNT>)
@@ -1592,6 +1592,8 @@ int skinny_dot_resident_waves(int rt, int ct) {
   return cache[rt][ct];
 }
 
+bool skinny_dot3_runnable(int rt, int kw) { return (rt == 1 || rt == 2) && kw >= 1 && kw <= 4; }
+
 bool skinny_dot_runnable(int rt, int ct, int kw) {
   if (!find_dot(rt, ct, true)) return false;
   return kw >= 1 && kw <= dot_max_waves(rt, ct) && skinny_dot_lds_bytes(rt, ct, kw) <= kDotMaxLds;
@@ -1601,7 +1603,7 @@ hipError_t launch_skinny_dot(int rt, int ct, bool bvec, int kw, const DotParams 
                              hipStream_t st) {
   if (p.kgroups < 1 || p.kchunk % kDotStageK != 0) return hipErrorInvalidValue;
   if (ct == 3) {
-    if (bvec || rt > 2 || p.N < 3 || kw < 1 || kw > 4) return hipErrorInvalidValue;
+    if (bvec || p.N < 3 || !skinny_dot3_runnable(rt, kw)) return hipErrorInvalidValue;
     return find_dot3(rt, a_loads_cached(p.A, p.sAm, ((p.N + 15) / 16 + 2) / 3))(kw, p, st);
   }
   if (!skinny_dot_runnable(rt, ct, kw)) return hipErrorInvalidValue;
@@ -1647,14 +1649,21 @@ const void *rows_fn(int ct) {
 // stages k_skinny_dot pipelines as well (16 x 128: 12.8 / 15.3 at 10^5 rows,
 // 100 / 105 at 10^6; 32 x 128 15.7 / 16.7 at 70000, 131 / 128 at 10^6; 16 x
 // 64: 10.2 / 11.1 at 10^5, 23.3 / 21.1 at 3 10^5).
-bool skinny_rows_better(int64_t M, int64_t N, int64_t K, int64_t lda) {
+bool skinny_rows_better(int64_t M, int64_t N, int64_t K) {
   if (K < 1 || K > kRowsMaxK || N < 1 || N > kRowsMaxN || M < kRowsMinM) return false;
-  if (lda > kRowsMaxLda || (lda != K && K % 4 != 0)) return false;
   return !(K == 128 && N <= 32) && !(K == 64 && N <= 16 && M < 4 * kRowsMinM);
 }
 
+// Rows at any distance when a row is whole 16-byte chunks, else one
+// contiguous block.
+bool skinny_rows_fit(int64_t K, int64_t lda) {
+  return lda <= kRowsMaxLda && (lda == K || K % 4 == 0);
+}
+
 hipError_t launch_skinny_rows(const DotParams &p, hipStream_t st) {
-  if (!skinny_rows_better(p.M, p.N, p.K, p.sAm)) return hipErrorInvalidValue;
+  if (p.M < 1 || p.N < 1 || p.N > kRowsMaxN || p.K < 1 || p.K > kRowsMaxK ||
+      !skinny_rows_fit(p.K, p.sAm))
+    return hipErrorInvalidValue;
   // passes of at most 4 column tiles, the tiles spread evenly
   const int nct = (int)((p.N + 15) / 16), passes = (nct + 3) / 4, ct = (nct + passes - 1) / passes;
   const void *fn = p.K % 4 == 0 ? rows_fn<true>(ct) : rows_fn<false>(ct);

@@ -30,6 +30,8 @@ struct GemmKey {
   int transA, transB, order;  // caller's layout (features of the learned selector)
   bool gemv_ok;  // N == 1 and x / y are unit-stride, GEMV kernels apply
   int64_t cM, cN;  // caller's M and N (before orientation)
+  bool b_rows = false;   // B N-contiguous: the tiles of 3 column tiles apply
+  bool rows_ok = false;  // A's leading dimension suits the row-streaming kernel
 };
 
 struct GemvKey {
@@ -98,8 +100,9 @@ bool selector_variant(const GemmKey &k, int cls, hmlSgemmVariant *v);
 
 // Selection entry used by the dispatch: a table rule of the problem's own
 // shape bucket (the exhaustive autotuner's answer), else the learned
-// selector, else the nearest table rule, else the heuristic.
-void select_sgemm(const GemmKey &k, hmlSgemmVariant *v, int *source);
+// selector, else the nearest table rule, else the heuristic.  exact (if
+// given): the answer is a rule of the problem's own bucket.
+void select_sgemm(const GemmKey &k, hmlSgemmVariant *v, int *source, bool *exact = nullptr);
 void select_sgemv(const GemvKey &k, hmlSgemvVariant *v, int *source);
 
 }  // namespace hml

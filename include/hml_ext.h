@@ -72,8 +72,12 @@ typedef enum {
                                   workgroup through LDS                   */
   HML_SGEMM_FAMILY_GEMVN  = 8, /* N in {2, 4, 8}, K-contiguous A: the GEMV
                                   DOT kernels with N accumulators per row */
-  HML_SGEMM_FAMILY_F16X3  = 9  /* split-precision fp16 MFMA, 2-term split
+  HML_SGEMM_FAMILY_F16X3  = 9, /* split-precision fp16 MFMA, 2-term split
                                   with power-of-two row / column scales   */
+  HML_SGEMM_FAMILY_ROWS   = 10 /* MFMA f32, K-contiguous A, K and N <= 128:
+                                  rows streamed by persistent waves, the
+                                  sums of an unsplit DOT variant
+                                  (10, 1, 1, 1, 4; it has no parameters)  */
 } hmlSgemmFamily;
 
 /* Skinny variants (DOT, AXPY): a wave computes rt row tiles (16 rows DOT,
@@ -168,17 +172,25 @@ size_t hmlSgemmWorkspaceSize(hmlOrder order, hmlOp transA, hmlOp transB,
                              int64_t M, int64_t N, int64_t K,
                              const hmlSgemmVariant *variant);
 
-/* The variant hmlSgemmEx would run for these arguments, and which selector
- * produced it (0 built-in heuristic, 1 config table, 2 learned MLP; the
- * order is given with hmlSelectorInstall).  Where a DOT-form variant is selected
- * for many rows of few k (K <= 128, M >= 65536), hmlSgemmEx runs a
- * row-streaming kernel in its place, with the results of an unsplit DOT
- * variant, and for more than 32 columns of row-major B it may run a DOT
- * variant in another tile and K split (never more partial sums nor longer
- * chains); hmlSgemmExVariant runs the variant it is given. */
+/* The variant the selectors choose for these arguments, and which one did
+ * (0 built-in heuristic, 1 config table, 2 learned MLP; the order is given
+ * with hmlSelectorInstall).  A rule of the problem's own shape bucket runs as
+ * it is.  In place of another choice hmlSgemmEx may run, where measured rules
+ * find it faster, the row-streaming kernel (for an unsplit tile, K <= 128 and
+ * M >= 65536), or, for more than 32 columns of row-major B, a DOT variant in
+ * another tile and K split (never more partial sums nor longer chains):
+ * hmlSgemmResolve names it.  hmlSgemmExVariant runs the variant it is given. */
 hmlStatus hmlSgemmSelect(hmlOrder order, hmlOp transA, hmlOp transB,
                          int64_t M, int64_t N, int64_t K, float beta,
                          hmlSgemmVariant *variant, int32_t *source);
+
+/* The variant hmlSgemmEx runs for these arguments (but for strides beyond the
+ * skinny kernels' offsets, which take the dense FP32 kernel), and which
+ * selector it comes from. */
+hmlStatus hmlSgemmResolve(hmlOrder order, hmlOp transA, hmlOp transB,
+                          int64_t M, int64_t N, int64_t K, int64_t lda,
+                          int64_t ldb, int64_t ldc, float beta, uint32_t flags,
+                          hmlSgemmVariant *variant, int32_t *source);
 
 /* Dense SGEMM on the matrix cores, no reference counterpart (the reference
  * has only its skinny kernels).  precision: 0 = plain FP32 MFMA

@@ -651,3 +651,62 @@ def test_host_entry_runs_the_device_entry(hml, M, N, K):
     C = C0.copy()
     hml.sgemm(C, A, B, 1.5, 0.5)
     np.testing.assert_array_equal(C, run_gemm(hml, A, B, C0, 1.5, 0.5, flags=hml.FLAG_READ_C_ALWAYS))
+
+
+def test_own_bucket_rule_gives_its_bits(hml):
+    """A loaded rule of the problem's own bucket runs, and not what the
+    dispatch would put in the place of another choice."""
+    rng = np.random.default_rng(4)
+    for M, N, K, variant in ((65536 + 9, 24, 100, (1, 2, 2, 2, 4)), (65536, 8, 48, (8, 16, 1, 1, 2)),
+                             (2000, 72, 5000, (1, 2, 4, 2, 4)), (65537, 40, 48, (10, 1, 1, 1, 4)),
+                             (2000, 72, 5000, (1, 1, 3, 16, 4))):
+        A, B, C0 = uniform(rng, (M, K)), uniform(rng, (K, N)), uniform(rng, (M, N))
+        shape, rule = hml.GemmShape(M, N, K, 0, 0, 0, 1), hml.SgemmVariant(*variant)
+        hml.check(hml.lib.hmlSgemmConfigAddRule(ctypes.byref(shape), ctypes.byref(rule)))
+        try:
+            got = run_gemm(hml, A, B, C0, 1.0, 0.0)
+        finally:
+            hml.config_clear()
+        np.testing.assert_array_equal(got, run_gemm(hml, A, B, C0, 1.0, 0.0, variant=variant))
+
+
+@pytest.mark.parametrize("N", [3, 4, 17, 40, 47, 48, 49, 96, 97])
+def test_three_column_tiles(hml, N):
+    """The tiles of 3 column tiles by name: column remainders, whole and
+    partial stages, several waves and K groups."""
+    rng = np.random.default_rng(N)
+    for M, K in ((100, 64), (129, 200), (1000, 513)):
+        A, B, C0 = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
+        R = exact_product(A, B, 2.0, -1.0, C0)
+        for v in ((1, 1, 3, 1, 1), (1, 2, 3, 1, 4), (1, 1, 3, 4, 4), (1, 2, 3, 8, 2)):
+            np.testing.assert_array_equal(run_gemm(hml, A, B, C0, 2.0, -1.0, variant=v), R, err_msg=str(v))
+    with pytest.raises(hml.HmlError):  # K-contiguous B has no such tile
+        run_gemm(hml, A, B, C0, 1.0, 0.0, tb=True, variant=(1, 2, 3, 1, 4))
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 33, 5000])
+def test_row_streaming_by_name(hml, M):
+    """The row-streaming kernel by name, also for few rows."""
+    rng = np.random.default_rng(M)
+    for N, K in ((1, 1), (1, 128), (7, 15), (16, 64), (100, 127), (128, 128)):
+        if N > M:
+            continue
+        A, B, C0 = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
+        np.testing.assert_array_equal(run_gemm(hml, A, B, C0, 2.0, -1.0, variant=(10, 1, 1, 1, 4)),
+                                      exact_product(A, B, 2.0, -1.0, C0))
+    for N, K in ((16, 129), (129, 16)):
+        A, B, C0 = int_matrix(rng, (200, K)), int_matrix(rng, (K, N)), int_matrix(rng, (200, N))
+        with pytest.raises(hml.HmlError):
+            run_gemm(hml, A, B, C0, 1.0, 0.0, variant=(10, 1, 1, 1, 4))
+
+
+@pytest.mark.parametrize("M,N,K,family", [(65537, 17, 100, 10), (65545, 113, 127, 10), (65536, 16, 128, 1),
+                                          (3000, 33, 4000, 1), (2500, 72, 2100, 1)])
+def test_replacement_runs(hml, M, N, K, family):
+    """sgemm_resolve names what runs: its variant by name gives the same bits."""
+    rng = np.random.default_rng(N)
+    A, B, C0 = uniform(rng, (M, K)), uniform(rng, (K, N)), uniform(rng, (M, N))
+    v = hml.sgemm_resolve(M, N, K)[0].astuple()
+    assert v[0] == family
+    np.testing.assert_array_equal(run_gemm(hml, A, B, C0, 1.0, 0.0),
+                                  run_gemm(hml, A, B, C0, 1.0, 0.0, variant=v))

@@ -179,3 +179,68 @@ def test_gemvn_runnable_and_selector_class():
     assert m[86] == 1
     v = hml.selector_variant(8192, 4, 8192, 86)
     assert hml.selector_class_of(8192, 4, 8192, v) == 86
+
+
+@pytest.fixture
+def rule():
+    """rule(shape, variant): a table with that one rule, gone at the end."""
+    def add(M, N, K, v):
+        s, v = hml.GemmShape(M, N, K, 0, 0, 0, 1), hml.SgemmVariant(*v)
+        hml.config_clear()
+        hml.check(hml.lib.hmlSgemmConfigAddRule(ctypes.byref(s), ctypes.byref(v)))
+    yield add
+    hml.config_clear()
+
+
+ROWS = (10, 1, 1, 1, 4)
+
+
+def resolved(M, N, K, **kw):
+    return hml.sgemm_resolve(M, N, K, **kw)[0].astuple()
+
+
+def test_own_bucket_rule_runs_as_it_is(rule):
+    """A table rule of the problem's own bucket is a measurement: neither the
+    row-streaming rule nor the tile model replaces it; a neighbour's rule and
+    the heuristic's choice they do."""
+    tall, wide = (1 << 20, 32, 48), (2000, 72, 5000)
+    split = (1, 2, 4, 8, 4)
+    assert resolved(*tall) == ROWS
+    rule(*tall, (1, 1, 2, 1, 4))
+    assert hml.sgemm_select(*tall)[1] == 1 and resolved(*tall) == (1, 1, 2, 1, 4)
+    rule(tall[0] // 2, tall[1], tall[2], (1, 1, 2, 1, 4))
+    assert hml.sgemm_select(*tall)[1] == 1 and resolved(*tall) == ROWS
+    rule(*wide, split)
+    assert resolved(*wide) == split
+    rule(wide[0] * 2, wide[1], wide[2], split)
+    assert hml.sgemm_select(*wide)[0].astuple() == split and resolved(*wide) != split
+    # and the rule of a table can name what the dispatch would run
+    rule(*tall, ROWS)
+    assert hml.sgemm_select(*tall)[0].astuple() == ROWS == resolved(*tall)
+    rule(*wide, (1, 2, 3, 8, 4))
+    assert resolved(*wide) == (1, 2, 3, 8, 4)
+
+
+def test_row_streaming_by_leading_dimension(rule):
+    """Rows that the row-streaming kernel cannot address go to the next
+    selector, in the workspace that the size query names."""
+    M, N, K = 1 << 17, 24, 99
+    rule(M, N, K, ROWS)
+    assert resolved(M, N, K) == ROWS and resolved(M, N, K, lda=K + 1)[0] == 1
+    assert resolved(M, N, 100, lda=107) == ROWS
+    v = hml.SgemmVariant(*resolved(M, N, K, lda=K + 1))
+    own = hml.lib.hmlSgemmWorkspaceSize(0, 0, 0, M, N, K, ctypes.byref(v))
+    assert hml.lib.hmlSgemmWorkspaceSize(0, 0, 0, M, N, K, None) >= own
+
+
+def test_replacements_are_candidates():
+    """What the dispatch may run in place of a choice can be measured: the
+    autotuner's candidates hold it."""
+    def cands(M, N, K, tb=0):
+        a = (hml.SgemmVariant * 1024)()
+        n = hml.lib.hmlSgemmCandidates(ctypes.byref(hml.GemmShape(M, N, K, 0, 0, tb, 1)), a, 1024)
+        return {a[i].astuple() for i in range(n)}
+    assert ROWS in cands(1 << 20, 32, 48) and ROWS not in cands(1 << 20, 32, 129)
+    c = cands(2000, 72, 5000)
+    assert {(1, 1, 3, 1, 4), (1, 2, 3, 1, 4), (1, 1, 3, 8, 4), (1, 2, 3, 32, 4)} <= c
+    assert not any(v[:1] == (1,) and v[2] == 3 for v in cands(2000, 72, 5000, tb=1))  # K-contiguous B
