@@ -10,24 +10,32 @@
 //
 //  1. Screening on the 16-bit matrix cores.  |x - c|^2 = |x|^2 - 2 a_k with
 //     a_k = x.c_k - |c_k|^2 / 2, and x.c_k for 32 rows against 32 centroids
-//     is a product of bf16 terms x = xh + xl, c = ch + cl (round to
-//     nearest): three v_mfma_f32_32x32x16_bf16 per 16 dims (cl.xh, ch.xl,
-//     ch.xh), the accumulator starting at -|c|^2 / 2.  FP32 MFMAs would take
-//     5 times as long for the same dims.
+//     is a product of fp16 terms x = xh + xl, c = ch + cl (round to nearest,
+//     22 bits together): three v_mfma_f32_32x32x16_f16 per 16 dims (cl.xh,
+//     ch.xl, ch.xh), the accumulator starting at -|c|^2 / 2.  Rows and
+//     centroids are scaled by one power of two that brings the centroids (a
+//     sample of 8) to about 1; what then leaves the range of fp16 is compared
+//     exactly.  FP32 MFMAs would take 5 times as long for the same dims; their
+//     rms error against 64 bits is 0.97e-7 (32 dims, clustered rows), that of
+//     the terms 1.17e-7 (64 dims, |x| >> |c|: 1.5e-7 and 0.8e-7).  Two bf16
+//     terms, 16 bits together, are off by up to 2^-15 |x||c|.
 //  2. A bound on how far the reference's float distance can be from
-//     |x|^2 - 2 a~_k (the screened value), in units of 2^-24 (|x| + |c_k|)^2:
-//       2D + 4   the reference's own roundings;
-//       D        the norm;
-//       96 KS    the accumulation, KS = D / 16 rounded up: 48 KS products
-//                added with an error of at most 2^-23 of the running sum's
-//                bound |x||c_k| + |c_k|^2 / 2 each, doubled in 2 a_k;
-//       96       the split: xl, cl round at 2^-18 of x, c, and xl.cl (2^-18)
-//                is left out: 3 2^-18 |x||c_k|, doubled, |x||c_k| being at
-//                most (|x| + |c_k|)^2 / 4;
-//       64       the index kept in the low 4 bits of a~_k.
-//     Their sum is below 4D + 96 KS + 256.  With M that factor times (|x| +
-//     max |c|)^2, only centroids with a~_k >= max a~ - M can be the exact
-//     argmin (each side's distance may be off by M, 2 a~ by 2 M).
+//     |x|^2 - 2 a~_k (the screened value).  With u = 2^-24, X = |x|, C >=
+//     |c_k|, q = X C + C^2 / 2 (which bounds the partial sums of a_k), KS =
+//     D / 16 rounded up, all scaled, a~_k is off by at most u times
+//       12 X C + 4 (X + C)  the terms: a residual is at most 2^-11 of the
+//                           value and rounds at 2^-22 of it or, below fp16's
+//                           normal range, at 2^-25; xl.cl (2^-22) is left out
+//       96 KS q             the accumulation of 48 KS products, 2 u of the
+//                           partial sums' bound each
+//       (4 KS + 1) C^2      the norm: 8 KS + 2 roundings of C^2 / 2
+//       30 q                the index kept in the low 4 bits of a~_k
+//     and the reference's distance by (D + 3) u of itself (D additions, the
+//     square twice the difference's rounding).  If k is the reference's
+//     argmin and j has the largest a~, then a~_k >= a~_j - M with
+//       M = (D + 4) u d + u (((192 KS + 84) X + (104 KS + 32) C) C + 8 (X + C))
+//     d bounding the distance of j.  Only centroids with a~_k >= max a~ - M can
+//     be the exact argmin.
 //  3. Each lane keeps the two largest a~ of its even and of its odd centroid
 //     tiles.  If a row's second largest value lies below the limit its
 //     argmin is known (the usual case: no distance is computed).  Otherwise
@@ -48,7 +56,7 @@
 // rarer and cost registers: up to 10% slower.  Rows equidistant from many
 // centroids cost up to two screenings and a distance per candidate.
 //
-// Centroids live in LDS as bf16 terms in MFMA operand order (a fragment is
+// Centroids live in LDS as fp16 terms in MFMA operand order (a fragment is
 // one conflict-free 16-byte read per lane) beside their norms, staged once
 // per workgroup when they fit, else chunk by chunk per row step with the
 // workgroup's waves in lockstep.  Every wave streams its rows 32 at a time
@@ -128,40 +136,47 @@ __device__ __forceinline__ float exact_dist(const float *__restrict__ xr,
   return dist;
 }
 
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
-// hi / lo bf16 terms of 8 floats (round to nearest; the residual is exact)
-__device__ __forceinline__ void split8(const float (&v)[8], b8 &hi, b8 &lo) {
+// hi / lo fp16 terms of 8 floats (round to nearest; the residual is exact)
+__device__ __forceinline__ void split8(const float (&v)[8], h8 &hi, h8 &lo) {
 #pragma unroll
   for (int j = 0; j < 8; j += 2) {
-    const b2 h = __builtin_convertvector(f2{v[j], v[j + 1]}, b2);
+    const h2 h = __builtin_convertvector(f2{v[j], v[j + 1]}, h2);
     hi[j] = h[0];
     hi[j + 1] = h[1];
-    const b2 l = __builtin_convertvector(f2{v[j] - (float)h[0], v[j + 1] - (float)h[1]}, b2);
+    const h2 l = __builtin_convertvector(f2{v[j] - (float)h[0], v[j + 1] - (float)h[1]}, h2);
     lo[j] = l[0];
     lo[j + 1] = l[1];
   }
 }
 
-// Squared norms at or above kKmNormMax (and NaN) take a centroid out of the
-// screen; rows that could still choose it (|x|^2 or the best screened
-// distance not below kKmRowMax) are refined over every centroid.
-constexpr float kKmNormMax = 1e37f;
-constexpr float kKmRowMax = 1e36f;
+// Scaled squared norms at or above kKmNormMax (and NaN) take a centroid out
+// of the screen; rows that could still choose it (|x|^2 or the best screened
+// distance not below kKmRowMax), or whose distances could overflow
+// (kKmDistMax, unscaled), are refined over every centroid.
+constexpr float kKmNormMax = 0x1p30f;
+constexpr float kKmRowMax = 0x1p26f;
+constexpr float kKmDistMax = 0x1p118f;
 // screen value of an excluded or padding centroid
 constexpr float kKmExcluded = -1e38f;
+constexpr float kKmSampleMax = 0x1p60f;
+constexpr int kKmSampleBytes = kKmWaves * 256;
 
 // KS = k-steps of 16 dims, MULTI = the centroids take several LDS chunks,
-// VEC = dims a multiple of 4.
+// VEC = dims a multiple of 4.  Several chunks fill a CU's LDS with one
+// workgroup, two waves per SIMD: they may use 256 registers (capped at 128, 64
+// dims spilled 19).
 template <int KS, bool MULTI, bool VEC, bool FUSED>
-__global__ __launch_bounds__(64 * kKmWaves, 4) void k_kmeans_screen(KmParams p) {
+__global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(KmParams p) {
   constexpr int NQ = KS * 2;  // 1 KB DMA loads per row tile (at most)
   extern __shared__ f4 km_lds4[];
   char *lds = reinterpret_cast<char *>(km_lds4);
-  b8 *cf = reinterpret_cast<b8 *>(lds);                                 // centroid fragments
-  float *nrm = reinterpret_cast<float *>(lds + (size_t)p.KC * KS * 64); // -|c|^2 / 2
+  float *smp = reinterpret_cast<float *>(lds);
+  h8 *cf = reinterpret_cast<h8 *>(lds + kKmSampleBytes);  // centroid fragments
+  float *nrm = reinterpret_cast<float *>(lds + kKmSampleBytes + (size_t)p.KC * KS * 64);  // -|c|^2 / 2
   // max as a median with infinity (in a register the compiler does not see
   // through), without the canonicalising moves fmaxf needs for unknown
   // inputs; a result that a NaN could have entered is never used
@@ -174,28 +189,59 @@ __global__ __launch_bounds__(64 * kKmWaves, 4) void k_kmeans_screen(KmParams p) 
   float *xs = nrm + p.KC + w * p.xfloats;  // this wave's row tile
   const int h = lane >> 5, r = lane & 31;
   const int nchunks = MULTI ? (K + p.KC - 1) / p.KC : 1;
-  // margin factor, see the error terms at the top of the file
-  const float tau = (float)(4 * D + 96 * KS + 256) * 0x1p-24f * (1.0f + 0x1p-8f);
+  // The scale sc is a power of two from the largest magnitude in a sample of
+  // centroids, one per wave, exchanged through LDS (smp, a row of 64 dims
+  // each): the loads start here, the exchange shares the barrier that
+  // staging the centroids begins with.
+  const float mine = lane < D ? p.ctrds[(int64_t)((uint64_t)w * (uint32_t)K / kKmWaves) * D + lane] : 0.f;
+  float sc = 1.f;
+  auto set_scale = [&]() {
+    float big = 0.f;
+#pragma unroll
+    for (int i = 0; i < kKmWaves; ++i) {
+      const float v = __builtin_fabsf(smp[64 * i + lane]);
+      big = v < kKmSampleMax ? __builtin_fmaxf(big, v) : big;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) big = __builtin_fmaxf(big, __shfl_xor(big, off));
+    const int ex = min(max((int)(__float_as_uint(big) >> 23) - 127, -60), 60);
+    sc = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane(127 - ex) << 23);
+  };
+  // margin factors, see the error terms at the top of the file (2^-7 for the
+  // second order and the margin's own roundings)
+  constexpr float kU = 0x1p-24f * (1.0f + 0x1p-7f);
+  constexpr float kMx = (192 * KS + 84) * kU, kMc = (104 * KS + 32) * kU, kMa = 8 * kU;
+  const float md = (float)(D + 4) * kU;
 
   // Stages centroids c0 .. c0 + KC - 1 (zeros past K) and returns the
   // largest norm among those in the screen.  Lanes l and l ^ 32 hold the two
   // halves of a centroid's dims, in the fragment layout itself: (tile of 32,
   // k-step, hi / lo, lane, 8 dims).
   auto stage = [&](int c0) -> float {
-    __syncthreads();  // every wave is done with the previous chunk
-    for (int i = threadIdx.x; i < p.KC * 2; i += 64 * kKmWaves) {
-      const int t = i >> 6, k = 32 * t + r;
+    float v[KS][8];
+    auto load = [&](int i) {  // the 8 KS dims of thread item i
+      const int k = 32 * (i >> 6) + r;
       const float *c = p.ctrds + (int64_t)(c0 + k) * D + 8 * h;
-      float v[KS][8], s2 = 0.f;
 #pragma unroll
       for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          v[s][j] = c0 + k < K && 16 * s + 8 * h + j < D ? c[16 * s + j] : 0.f;
+          v[s][j] = i < p.KC * 2 && c0 + k < K && 16 * s + 8 * h + j < D ? c[16 * s + j] : 0.f;
+    };
+    if (!MULTI) load(threadIdx.x);
+    __syncthreads();  // every wave is done with the previous chunk, or has its sample in LDS
+    if (!MULTI) set_scale();
+    for (int i = threadIdx.x; i < p.KC * 2; i += 64 * kKmWaves) {
+      const int t = i >> 6, k = 32 * t + r;
+      if (MULTI || i != (int)threadIdx.x) load(i);
+      float s2 = 0.f;
 #pragma unroll
       for (int s = 0; s < KS; ++s)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s2 = __builtin_fmaf(v[s][j], v[s][j], s2);
+        for (int j = 0; j < 8; ++j) {
+          v[s][j] *= sc;
+          s2 = __builtin_fmaf(v[s][j], v[s][j], s2);
+        }
       s2 += __shfl_xor(s2, 32);
       const bool in = c0 + k < K && s2 < kKmNormMax;
       if (h == 0) nrm[k] = in ? -0.5f * s2 : kKmExcluded;
@@ -205,7 +251,7 @@ __global__ __launch_bounds__(64 * kKmWaves, 4) void k_kmeans_screen(KmParams p) 
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[s][j] = 0.f;
         }
-        b8 hi, lo;
+        h8 hi, lo;
         split8(v[s], hi, lo);
         cf[(t * KS + s) * 128 + lane] = hi;
         cf[(t * KS + s) * 128 + 64 + lane] = lo;
@@ -283,14 +329,20 @@ __global__ __launch_bounds__(64 * kKmWaves, 4) void k_kmeans_screen(KmParams p) 
 
   load_rows(tile);
   float cmax = 0.f;
-  if (!MULTI) cmax = stage(0);
+  smp[64 * w + lane] = mine;
+  if (!MULTI) {
+    cmax = stage(0);
+  } else {
+    __syncthreads();
+    set_scale();
+  }
 
   for (int64_t st = 0; st < p.steps; ++st, tile += wstep) {
     const int64_t row0 = tile * 32;
     const bool live = row0 < p.nrows;  // wave-uniform
     if (!MULTI && !live) break;        // later steps only go further
 
-    b8 xh[KS], xl[KS];
+    h8 xh[KS], xl[KS];
     float xx = 0.f;
     if (!MULTI || live) {
       __builtin_amdgcn_s_waitcnt(kWaitAll);  // the tile is in LDS
@@ -323,7 +375,10 @@ __global__ __launch_bounds__(64 * kKmWaves, 4) void k_kmeans_screen(KmParams p) 
           for (int j = 0; j < 8; ++j) v[s][j] = 16 * s + 8 * h + j < D ? v[s][j] : 0.f;
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xx = __builtin_fmaf(v[s][j], v[s][j], xx);
+        for (int j = 0; j < 8; ++j) {
+          v[s][j] *= sc;
+          xx = __builtin_fmaf(v[s][j], v[s][j], xx);
+        }
         split8(v[s], xh[s], xl[s]);
       }
       xx += __shfl_xor(xx, 32);
@@ -339,13 +394,13 @@ __global__ __launch_bounds__(64 * kKmWaves, 4) void k_kmeans_screen(KmParams p) 
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[4 * i + e] = q[e];
       }
-      const b8 *f = cf + tl * KS * 128 + lane;
+      const h8 *f = cf + tl * KS * 128 + lane;
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        const b8 ch = f[s * 128], cl = f[s * 128 + 64];
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cl, xh[s], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xl[s], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, xh[s], acc, 0, 0, 0);
+        const h8 ch = f[s * 128], cl = f[s * 128 + 64];
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(cl, xh[s], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch, xl[s], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch, xh[s], acc, 0, 0, 0);
       }
       return acc;
     };
@@ -404,11 +459,17 @@ __global__ __launch_bounds__(64 * kKmWaves, 4) void k_kmeans_screen(KmParams p) 
       const float s1 = vmax(a1, o1);
       const float unnamed = vmax(rest, orest);  // every value that no tracker names is below
       const float s2 = vmax(vmax(unnamed, o1 < a1 ? o1 : a1), vmax(a2, o2));
-      const float xc = __builtin_sqrtf(xx) + cmax;
-      const float M = __builtin_fmaf(tau, xc * xc, 0x1p-100f);
+      const float X = __builtin_amdgcn_sqrtf(xx);
+      const float d = __builtin_fmaxf(xx - 2.f * s1, 0.f) + 0x1p-10f * xx + 0x1p-20f * (X + cmax);
+      // an absolute term for underflow, in the screen and, D 2^-149 unscaled,
+      // in the reference
+      const float m0 = __builtin_fmaf((float)D * 0x1p-148f * sc, sc, 0x1p-40f);
+      const float M = __builtin_fmaf(kMx * X + kMc * cmax, cmax,
+                                     __builtin_fmaf(kMa, X + cmax, __builtin_fmaf(md, d, m0)));
       // small enough that no distance overflows and excluded centroids are
       // farther (false for NaN)
-      const bool range = xx < kKmRowMax && xx - 2.f * s1 < kKmRowMax;
+      const float rmax = __builtin_fminf(kKmRowMax, kKmDistMax * sc * sc);
+      const bool range = xx < rmax && xx - 2.f * s1 < rmax;
       ans = (uint32_t)(o1 > a1 ? ok : k);
       need = row0 + r < p.nrows && !(range && s1 - s2 > M);
       full = need && !(range && s1 - unnamed > M);
@@ -645,11 +706,11 @@ KmeansPlan plan_kmeans(int64_t nrows, int D, int K, int mode) {
   }
   pl.ni = (D + 15) / 16;
   const int64_t kpad = ((int64_t)K + 31) / 32 * 32;
-  // LDS: per centroid 64 ni bytes of bf16 terms and its norm, each wave's
-  // row tile in whole 1 KB loads, 256 bytes that reads past the last tile's
+  // LDS: the sample of centroids, per centroid 64 ni bytes of fp16 terms and
+  // its norm, each wave's row tile in whole 1 KB loads, 256 bytes that reads past the last tile's
   // last row may touch, and 256 for the workgroup vote
   pl.xfloats = (D + 7) / 8 * 256;
-  const int64_t rows_b = (int64_t)kKmWaves * pl.xfloats * 4 + 256;
+  const int64_t rows_b = (int64_t)kKmWaves * pl.xfloats * 4 + 256 + kKmSampleBytes;
   const int64_t room = (int64_t)kKmLdsBytes - 256 - rows_b;
   pl.KC = (int)std::min<int64_t>(kpad, room / (64 * pl.ni + 4) / 32 * 32);
   pl.lds = (size_t)(pl.KC * (64 * pl.ni + 4) + rows_b);
