@@ -13,16 +13,19 @@
 //     is a product of fp16 terms x = xh + xl, c = ch + cl (round to nearest,
 //     22 bits together): three v_mfma_f32_32x32x16_f16 per 16 dims (cl.xh,
 //     ch.xl, ch.xh), the accumulator starting at -|c|^2 / 2.  Rows and
-//     centroids are scaled by one power of two that brings the centroids (a
-//     sample of 8) to about 1; what then leaves the range of fp16 is compared
-//     exactly.  FP32 MFMAs would take 5 times as long for the same dims; their
-//     rms error against 64 bits is 0.97e-7 (32 dims, clustered rows), that of
-//     the terms 1.17e-7 (64 dims, |x| >> |c|: 1.5e-7 and 0.8e-7).  Two bf16
-//     terms, 16 bits together, are off by up to 2^-15 |x||c|.
+//     centroids are taken relative to a point amid the centroids (when the
+//     origin is not amid them) and scaled by one power of two that brings them
+//     to about 1, both from a sample of 8; what then leaves the range of fp16
+//     is compared exactly.  FP32 MFMAs would take 5 times as long for the same
+//     dims; their rms error against 64 bits is 0.97e-7 (32 dims, clustered
+//     rows), that of the terms 1.17e-7 (64 dims, |x| >> |c|: 1.5e-7 and
+//     0.8e-7).  Two bf16 terms, 16 bits together, are off by up to
+//     2^-15 |x||c|.
 //  2. A bound on how far the reference's float distance can be from
 //     |x|^2 - 2 a~_k (the screened value).  With u = 2^-24, X = |x|, C >=
 //     |c_k|, q = X C + C^2 / 2 (which bounds the partial sums of a_k), KS =
-//     D / 16 rounded up, all scaled, a~_k is off by at most u times
+//     D / 16 rounded up, all moved and scaled, a~_k is off by at most u times
+//       2 q                 moving the values, a rounding each
 //       12 X C + 4 (X + C)  the terms: a residual is at most 2^-11 of the
 //                           value and rounds at 2^-22 of it or, below fp16's
 //                           normal range, at 2^-25; xl.cl (2^-22) is left out
@@ -32,10 +35,16 @@
 //       30 q                the index kept in the low 4 bits of a~_k
 //     and the reference's distance by (D + 3) u of itself (D additions, the
 //     square twice the difference's rounding).  If k is the reference's
-//     argmin and j has the largest a~, then a~_k >= a~_j - M with
-//       M = (D + 4) u d + u (((192 KS + 84) X + (104 KS + 32) C) C + 8 (X + C))
-//     d bounding the distance of j.  Only centroids with a~_k >= max a~ - M can
-//     be the exact argmin.
+//     argmin and j has the largest a~, then a~_k >= a~_j - M, and with X C <=
+//     (X^2 + C^2) / 2, X + C <= (X^2 + C^2) / 2 + 1
+//       M = (D + 4) u d + u ((96 KS + 48) X^2 + (200 KS + 82) C^2 + 8)
+//     d bounding the distance of j: (1 + 2^-9) ||x|^2 - 2 a~_j| + 3 2^-11 X^2 +
+//     2^-20 max |c| + 2^-31 (its error is below 2^-10 X^2 + 2^-20 (X + max |c|),
+//     and 2^-20 X below 2^-11 X^2 + 2^-31).  Neither j nor k is then farther
+//     from x than sqrt(d), so C^2 = (X + sqrt(d))^2 <= 2 (X^2 + d) will do where
+//     that is less than max |c|^2: a few far centroids do not widen the margin
+//     of the others' rows.  Only centroids with a~_k >= max a~ - M can be the
+//     exact argmin.
 //  3. Each lane keeps the two largest a~ of its even and of its odd centroid
 //     tiles.  If a row's second largest value lies below the limit its
 //     argmin is known (the usual case: no distance is computed).  Otherwise
@@ -65,6 +74,7 @@
 #include <float.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 
 #include "hml_internal.h"
@@ -136,6 +146,23 @@ __device__ __forceinline__ float exact_dist(const float *__restrict__ xr,
   return dist;
 }
 
+// Largest of the lanes' values (none negative), the same in every lane:
+// rotations within rows of 16 lanes, then the four rows.
+__device__ __forceinline__ float wave_max(float x) {
+#define KM_ROR(n) \
+  __builtin_fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + n, 0xf, 0xf, true)))
+  x = KM_ROR(1);
+  x = KM_ROR(2);
+  x = KM_ROR(4);
+  x = KM_ROR(8);
+#undef KM_ROR
+  float m = 0.f;
+#pragma unroll
+  for (int i = 0; i < 64; i += 16)
+    m = __builtin_fmaxf(m, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), i)));
+  return m;
+}
+
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f16v __attribute__((ext_vector_type(16)));
@@ -163,7 +190,7 @@ constexpr float kKmDistMax = 0x1p118f;
 // screen value of an excluded or padding centroid
 constexpr float kKmExcluded = -1e38f;
 constexpr float kKmSampleMax = 0x1p60f;
-constexpr int kKmSampleBytes = kKmWaves * 256;
+constexpr int kKmSampleBytes = (kKmWaves + 1) * 256;  // the sample and the point
 
 // KS = k-steps of 16 dims, MULTI = the centroids take several LDS chunks,
 // VEC = dims a multiple of 4.  Several chunks fill a CU's LDS with one
@@ -174,7 +201,7 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
   constexpr int NQ = KS * 2;  // 1 KB DMA loads per row tile (at most)
   extern __shared__ f4 km_lds4[];
   char *lds = reinterpret_cast<char *>(km_lds4);
-  float *smp = reinterpret_cast<float *>(lds);
+  float *smp = reinterpret_cast<float *>(lds), *mus = smp + 64 * kKmWaves;
   h8 *cf = reinterpret_cast<h8 *>(lds + kKmSampleBytes);  // centroid fragments
   float *nrm = reinterpret_cast<float *>(lds + kKmSampleBytes + (size_t)p.KC * KS * 64);  // -|c|^2 / 2
   // max as a median with infinity (in a register the compiler does not see
@@ -189,32 +216,53 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
   float *xs = nrm + p.KC + w * p.xfloats;  // this wave's row tile
   const int h = lane >> 5, r = lane & 31;
   const int nchunks = MULTI ? (K + p.KC - 1) / p.KC : 1;
-  // The scale sc is a power of two from the largest magnitude in a sample of
-  // centroids, one per wave, exchanged through LDS (smp, a row of 64 dims
-  // each): the loads start here, the exchange shares the barrier that
-  // staging the centroids begins with.
+  // The point that rows and centroids are moved by, and the scale, a power of
+  // two, from a sample of centroids, one per wave: per dim a middle value (a
+  // median of medians) and, over the dims, the largest distance from it but
+  // for one extreme in each group of three.  Centroids that lie about the
+  // origin, no dim's middle farther from it than that, stay: moving each row
+  // costs LDS reads, and the middle of 8 is off by as much.  The sample is
+  // exchanged through LDS (smp, a row of 64 dims each): the loads start here,
+  // the exchange shares the barrier that staging the centroids begins with.
+  // Every wave then writes the same -point x scale to mus.
   const float mine = lane < D ? p.ctrds[(int64_t)((uint64_t)w * (uint32_t)K / kKmWaves) * D + lane] : 0.f;
   float sc = 1.f;
+  bool moved = false;
   auto set_scale = [&]() {
-    float big = 0.f;
+    static_assert(kKmWaves == 8, "groups of a sample of 8");
+    float v[kKmWaves];
+#pragma unroll
+    for (int i = 0; i < kKmWaves; ++i) v[i] = smp[64 * i + lane];
+    auto med = [](float a, float b, float c) { return __builtin_amdgcn_fmed3f(a, b, c); };
+    float mid = med(med(v[0], v[1], v[2]), med(v[3], v[4], v[5]), 0.5f * v[6] + 0.5f * v[7]);
+    float far = 0.f;
 #pragma unroll
     for (int i = 0; i < kKmWaves; ++i) {
-      const float v = __builtin_fabsf(smp[64 * i + lane]);
-      big = v < kKmSampleMax ? __builtin_fmaxf(big, v) : big;
+      v[i] = __builtin_fabsf(v[i] - mid);
+      far = __builtin_fmaxf(far, v[i]);
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) big = __builtin_fmaxf(big, __shfl_xor(big, off));
+    const float dev = __builtin_fmaxf(__builtin_fmaxf(med(v[0], v[1], v[2]), med(v[3], v[4], v[5])),
+                                      __builtin_fminf(v[6], v[7]));
+    const float at = wave_max(__builtin_fabsf(mid));
+    float big = wave_max(dev);
+    moved = at > big;
+    if (!moved) mid = 0.f;
+    // without any spread all of the sample's, else the point's own size
+    if (!(big > 0.f)) big = wave_max(far);
+    if (!(big > 0.f)) big = at;
     const int ex = min(max((int)(__float_as_uint(big) >> 23) - 127, -60), 60);
-    sc = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane(127 - ex) << 23);
+    sc = __uint_as_float((uint32_t)(127 - ex) << 23);
+    mus[lane] = -mid * sc;
+    wave_lds_sync();
   };
   // margin factors, see the error terms at the top of the file (2^-7 for the
   // second order and the margin's own roundings)
   constexpr float kU = 0x1p-24f * (1.0f + 0x1p-7f);
-  constexpr float kMx = (192 * KS + 84) * kU, kMc = (104 * KS + 32) * kU, kMa = 8 * kU;
+  constexpr float kMx = (96 * KS + 48) * kU, kMc = (200 * KS + 82) * kU;
   const float md = (float)(D + 4) * kU;
 
   // Stages centroids c0 .. c0 + KC - 1 (zeros past K) and returns the
-  // largest norm among those in the screen.  Lanes l and l ^ 32 hold the two
+  // largest |c|^2 among those in the screen.  Lanes l and l ^ 32 hold the two
   // halves of a centroid's dims, in the fragment layout itself: (tile of 32,
   // k-step, hi / lo, lane, 8 dims).
   auto stage = [&](int c0) -> float {
@@ -239,7 +287,7 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
       for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          v[s][j] *= sc;
+          v[s][j] = __builtin_fmaf(v[s][j], sc, mus[16 * s + 8 * h + j]);  // zero past D
           s2 = __builtin_fmaf(v[s][j], v[s][j], s2);
         }
       s2 += __shfl_xor(s2, 32);
@@ -258,14 +306,14 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
       }
     }
     __syncthreads();
-    float mx = 0.f;
+    float mx = 0.f;  // the largest |c|^2 in the screen
     for (int k = lane; k < p.KC; k += 64) {
       const float n2 = nrm[k];
       mx = n2 > 0.5f * kKmExcluded ? __builtin_fmaxf(mx, -2.0f * n2) : mx;
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, off));
-    return __builtin_sqrtf(mx);
+    return mx;
   };
 
   // The wave's 32 rows are one contiguous block of memory, DMAed flat
@@ -328,207 +376,226 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
   };
 
   load_rows(tile);
-  float cmax = 0.f;
-  smp[64 * w + lane] = mine;
+  float cmax2 = 0.f;  // largest |c|^2 so far
+  smp[64 * w + lane] = __builtin_fabsf(mine) < kKmSampleMax ? mine : 0.f;
   if (!MULTI) {
-    cmax = stage(0);
+    cmax2 = stage(0);
   } else {
     __syncthreads();
     set_scale();
   }
+  // absolute terms of M (8 u, and underflow: in the screen and, D 2^-149
+  // unscaled, in the reference) and the largest row in range
+  const float m0 = __builtin_fmaf((float)D * 0x1p-148f * sc, sc, 8 * kU);
+  const float rmax = __builtin_fminf(kKmRowMax, kKmDistMax * sc * sc);
 
-  for (int64_t st = 0; st < p.steps; ++st, tile += wstep) {
-    const int64_t row0 = tile * 32;
-    const bool live = row0 < p.nrows;  // wave-uniform
-    if (!MULTI && !live) break;        // later steps only go further
+  // the row steps; rows that stay where they are have a loop of their own
+  auto steps = [&](auto move) {
+    for (int64_t st = 0; st < p.steps; ++st, tile += wstep) {
+      const int64_t row0 = tile * 32;
+      const bool live = row0 < p.nrows;  // wave-uniform
+      if (!MULTI && !live) break;        // later steps only go further
 
-    h8 xh[KS], xl[KS];
-    float xx = 0.f;
-    if (!MULTI || live) {
-      __builtin_amdgcn_s_waitcnt(kWaitAll);  // the tile is in LDS
-      __builtin_amdgcn_sched_barrier(0);
-      wave_lds_sync();
-      float v[KS][8];
+      h8 xh[KS], xl[KS];
+      float xx = 0.f;
+      if (!MULTI || live) {
+        __builtin_amdgcn_s_waitcnt(kWaitAll);  // the tile is in LDS
+        __builtin_amdgcn_sched_barrier(0);
+        wave_lds_sync();
+        float v[KS][8];
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        if (VEC) {
+        for (int s = 0; s < KS; ++s) {
+          if (VEC) {
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const f4 q = *reinterpret_cast<const f4 *>(xs + xo[2 * s + j]);
+            for (int j = 0; j < 2; ++j) {
+              const f4 q = *reinterpret_cast<const f4 *>(xs + xo[2 * s + j]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[s][4 * j + e] = q[e];
+              for (int e = 0; e < 4; ++e) v[s][4 * j + e] = q[e];
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[s][j] = xs[xo[0] + 16 * s + j];
           }
+        }
+        wave_lds_sync();
+        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);  // the reads above are done
+        __builtin_amdgcn_sched_barrier(0);
+        load_rows(tile + wstep);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (decltype(move)::value) {
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              const f4 q = *reinterpret_cast<const f4 *>(mus + 16 * s + 8 * h + 4 * j);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[s][4 * j + e] = __builtin_fmaf(v[s][4 * j + e], sc, q[e]);
+            }
         } else {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[s][j] = xs[xo[0] + 16 * s + j];
-        }
-      }
-      wave_lds_sync();
-      __builtin_amdgcn_s_waitcnt(kWaitLgkm0);  // the reads above are done
-      __builtin_amdgcn_sched_barrier(0);
-      load_rows(tile + wstep);
-      __builtin_amdgcn_sched_barrier(0);
+          for (int s = 0; s < KS; ++s)
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        if (s == KS - 1) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) v[s][j] = 16 * s + 8 * h + j < D ? v[s][j] : 0.f;
+            for (int j = 0; j < 8; ++j) v[s][j] *= sc;
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          v[s][j] *= sc;
-          xx = __builtin_fmaf(v[s][j], v[s][j], xx);
-        }
-        split8(v[s], xh[s], xl[s]);
-      }
-      xx += __shfl_xor(xx, 32);
-    }
-
-    // lane (h, r), entry i: x.c - |c|^2 / 2 for row r and centroid
-    // 32 tl + 8 (i / 4) + 4 h + i % 4 of the chunk
-    auto screen_tile = [&](int tl) -> f16v {
-      f16v acc;
+        for (int s = 0; s < KS; ++s) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const f4 q = *reinterpret_cast<const f4 *>(nrm + 32 * tl + 8 * i + 4 * h);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[4 * i + e] = q[e];
-      }
-      const h8 *f = cf + tl * KS * 128 + lane;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const h8 ch = f[s * 128], cl = f[s * 128 + 64];
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(cl, xh[s], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch, xl[s], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch, xh[s], acc, 0, 0, 0);
-      }
-      return acc;
-    };
-
-    // The two largest screen values of each lane's even (g = 0) and odd
-    // centroid tiles.  The entry's index in its tile sits in the low 4 bits
-    // of the value; bk holds the first centroid of the largest's tile.
-    float m1[2], m2[2];
-    int bk[2] = {0, 0};
-#pragma unroll
-    for (int g = 0; g < 2; ++g) m1[g] = m2[g] = 2.f * kKmExcluded;
-    for (int c = 0; c < nchunks; ++c) {
-      if (MULTI) {
-        const float cm = stage(c * p.KC);
-        cmax = __builtin_fmaxf(cmax, cm);
-        if (!live) continue;
-      }
-      const int k0 = c * p.KC;
-      const int ntl = (min(p.KC, K - k0) + 31) >> 5;
-      for (int tl = 0; tl < ntl; tl += 2) {
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          if (tl + g >= ntl) break;  // wave-uniform
-          const f16v acc = screen_tile(tl + g);
-          const float was = m1[g];
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const float v = __uint_as_float((__float_as_uint(acc[i]) & ~15u) | (uint32_t)i);
-            m2[g] = __builtin_amdgcn_fmed3f(m1[g], m2[g], v);
-            m1[g] = vmax(m1[g], v);
+          for (int j = 0; j < 8; ++j) {
+            if (s == KS - 1) v[s][j] = 16 * s + 8 * h + j < D ? v[s][j] : 0.f;
+            xx = __builtin_fmaf(v[s][j], v[s][j], xx);
           }
-          bk[g] = m1[g] != was ? k0 + 32 * (tl + g) : bk[g];
+          split8(v[s], xh[s], xl[s]);
         }
+        xx += __shfl_xor(xx, 32);
       }
-    }
 
-    // The row's unique candidate, or refinement of the largest value of each
-    // tracker (need) or of every centroid above the limit (full).
-    float lim = 0.f;
-    uint32_t ans = 0;
-    int kc[2] = {0, 0};
-    bool need = false, full = false;
-    if (!MULTI || live) {
+      // lane (h, r), entry i: x.c - |c|^2 / 2 for row r and centroid
+      // 32 tl + 8 (i / 4) + 4 h + i % 4 of the chunk
+      auto screen_tile = [&](int tl) -> f16v {
+        f16v acc;
 #pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        const int id = (int)(__float_as_uint(m1[g]) & 15u);
-        kc[g] = bk[g] + 8 * (id >> 2) + (id & 3) + 4 * h;
-      }
-      const bool odd = m1[1] > m1[0];
-      const float a1 = odd ? m1[1] : m1[0];  // this lane's largest, its other tracker's
-      const float a2 = odd ? m1[0] : m1[1];
-      const float rest = vmax(m2[0], m2[1]);
-      const int k = odd ? kc[1] : kc[0];
-      const float o1 = __shfl_xor(a1, 32), o2 = __shfl_xor(a2, 32), orest = __shfl_xor(rest, 32);
-      const int ok = __shfl_xor(k, 32);
-      const float s1 = vmax(a1, o1);
-      const float unnamed = vmax(rest, orest);  // every value that no tracker names is below
-      const float s2 = vmax(vmax(unnamed, o1 < a1 ? o1 : a1), vmax(a2, o2));
-      const float X = __builtin_amdgcn_sqrtf(xx);
-      const float d = __builtin_fmaxf(xx - 2.f * s1, 0.f) + 0x1p-10f * xx + 0x1p-20f * (X + cmax);
-      // an absolute term for underflow, in the screen and, D 2^-149 unscaled,
-      // in the reference
-      const float m0 = __builtin_fmaf((float)D * 0x1p-148f * sc, sc, 0x1p-40f);
-      const float M = __builtin_fmaf(kMx * X + kMc * cmax, cmax,
-                                     __builtin_fmaf(kMa, X + cmax, __builtin_fmaf(md, d, m0)));
-      // small enough that no distance overflows and excluded centroids are
-      // farther (false for NaN)
-      const float rmax = __builtin_fminf(kKmRowMax, kKmDistMax * sc * sc);
-      const bool range = xx < rmax && xx - 2.f * s1 < rmax;
-      ans = (uint32_t)(o1 > a1 ? ok : k);
-      need = row0 + r < p.nrows && !(range && s1 - s2 > M);
-      full = need && !(range && s1 - unnamed > M);
-      lim = range ? s1 - M : -__builtin_inff();
-    }
-    const bool any_need = __any(need), any_full = __any(full);
+        for (int i = 0; i < 4; ++i) {
+          const f4 q = *reinterpret_cast<const f4 *>(nrm + 32 * tl + 8 * i + 4 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[4 * i + e] = q[e];
+        }
+        const h8 *f = cf + tl * KS * 128 + lane;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const h8 ch = f[s * 128], cl = f[s * 128 + 64];
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(cl, xh[s], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch, xl[s], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch, xh[s], acc, 0, 0, 0);
+        }
+        return acc;
+      };
 
-    // Reference distances of the candidates, the two lanes of a row their
-    // own; equal distances go to the smaller index (the reference's first
-    // strict minimum).
-    float bd = FLT_MAX;
-    uint32_t bi = kNone;
-    auto refine = [&](int k) {
-      const float dist = exact_dist<FUSED, KS>(p.rows + (row0 + r) * D, p.ctrds + (int64_t)k * D, D);
-      if (dist < bd || (dist == bd && bi != kNone && (uint32_t)k < bi)) {
-        bd = dist;
-        bi = (uint32_t)k;
-      }
-    };
-    if (any_need) {
-      uint32_t cand = need && !full ? (m1[0] >= lim ? 1u : 0u) | (m1[1] >= lim ? 2u : 0u) : 0u;
-      while (cand) {
-        const bool g0 = cand & 1u;
-        cand &= cand - 1;
-        refine(g0 ? kc[0] : kc[1]);
-      }
-    }
-    if (MULTI ? (bool)__syncthreads_or(any_full) : any_full) {
-#pragma unroll 1
+      // The two largest screen values of each lane's even (g = 0) and odd
+      // centroid tiles.  The entry's index in its tile sits in the low 4 bits
+      // of the value; bk holds the first centroid of the largest's tile.
+      float m1[2], m2[2];
+      int bk[2] = {0, 0};
+#pragma unroll
+      for (int g = 0; g < 2; ++g) m1[g] = m2[g] = 2.f * kKmExcluded;
       for (int c = 0; c < nchunks; ++c) {
         if (MULTI) {
-          stage(c * p.KC);
-          if (!any_full) continue;
+          const float cm = stage(c * p.KC);
+          cmax2 = __builtin_fmaxf(cmax2, cm);
+          if (!live) continue;
         }
         const int k0 = c * p.KC;
         const int ntl = (min(p.KC, K - k0) + 31) >> 5;
-#pragma unroll 1
-        for (int tl = 0; tl < ntl; ++tl) {
-          const f16v acc = screen_tile(tl);
-          uint32_t cand = 0;
+        for (int tl = 0; tl < ntl; tl += 2) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) cand |= full && !(acc[i] < lim) ? 1u << i : 0u;
-          while (cand) {
-            const int b = __builtin_ctz(cand);
-            cand &= cand - 1;
-            const int k = k0 + 32 * tl + 8 * (b >> 2) + 4 * h + (b & 3);
-            if (k < K) refine(k);
+          for (int g = 0; g < 2; ++g) {
+            if (tl + g >= ntl) break;  // wave-uniform
+            const f16v acc = screen_tile(tl + g);
+            const float was = m1[g];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const float v = __uint_as_float((__float_as_uint(acc[i]) & ~15u) | (uint32_t)i);
+              m2[g] = __builtin_amdgcn_fmed3f(m1[g], m2[g], v);
+              m1[g] = vmax(m1[g], v);
+            }
+            bk[g] = m1[g] != was ? k0 + 32 * (tl + g) : bk[g];
           }
         }
       }
+
+      const float d0 = __builtin_fmaf(0x1p-20f, __builtin_amdgcn_sqrtf(cmax2), 0x1p-31f);  // absolute part of d
+      // The row's unique candidate, or refinement of the largest value of each
+      // tracker (need) or of every centroid above the limit (full).
+      float lim = 0.f;
+      uint32_t ans = 0;
+      int kc[2] = {0, 0};
+      bool need = false, full = false;
+      if (!MULTI || live) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          const int id = (int)(__float_as_uint(m1[g]) & 15u);
+          kc[g] = bk[g] + 8 * (id >> 2) + (id & 3) + 4 * h;
+        }
+        const bool odd = m1[1] > m1[0];
+        const float a1 = odd ? m1[1] : m1[0];  // this lane's largest, its other tracker's
+        const float a2 = odd ? m1[0] : m1[1];
+        const float rest = vmax(m2[0], m2[1]);
+        const int k = odd ? kc[1] : kc[0];
+        const float o1 = __shfl_xor(a1, 32), o2 = __shfl_xor(a2, 32), orest = __shfl_xor(rest, 32);
+        const int ok = __shfl_xor(k, 32);
+        const float s1 = vmax(a1, o1);
+        const float unnamed = vmax(rest, orest);  // every value that no tracker names is below
+        const float s2 = vmax(vmax(unnamed, o1 < a1 ? o1 : a1), vmax(a2, o2));
+        const float t = xx - 2.f * s1;
+        const float d = __builtin_fmaf(1.0f + 0x1p-9f, __builtin_fabsf(t), __builtin_fmaf(3 * 0x1p-11f, xx, d0));
+        const float C2 = __builtin_fminf(cmax2, 2.f * (xx + d));
+        const float M = __builtin_fmaf(kMx, xx, __builtin_fmaf(kMc, C2, __builtin_fmaf(md, d, m0)));
+        // small enough that no distance overflows and excluded centroids are
+        // farther (false for NaN)
+        const bool range = xx < rmax && t < rmax;
+        ans = (uint32_t)(o1 > a1 ? ok : k);
+        need = row0 + r < p.nrows && !(range && s1 - s2 > M);
+        full = need && !(range && s1 - unnamed > M);
+        lim = range ? s1 - M : -__builtin_inff();
+      }
+      const bool any_need = __any(need), any_full = __any(full);
+
+      // Reference distances of the candidates, the two lanes of a row their
+      // own; equal distances go to the smaller index (the reference's first
+      // strict minimum).
+      float bd = FLT_MAX;
+      uint32_t bi = kNone;
+      auto refine = [&](int k) {
+        const float dist = exact_dist<FUSED, KS>(p.rows + (row0 + r) * D, p.ctrds + (int64_t)k * D, D);
+        if (dist < bd || (dist == bd && bi != kNone && (uint32_t)k < bi)) {
+          bd = dist;
+          bi = (uint32_t)k;
+        }
+      };
+      if (any_need) {
+        uint32_t cand = need && !full ? (m1[0] >= lim ? 1u : 0u) | (m1[1] >= lim ? 2u : 0u) : 0u;
+        while (cand) {
+          const bool g0 = cand & 1u;
+          cand &= cand - 1;
+          refine(g0 ? kc[0] : kc[1]);
+        }
+      }
+      if (MULTI ? (bool)__syncthreads_or(any_full) : any_full) {
+#pragma unroll 1
+        for (int c = 0; c < nchunks; ++c) {
+          if (MULTI) {
+            stage(c * p.KC);
+            if (!any_full) continue;
+          }
+          const int k0 = c * p.KC;
+          const int ntl = (min(p.KC, K - k0) + 31) >> 5;
+#pragma unroll 1
+          for (int tl = 0; tl < ntl; ++tl) {
+            const f16v acc = screen_tile(tl);
+            uint32_t cand = 0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) cand |= full && !(acc[i] < lim) ? 1u << i : 0u;
+            while (cand) {
+              const int b = __builtin_ctz(cand);
+              cand &= cand - 1;
+              const int k = k0 + 32 * tl + 8 * (b >> 2) + 4 * h + (b & 3);
+              if (k < K) refine(k);
+            }
+          }
+        }
+      }
+      if (any_need) {
+        const float od = __shfl_xor(bd, 32);
+        const uint32_t oi = (uint32_t)__shfl_xor((int)bi, 32);
+        if (od < bd || (od == bd && oi < bi)) bi = oi;
+        if (need) ans = bi == kNone ? (uint32_t)K : bi;
+      }
+      if ((!MULTI || live) && h == 0 && row0 + r < p.nrows) p.assign[row0 + r] = ans;
     }
-    if (any_need) {
-      const float od = __shfl_xor(bd, 32);
-      const uint32_t oi = (uint32_t)__shfl_xor((int)bi, 32);
-      if (od < bd || (od == bd && oi < bi)) bi = oi;
-      if (need) ans = bi == kNone ? (uint32_t)K : bi;
-    }
-    if ((!MULTI || live) && h == 0 && row0 + r < p.nrows) p.assign[row0 + r] = ans;
-  }
+  };
+  if (moved)
+    steps(std::true_type());
+  else
+    steps(std::false_type());
 }
 
 typedef void (*KmKernel)(KmParams);

@@ -198,3 +198,57 @@ def test_screen_edges(hml, D, K):
             want = oracle.kmeans_assign(r, cc)
             got = run(hml, r, cc, kernel="screened")
             np.testing.assert_array_equal(got, want, err_msg="scale %g" % scale)
+
+
+@pytest.mark.parametrize("D,K", [(4, 70), (17, 33), (32, 64), (50, 100), (64, 300)])
+def test_off_centre(hml, D, K):
+    """Rows and centroids far from the origin, with a far centroid, with most
+    of the sampled centroids equal or not finite: the point that the screen
+    moves them by, and its scale, change no index."""
+    rng = np.random.default_rng(D + K)
+    for make in (clustered, near_ties):
+        rows, ctrds = make(rng, 1500, D, K)
+        for off in (3.0, 300.0, 3e4, np.float32(1e4) * rng.standard_normal(D).astype(np.float32)):
+            for change in (None, "far", "equal", "nan"):
+                r, c = (rows + off).astype(np.float32), (ctrds + off).astype(np.float32)
+                if change == "far":
+                    c[K // 2] += 1e3
+                elif change == "equal":
+                    c[: K - 3] = c[0]
+                elif change == "nan":
+                    c[:: max(1, K // 8)] = np.nan
+                want = oracle.kmeans_assign(r, c)
+                got = run(hml, r, c, kernel="screened")
+                np.testing.assert_array_equal(got, want, err_msg="%s %s %s" % (make.__name__, off, change))
+
+
+def seconds(hml, rows, ctrds, reps=20):
+    """Best of three timings of `reps` assignments."""
+    n, D = rows.shape
+    dr, dc = hml.DeviceBuffer.from_numpy(rows), hml.DeviceBuffer.from_numpy(ctrds)
+    da = hml.DeviceBuffer(4 * n)
+    best = float("inf")
+    for _ in range(4):
+        e0, e1 = hml.Event(), hml.Event()
+        e0.record()
+        for _ in range(reps):
+            hml.kmeans_assign(dr, dc, da, n, D, ctrds.shape[0], kernel="screened")
+        e1.record()
+        e1.synchronize()
+        best = min(best, e0.elapsed_ms(e1) / reps)
+    return best
+
+
+@pytest.mark.parametrize("D,K", [(32, 64), (64, 256)])
+def test_off_centre_is_not_slower(hml, D, K):
+    """Moving the data away from the origin, or one centroid away from the
+    others, does not send every row to the exact comparison (30 times slower
+    when it does): within 3 times the centred time."""
+    rng = np.random.default_rng(1)
+    ctrds = rng.uniform(-1, 1, (K, D)).astype(np.float32)
+    rows = rng.uniform(-1, 1, (1 << 17, D)).astype(np.float32)
+    centred = seconds(hml, rows, ctrds)
+    far = ctrds.copy()
+    far[K // 2] = 1000.0
+    for r, c in ((rows + np.float32(100), ctrds + np.float32(100)), (rows, far)):
+        assert seconds(hml, r, c) < 3 * centred

@@ -19,12 +19,13 @@ U = 2.0 ** -24
 
 
 def factors(ks):
-    """(kMx, kMc, kMa) of the source for ks k-steps, in units of u."""
+    """The source's factors of |x|^2 and |c|^2 and its constant for ks
+    k-steps, in units of u."""
     text = open(SRC).read()
-    m = re.search(r"kMx = \((\d+) \* KS \+ (\d+)\) \* kU, kMc = \((\d+) \* KS \+ (\d+)\) \* kU, "
-                  r"kMa = (\d+) \* kU", text)
-    a, b, c, d, e = (int(v) for v in m.groups())
-    return a * ks + b, c * ks + d, e
+    a, b, c, d = (int(v) for v in re.search(
+        r"kMx = \((\d+) \* KS \+ (\d+)\) \* kU, kMc = \((\d+) \* KS \+ (\d+)\) \* kU;", text).groups())
+    e, = re.search(r"const float m0 = .*, (\d+) \* kU\);", text).groups()
+    return a * ks + b, c * ks + d, int(e)
 
 
 def terms(v):
@@ -70,7 +71,7 @@ def test_margin_covers_the_screen(D):
         x64, c64 = x.astype(np.float64), c.astype(np.float64)
         a = (x64 * c64).sum(1) - 0.5 * (c64 ** 2).sum(1)
         X, C = np.linalg.norm(x64, axis=1), np.linalg.norm(c64, axis=1)
-        half = 0.5 * U * ((mx * X + mc * C) * C + ma * (X + C)) + 2.0 ** -41
+        half = 0.5 * U * (mx * X ** 2 + mc * C ** 2 + ma)
         for got in screen(x, c):
             err = np.abs(got.astype(np.float64) - a)
             assert (err <= half).all(), (err / half).max()
