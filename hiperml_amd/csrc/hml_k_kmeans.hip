@@ -48,12 +48,14 @@
 //  3. Each lane keeps the two largest a~ of its even and of its odd centroid
 //     tiles.  If a row's second largest value lies below the limit its
 //     argmin is known (the usual case: no distance is computed).  Otherwise
-//     the trackers' centroids above the limit are compared by the
-//     reference's own arithmetic, or, when a value that no tracker names
-//     could be above it, the tile is screened again and every centroid above
-//     the limit compared.  The two lanes of a row hold disjoint centroids
-//     and combine by (distance, index): the reference's "first strict
-//     minimum".
+//     the trackers' centroids above the limit or, when a value that no tracker
+//     names could be above it, all centroids above it (found by screening the
+//     tile again) are compared by the reference's own arithmetic.  A wave
+//     gathers such (row, centroid) pairs over its lanes and compares 64 at a
+//     time, a lane each; the smallest (distance, index) of a row is the
+//     reference's "first strict minimum".  Each lane on its own candidates in
+//     turn waited for memory once per candidate of the busiest lane: 0/1
+//     features, 2^20 rows 32 x 64, 135 us, now 61.
 //
 // What bounds it: for few centroids the row stream (2^24 rows, 32 dims x 16
 // clusters: 0.38 ms, 5.8 TB/s, was 0.54), for many the matrix cores and the
@@ -62,8 +64,7 @@
 // 0.46 ms (was 1.04), 64 x 64 0.96 (was 1.75), 2^23 rows 64 x 256 0.92 (was
 // 3.11).  64 rows per wave halve the LDS reads per row but held 2-3 waves
 // per SIMD: 2-15% slower.  Four trackers per lane make the second screening
-// rarer and cost registers: up to 10% slower.  Rows equidistant from many
-// centroids cost up to two screenings and a distance per candidate.
+// rarer and cost registers: up to 10% slower.
 //
 // Centroids live in LDS as fp16 terms in MFMA operand order (a fragment is
 // one conflict-free 16-byte read per lane) beside their norms, staged once
@@ -190,7 +191,9 @@ constexpr float kKmDistMax = 0x1p118f;
 // screen value of an excluded or padding centroid
 constexpr float kKmExcluded = -1e38f;
 constexpr float kKmSampleMax = 0x1p60f;
-constexpr int kKmSampleBytes = (kKmWaves + 1) * 256;  // the sample and the point
+// LDS before the centroids: the sample (later the pairs to compare), the
+// point, the rows' best keys and the pairs' rows
+constexpr int kKmHeadBytes = (2 * kKmWaves + 1) * 256 + kKmWaves * 64;
 
 // KS = k-steps of 16 dims, MULTI = the centroids take several LDS chunks,
 // VEC = dims a multiple of 4.  Several chunks fill a CU's LDS with one
@@ -202,8 +205,8 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
   extern __shared__ f4 km_lds4[];
   char *lds = reinterpret_cast<char *>(km_lds4);
   float *smp = reinterpret_cast<float *>(lds), *mus = smp + 64 * kKmWaves;
-  h8 *cf = reinterpret_cast<h8 *>(lds + kKmSampleBytes);  // centroid fragments
-  float *nrm = reinterpret_cast<float *>(lds + kKmSampleBytes + (size_t)p.KC * KS * 64);  // -|c|^2 / 2
+  h8 *cf = reinterpret_cast<h8 *>(lds + kKmHeadBytes);  // centroid fragments
+  float *nrm = reinterpret_cast<float *>(lds + kKmHeadBytes + (size_t)p.KC * KS * 64);  // -|c|^2 / 2
   // max as a median with infinity (in a register the compiler does not see
   // through), without the canonicalising moves fmaxf needs for unknown
   // inputs; a result that a NaN could have entered is never used
@@ -214,6 +217,11 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int D = p.D, K = p.K;
   float *xs = nrm + p.KC + w * p.xfloats;  // this wave's row tile
+  // this wave's pairs to compare (the sample's row, once that is used) and
+  // the best of each of its rows
+  int *pair_k = reinterpret_cast<int *>(smp + 64 * w);
+  unsigned long long *best = reinterpret_cast<unsigned long long *>(lds + (kKmWaves + 1) * 256) + 32 * w;
+  uint8_t *pair_r = reinterpret_cast<uint8_t *>(lds + (2 * kKmWaves + 1) * 256) + 64 * w;
   const int h = lane >> 5, r = lane & 31;
   const int nchunks = MULTI ? (K + p.KC - 1) / p.KC : 1;
   // The point that rows and centroids are moved by, and the scale, a power of
@@ -503,8 +511,8 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
       }
 
       const float d0 = __builtin_fmaf(0x1p-20f, __builtin_amdgcn_sqrtf(cmax2), 0x1p-31f);  // absolute part of d
-      // The row's unique candidate, or refinement of the largest value of each
-      // tracker (need) or of every centroid above the limit (full).
+      // The row's unique candidate, or a comparison of the trackers' largest
+      // values (need) or of every centroid above the limit (full).
       float lim = 0.f;
       uint32_t ans = 0;
       int kc[2] = {0, 0};
@@ -539,25 +547,41 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
       }
       const bool any_need = __any(need), any_full = __any(full);
 
-      // Reference distances of the candidates, the two lanes of a row their
-      // own; equal distances go to the smaller index (the reference's first
-      // strict minimum).
-      float bd = FLT_MAX;
-      uint32_t bi = kNone;
-      auto refine = [&](int k) {
-        const float dist = exact_dist<FUSED, KS>(p.rows + (row0 + r) * D, p.ctrds + (int64_t)k * D, D);
-        if (dist < bd || (dist == bd && bi != kNone && (uint32_t)k < bi)) {
-          bd = dist;
-          bi = (uint32_t)k;
+      // Reference distances of the candidates: (row, centroid) pairs gathered
+      // over the wave, 64 at a time, a lane each.  The smallest (distance,
+      // index) of a row is the reference's first strict minimum.
+      int npair = 0;  // wave-uniform
+      auto compare = [&]() {
+        wave_lds_sync();
+        if (lane < npair) {
+          const int k = pair_k[lane], rr = pair_r[lane];
+          const float dist = exact_dist<FUSED, KS>(p.rows + (row0 + rr) * D, p.ctrds + (int64_t)k * D, D);
+          if (dist < FLT_MAX)
+            atomicMin(best + rr, (unsigned long long)__float_as_uint(dist) << 32 | (uint32_t)k);
+        }
+        wave_lds_sync();
+        npair = 0;
+      };
+      // the set bits of cand, each a centroid of the lane's row
+      auto gather = [&](uint32_t cand, auto centroid) {
+        while (const unsigned long long who = __ballot(cand != 0)) {
+          const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0));
+          if (cand && npair + rank < 64) {
+            pair_k[npair + rank] = centroid(__builtin_ctz(cand));
+            pair_r[npair + rank] = (uint8_t)r;
+            cand &= cand - 1;
+          }
+          npair = min(64, npair + (int)__popcll(who));
+          if (npair == 64) compare();
         }
       };
       if (any_need) {
-        uint32_t cand = need && !full ? (m1[0] >= lim ? 1u : 0u) | (m1[1] >= lim ? 2u : 0u) : 0u;
-        while (cand) {
-          const bool g0 = cand & 1u;
-          cand &= cand - 1;
-          refine(g0 ? kc[0] : kc[1]);
-        }
+        if (h == 0) best[r] = ~0ull;
+        wave_lds_sync();
+        if (!any_full)
+          gather(need ? (m1[0] >= lim ? 1u : 0u) | (m1[1] >= lim ? 2u : 0u) : 0u,
+                 [&](int b) { return kc[b]; });
       }
       if (MULTI ? (bool)__syncthreads_or(any_full) : any_full) {
 #pragma unroll 1
@@ -571,23 +595,19 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
 #pragma unroll 1
           for (int tl = 0; tl < ntl; ++tl) {
             const f16v acc = screen_tile(tl);
+            const int k = k0 + 32 * tl + 4 * h;
             uint32_t cand = 0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) cand |= full && !(acc[i] < lim) ? 1u << i : 0u;
-            while (cand) {
-              const int b = __builtin_ctz(cand);
-              cand &= cand - 1;
-              const int k = k0 + 32 * tl + 8 * (b >> 2) + 4 * h + (b & 3);
-              if (k < K) refine(k);
-            }
+            for (int i = 0; i < 16; ++i)
+              cand |= !(acc[i] < lim) && k + 8 * (i >> 2) + (i & 3) < K ? 1u << i : 0u;
+            gather(need ? cand : 0u, [&](int b) { return k + 8 * (b >> 2) + (b & 3); });
           }
         }
       }
       if (any_need) {
-        const float od = __shfl_xor(bd, 32);
-        const uint32_t oi = (uint32_t)__shfl_xor((int)bi, 32);
-        if (od < bd || (od == bd && oi < bi)) bi = oi;
-        if (need) ans = bi == kNone ? (uint32_t)K : bi;
+        if (npair) compare();
+        const unsigned long long key = best[r];
+        if (need) ans = key == ~0ull ? (uint32_t)K : (uint32_t)key;
       }
       if ((!MULTI || live) && h == 0 && row0 + r < p.nrows) p.assign[row0 + r] = ans;
     }
@@ -777,7 +797,7 @@ KmeansPlan plan_kmeans(int64_t nrows, int D, int K, int mode) {
   // its norm, each wave's row tile in whole 1 KB loads, 256 bytes that reads past the last tile's
   // last row may touch, and 256 for the workgroup vote
   pl.xfloats = (D + 7) / 8 * 256;
-  const int64_t rows_b = (int64_t)kKmWaves * pl.xfloats * 4 + 256 + kKmSampleBytes;
+  const int64_t rows_b = (int64_t)kKmWaves * pl.xfloats * 4 + 256 + kKmHeadBytes;
   const int64_t room = (int64_t)kKmLdsBytes - 256 - rows_b;
   pl.KC = (int)std::min<int64_t>(kpad, room / (64 * pl.ni + 4) / 32 * 32);
   pl.lds = (size_t)(pl.KC * (64 * pl.ni + 4) + rows_b);
