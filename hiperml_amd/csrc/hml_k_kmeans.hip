@@ -278,11 +278,23 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
     auto load = [&](int i) {  // the 8 KS dims of thread item i
       const int k = 32 * (i >> 6) + r;
       const float *c = p.ctrds + (int64_t)(c0 + k) * D + 8 * h;
+      const int n = i < p.KC * 2 && c0 + k < K ? D - 8 * h : 0;  // floats at c
 #pragma unroll
       for (int s = 0; s < KS; ++s)
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          v[s][j] = i < p.KC * 2 && c0 + k < K && 16 * s + 8 * h + j < D ? c[16 * s + j] : 0.f;
+        for (int j = 0; j < 8; j += 4) {
+          // 16 bytes at a time: element loads are 64 lines each, 10 us per
+          // chunk of 350 centroids of 64 dims
+          KmQuad q = {};
+          if (16 * s + j + 4 <= n)
+            q = *reinterpret_cast<const KmQuad *>(c + 16 * s + j);
+          else if (!VEC)
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+              if (16 * s + j + e < n) q.v[e] = c[16 * s + j + e];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[s][j + e] = q.v[e];
+        }
     };
     if (!MULTI) load(threadIdx.x);
     __syncthreads();  // every wave is done with the previous chunk, or has its sample in LDS
