@@ -228,14 +228,15 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
   // two, from a sample of centroids, one per wave: per dim a middle value (a
   // median of medians) and, over the dims, the largest distance from it but
   // for one extreme in each group of three.  Centroids that lie about the
-  // origin, no dim's middle farther from it than that, stay: moving each row
-  // costs LDS reads, and the middle of 8 is off by as much.  The sample is
+  // origin, no dim's middle farther from it than that, stay (moving each row
+  // costs LDS reads, and the middle of 8 is off by as much), and where they are
+  // of a size of 1/2 to 64 nothing is scaled either.  The sample is
   // exchanged through LDS (smp, a row of 64 dims each): the loads start here,
   // the exchange shares the barrier that staging the centroids begins with.
   // Every wave then writes the same -point x scale to mus.
   const float mine = lane < D ? p.ctrds[(int64_t)((uint64_t)w * (uint32_t)K / kKmWaves) * D + lane] : 0.f;
   float sc = 1.f;
-  bool moved = false;
+  bool moved = false;  // or scaled
   auto set_scale = [&]() {
     static_assert(kKmWaves == 8, "groups of a sample of 8");
     float v[kKmWaves];
@@ -253,12 +254,14 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
                                       __builtin_fminf(v[6], v[7]));
     const float at = wave_max(__builtin_fabsf(mid));
     float big = wave_max(dev);
-    moved = at > big;
-    if (!moved) mid = 0.f;
+    const bool off = at > big;
+    if (!off) mid = 0.f;
     // without any spread all of the sample's, else the point's own size
     if (!(big > 0.f)) big = wave_max(far);
     if (!(big > 0.f)) big = at;
-    const int ex = min(max((int)(__float_as_uint(big) >> 23) - 127, -60), 60);
+    int ex = min(max((int)(__float_as_uint(big) >> 23) - 127, -60), 60);
+    moved = off || ex < -1 || ex > 5;
+    if (!moved) ex = 0;
     sc = __uint_as_float((uint32_t)(127 - ex) << 23);
     mus[lane] = -mid * sc;
     wave_lds_sync();
@@ -409,7 +412,7 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
   const float m0 = __builtin_fmaf((float)D * 0x1p-148f * sc, sc, 8 * kU);
   const float rmax = __builtin_fminf(kKmRowMax, kKmDistMax * sc * sc);
 
-  // the row steps; rows that stay where they are have a loop of their own
+  // the row steps; rows that stay as they are have a loop of their own
   auto steps = [&](auto move) {
     for (int64_t st = 0; st < p.steps; ++st, tile += wstep) {
       const int64_t row0 = tile * 32;
@@ -451,11 +454,6 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
 #pragma unroll
               for (int e = 0; e < 4; ++e) v[s][4 * j + e] = __builtin_fmaf(v[s][4 * j + e], sc, q[e]);
             }
-        } else {
-#pragma unroll
-          for (int s = 0; s < KS; ++s)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[s][j] *= sc;
         }
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
