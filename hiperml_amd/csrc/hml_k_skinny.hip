@@ -516,23 +516,43 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
       }
       ap[q] = x;
     }
-#pragma unroll
-    for (int c = 0; c < CT; ++c)
+    if constexpr (BROW) {
+      // CT columns per load here too: element by element, a lane's columns lie
+      // CT apart from the next lane's and a load touches 4 times the lines (us,
+      // element loads / these: 53090 x 104 x 34 27.1 / 18.3, x 98 34.9 / 27.9,
+      // 37457 x 772 x 120 133 / 110)
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int v = 0; v < 2; ++v) {
-          f4 x;
+        for (int v = 0; v < 2; ++v)
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {
             const int64_t ko = nst * kDotStageK + 32 * u + 16 * v + jj;
-            const uint32_t bo = boff[BROW ? 0 : c];
-            const uint32_t vo = (bo == kOOB || kb + ko + 4 * g >= ke) ? kOOB
-                                : bo + (uint32_t)((ko * sBk + (BROW ? c : 0)) * 4);
-            x[jj] = buf_load1(rbs, vo, 0);
+            const uint32_t vo = (boff[0] == kOOB || kb + ko + 4 * g >= ke)
+                                    ? kOOB : boff[0] + (uint32_t)(ko * sBk * 4);
+            float x[CT];
+            buf_load_n<CT>(rbs, vo, 0, x);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) b[c][u][v][jj] = x[c];
           }
-          b[c][u][v] = x;
-        }
+    } else {
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int v = 0; v < 2; ++v) {
+            f4 x;
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj) {
+              const int64_t ko = nst * kDotStageK + 32 * u + 16 * v + jj;
+              const uint32_t vo = (boff[c] == kOOB || kb + ko + 4 * g >= ke)
+                                      ? kOOB : boff[c] + (uint32_t)(ko * sBk * 4);
+              x[jj] = buf_load1(rbs, vo, 0);
+            }
+            b[c][u][v] = x;
+          }
+    }
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
       *reinterpret_cast<f4 *>(T + dot_tile_off(4 * q + g, r)) = ap[q];

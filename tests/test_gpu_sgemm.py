@@ -710,3 +710,22 @@ def test_replacement_runs(hml, M, N, K, family):
     assert v[0] == family
     np.testing.assert_array_equal(run_gemm(hml, A, B, C0, 1.0, 0.0),
                                   run_gemm(hml, A, B, C0, 1.0, 0.0, variant=v))
+
+
+@pytest.mark.parametrize("K", [1, 3, 17, 31, 33, 63, 65, 100, 127])
+def test_partial_stage_columns(hml, K):
+    """The partial stage of the 3- and 4-column tiles reads a lane's columns at
+    once: every k remainder, columns that end inside a lane's, B's last row
+    ending its allocation, NaN beside B and behind A's k."""
+    rng = np.random.default_rng(K)
+    for M, N, pad in ((40, 33, 0), (33, 4, 3), (70, 62, 0), (70, 62, 1), (35, 35, 5)):
+        A, B, C0 = int_matrix(rng, (M, K)), int_matrix(rng, (K, N)), int_matrix(rng, (M, N))
+        R = exact_product(A, B, 2.0, -1.0, C0)
+        Aw, Bw = np.full((M, K + pad), np.nan, np.float32), np.full((K, N + pad), np.nan, np.float32)
+        Aw[:, :K], Bw[:, :N] = A, B
+        dA, dB = hml.DeviceBuffer.from_numpy(Aw), hml.DeviceBuffer.from_numpy(Bw.ravel()[:(K - 1) * (N + pad) + N])
+        for v in ((1, 1, 3, 1, 1), (1, 2, 3, 1, 1), (1, 1, 4, 1, 1), (1, 2, 4, 1, 1), (1, 2, 4, 2, 2)):
+            dC = hml.DeviceBuffer.from_numpy(C0)
+            hml.sgemm_ex(M, N, K, dA, dB, dC, 2.0, -1.0, lda=K + pad, ldb=N + pad, variant=v)
+            hml.synchronize()
+            np.testing.assert_array_equal(dC.to_numpy((M, N)), R, err_msg="%r %r" % (v, (M, N, pad)))
