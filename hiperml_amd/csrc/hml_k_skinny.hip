@@ -24,6 +24,7 @@
 //    are summed in a fixed order by a second kernel (deterministic, no
 //    atomics).
 #include <algorithm>
+#include <type_traits>
 #include <mutex>
 
 #include "hml_internal.h"
@@ -161,6 +162,20 @@ __device__ __forceinline__ void dot_store(const DotParams &p, int64_t row,
   }
 }
 
+// Whether a grid of `waves` waves spreads B's loads over the stage.  A wave
+// alone on its SIMD gains (it waits for nothing else), as do 16-row tiles,
+// whose stages are short; with more than two waves of a 32-row tile for each
+// SIMD the others fill its waits, and the barriers that keep the loads spread
+// only hold them back.  us, spread / not: 2x4, 546 waves 8730 x 98 x 926 36.3 /
+// 39.9, 1976 7885 x 460 x 726 61.1 / 63.4, 2048 8192 x 128 x 8192 135.0 /
+// 138.2, 2656 5283 x 97 x 8840 154 / 125, 3008 6000 x 64 x 6144 63.7 / 52.7,
+// 3014 48224 x 128 x 896 141 / 118, 12032 3001 x 2047 x 2500 271 / 263; 2x3,
+// 488 1926 x 90 x 3287 25.1 / 28.1, 4560 36457 x 35 x 4415 176.7 / 173.7; 1x4,
+// 3300 53090 x 104 x 64 16.8 / 17.5, 1x3 1320 x 127 x 7978 37.0 / 40.2.
+__host__ __device__ constexpr bool dot_spread(int rt, int ct, bool bvec, int64_t waves) {
+  return !bvec && ct >= 3 && (rt == 1 || waves <= 2 * 4 * 256);
+}
+
 // Columns of lane r in a tile of CT column tiles that starts at column n0:
 // n0 + 16 c + r in tile c or, for N-contiguous B and 3 or 4 tiles (BROW), the
 // CT consecutive columns base .. base + CT - 1, one per tile, so that one
@@ -277,7 +292,7 @@ __device__ __forceinline__ void buf_load_n(__amdgpu_buffer_rsrc_t rs, uint32_t v
 // there are so the NQ of the next stage's A and at least one stage of B.
 // Before a stage's reads: vmcnt(NQ); SPREAD, with 16 loads of B per stage,
 // vmcnt(NQ + 8).  Before a tile is refilled: lgkmcnt(0) (its reads are done).
-template <int RT, int CT, bool BVEC, bool DMA, int APOL = kBufNT>
+template <int RT, int CT, bool BVEC, bool DMA, int APOL, bool SPREAD>
 __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_t sAm,
                                              const float *__restrict__ B, int64_t sBk,
                                              int64_t sBn, int64_t M, int64_t N,
@@ -287,6 +302,7 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
   constexpr int NQ = 4 * RT;  // A load instructions per stage
   constexpr int TF = dot_tile_floats(RT);
   constexpr bool BROW = dot_brow(CT, BVEC);
+  static_assert(!SPREAD || (DMA && BROW), "spread loads: DMA tiles, N-contiguous B");
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
   const int64_t nst = ke > kb ? (ke - kb) / kDotStageK : 0;
@@ -377,15 +393,10 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
       *reinterpret_cast<f4 *>(Tj + dot_tile_off(4 * q + g, r)) = a[j][q];
     wave_sync();
   };
-  // The DMA tiles with N-contiguous B: each B register is refilled right
-  // behind the MFMAs that read it, and the tile is read one half k-step
-  // ahead, a scheduling barrier per MFMA group keeping the loads spread over
-  // the stage.  Left to the scheduler they gather at the stage's end and the
-  // next stage waits for them.  8192 x 64 x 8192 (K split 4): 94 us with
-  // element loads of B in one burst, 91 with CT-column loads, 83 spread;
-  // 8192 x 128 x 8192 153 / 144 / 138.  K-contiguous B and fewer column tiles
-  // load little enough that the plain order is as good or better.
-  constexpr bool SPREAD = DMA && BROW;
+  // SPREAD: each B register is refilled right behind the MFMAs that read it,
+  // and the tile is read one half k-step ahead, a scheduling barrier per MFMA
+  // group keeping the loads spread over the stage; left to the scheduler they
+  // gather at the stage's end.  dot_spread says where.
   auto compute_spread = [&](const float *Tj, int64_t s_next) {
     const __amdgpu_buffer_rsrc_t rs = s_next < nst ? rbs : rnull;
     f4 x[2][RT];
@@ -563,7 +574,7 @@ __device__ __forceinline__ void dot_tile_lds(const float *__restrict__ A, int64_
   }
 }
 
-template <int RT, int CT, bool BVEC, int APOL = kBufNT>
+template <int RT, int CT, bool BVEC, int APOL, bool SPREAD>
 __global__ __launch_bounds__(64 * dot_max_waves(RT, CT)) void k_skinny_dot(DotParams p) {
   constexpr int WF = dot_wave_floats(RT, CT);
   extern __shared__ f4 dot_lds[];
@@ -584,7 +595,7 @@ __global__ __launch_bounds__(64 * dot_max_waves(RT, CT)) void k_skinny_dot(DotPa
   int64_t ke = kb + p.kchunk;
   if (ke > p.K) ke = p.K;
   f4 acc[RT][CT];
-  dot_tile_lds<RT, CT, BVEC, dot_dma(RT, CT), APOL>(p.A, p.sAm, p.B, p.sBk, p.sBn, p.M, p.N,
+  dot_tile_lds<RT, CT, BVEC, dot_dma(RT, CT), APOL, SPREAD>(p.A, p.sAm, p.B, p.sBk, p.sBn, p.M, p.N,
                                                    row0, ct0, kb, ke,
                                                    reinterpret_cast<float *>(dot_lds) + w * WF, acc);
 
@@ -856,7 +867,8 @@ __global__ __launch_bounds__(64 * kGroupWaveWpb, 2) void k_grouped_dot(const Gro
     const int64_t nct = (gp.N + 15) / 16;
     for (int ct0 = 0; ct0 < nct; ct0 += CT) {
       f4 acc[RT][CT];
-      dot_tile_lds<RT, CT, false, dot_dma(RT, CT), 0>(gp.A, gp.lda, gp.B, gp.ldb, 1, gp.M, gp.N,
+      // (the grid keeps two waves per SIMD busy)
+      dot_tile_lds<RT, CT, false, dot_dma(RT, CT), 0, dot_spread(RT, CT, false, 1 << 20)>(gp.A, gp.lda, gp.B, gp.ldb, 1, gp.M, gp.N,
                                                      row0, ct0, 0, gp.K, T, acc);
       grouped_store<RT, CT, dot_brow(CT, false)>(gp, row0, ct0, acc);
     }
@@ -1444,14 +1456,23 @@ hipError_t run_dot(int kw, const DotParams &p, hipStream_t st) {
   const int64_t nblk = nrb * p.kgroups;
   if (nblk > 0x7fffffff || ncb > 65535) return hipErrorInvalidConfiguration;
   const size_t lds = (size_t)kw * dot_wave_floats(RT, CT) * sizeof(float);
-  if (lds > 65536) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_skinny_dot<RT, CT, BV, APOL>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL((k_skinny_dot<RT, CT, BV, APOL>), dim3((unsigned)nblk, (unsigned)ncb),
-                     dim3(64 * kw), lds, st, p);
-  return hipGetLastError();
+  auto run = [&](auto spread) {
+    const void *fn = (const void *)k_skinny_dot<RT, CT, BV, APOL, decltype(spread)::value>;
+    if (lds > 65536) {
+      const hipError_t e =
+          hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return e;
+    }
+    DotParams q = p;
+    void *args[] = {&q};
+    return hipLaunchKernel(fn, dim3((unsigned)nblk, (unsigned)ncb), dim3(64 * kw), args, lds, st);
+  };
+  if constexpr (!dot_brow(CT, BV))
+    return run(std::false_type());
+  else if (RT == 1 || dot_spread(RT, CT, BV, nblk * ncb * kw))
+    return run(std::true_type());
+  else
+    return run(std::integral_constant<bool, RT == 1>());
 }
 
 typedef hipError_t (*DotFn)(int, const DotParams &, hipStream_t);
@@ -1598,14 +1619,14 @@ int skinny_dot_resident_waves(int rt, int ct) {
   if (cache[rt][ct]) return cache[rt][ct];
   const void *fn = nullptr;
   switch (rt * 16 + ct) {
-    case 17: fn = (const void *)k_skinny_dot<1, 1, false>; break;
-    case 18: fn = (const void *)k_skinny_dot<1, 2, false>; break;
-    case 20: fn = (const void *)k_skinny_dot<1, 4, false>; break;
-    case 33: fn = (const void *)k_skinny_dot<2, 1, false>; break;
-    case 34: fn = (const void *)k_skinny_dot<2, 2, false>; break;
-    case 36: fn = (const void *)k_skinny_dot<2, 4, false>; break;
-    case 65: fn = (const void *)k_skinny_dot<4, 1, false>; break;
-    case 66: fn = (const void *)k_skinny_dot<4, 2, false>; break;
+    case 17: fn = (const void *)k_skinny_dot<1, 1, false, kBufNT, false>; break;
+    case 18: fn = (const void *)k_skinny_dot<1, 2, false, kBufNT, false>; break;
+    case 20: fn = (const void *)k_skinny_dot<1, 4, false, kBufNT, true>; break;
+    case 33: fn = (const void *)k_skinny_dot<2, 1, false, kBufNT, false>; break;
+    case 34: fn = (const void *)k_skinny_dot<2, 2, false, kBufNT, false>; break;
+    case 36: fn = (const void *)k_skinny_dot<2, 4, false, kBufNT, true>; break;
+    case 65: fn = (const void *)k_skinny_dot<4, 1, false, kBufNT, false>; break;
+    case 66: fn = (const void *)k_skinny_dot<4, 2, false, kBufNT, false>; break;
     default: return 0;
   }
   cache[rt][ct] = 4 * resident_blocks(fn, skinny_dot_lds_bytes(rt, ct, 4));
