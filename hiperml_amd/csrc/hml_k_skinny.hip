@@ -133,11 +133,11 @@ __device__ __forceinline__ int dot_tile_off(int x, int kc) {
 // A, L is read so that the column blocks of one (row block, K group) land
 // on one XCD, dispatched 8 workgroups apart: the second reads of A come
 // from that XCD's L2 instead of HBM.  (A bijection whenever gridDim.x is a
-// multiple of 8; other grids keep the plain order.)
-__device__ __forceinline__ void xcd_block(int64_t *bx, int *by) {
+// multiple of 8; other grids, and calls without `share`, keep the plain order.)
+__device__ __forceinline__ void xcd_block(bool share, int64_t *bx, int *by) {
   const int64_t nx = gridDim.x;
   const int ny = (int)gridDim.y;
-  if (ny == 1 || (nx & 7)) {
+  if (!share || ny == 1 || (nx & 7)) {
     *bx = blockIdx.x;
     *by = (int)blockIdx.y;
     return;
@@ -146,6 +146,18 @@ __device__ __forceinline__ void xcd_block(int64_t *bx, int *by) {
   const int64_t j = L >> 3;
   *by = (int)(j % ny);
   *bx = (j / ny) * 8 + (L & 7);
+}
+
+// Whether k_skinny_dot's column blocks share their rows that way.  In that
+// order an XCD goes through all of B for every few row tiles, in the plain one
+// through a column block of it for all of them: B has to fit an XCD's 4 MB L2,
+// or 32-row tiles to read it in at most 8 blocks.  us, shared / plain: 16384 x
+// 128 x 8192 (4 MB) 2x4 274 / 307, 2x2 315 / 438; 4096 x 256 x 8192 (8 MB) 2x4
+// 130 / 135, 1x4 158 / 151; 4096 x 512 x 8192 (16 MB) 2x4 254 / 258, 1x4 361 /
+// 289; 4096 x 2048 x 1024 (8 MB) 2x4 175 / 152, 1x4 319 / 150; 4096 x 1024 x
+// 1024 (4 MB) 2x4 77.8 / 79.3, 1x4 78.5 / 78.6.
+__device__ __forceinline__ bool dot_share(const DotParams &p, int rt) {
+  return p.K * p.N <= 1 << 20 || (rt > 1 && gridDim.y <= 8);
 }
 
 __device__ __forceinline__ void dot_store(const DotParams &p, int64_t row,
@@ -586,7 +598,7 @@ __global__ __launch_bounds__(64 * dot_max_waves(RT, CT)) void k_skinny_dot(DotPa
   const int r = lane & 15, g = lane >> 4;
   int64_t bx;
   int by;
-  xcd_block(&bx, &by);
+  xcd_block(dot_share(p, RT), &bx, &by);
   const int64_t rb = bx / p.kgroups;
   const int kgi = (int)(bx - rb * p.kgroups);
   const int64_t row0 = rb * 16 * RT;
@@ -939,7 +951,7 @@ __global__ __launch_bounds__(64 * axpy_max_waves(RT, CT)) void k_skinny_axpy(Ski
   const int r = lane & 15, g = lane >> 4;
   int64_t bx;
   int by;
-  xcd_block(&bx, &by);
+  xcd_block(true, &bx, &by);
   const int64_t rb = bx / p.kgroups;
   const int kgi = (int)(bx - rb * p.kgroups);
   const int64_t m0 = rb * kAxpyRowsPerTile * RT;
@@ -1393,7 +1405,7 @@ __global__ __launch_bounds__(64 * kDotbWaves) void k_skinny_dotb(DotParams p) {
   const int r = lane & 15, g = lane >> 4;
   int64_t bx;
   int by;
-  xcd_block(&bx, &by);
+  xcd_block(true, &bx, &by);
   const int64_t rbk = bx / p.kgroups;
   const int kgi = (int)(bx - rbk * p.kgroups);
   const int64_t row0 = (rbk * kDotbWaves + w) * 16 * RT;
