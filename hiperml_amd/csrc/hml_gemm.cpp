@@ -406,7 +406,9 @@ double dot_model_us(const GemmKey &k, const hmlSgemmVariant &v) {
 // chunks instead of 8 would be 77 us instead of 81, at 1.4 times the error).
 // Unsplit 32-row tiles stay out: single-wave workgroups with 16 KB of LDS
 // each fill the chip unevenly (2500 x 2500 x 1000 169 us, unsplit 16-row tiles
-// 139).  Nor does it take a tile whose rows are too far apart for the skinny
+// 139).  So do 16-row tiles in place of 2x4 ones where long chunks are split
+// over a workgroup and A is read for several column blocks (12777 x 74 x 9387
+// 292 us, 1x3 361; 6435 x 94 x 13467 230, 1x3 283).  Nor does it take a tile whose rows are too far apart for the skinny
 // kernels' offsets where the chosen variant's are not.
 void dot_geometry(const GemmCanon &g, const GemmKey &k, hmlSgemmVariant *v) {
   if ((double)k.M * (double)k.N * (double)k.K < 3.5e8) return;
@@ -420,6 +422,7 @@ void dot_geometry(const GemmCanon &g, const GemmKey &k, hmlSgemmVariant *v) {
         const hmlSgemmVariant c{HML_SGEMM_FAMILY_DOT, rt, ct, ks, 4};
         const SkinnyPlan pl = plan_skinny(k, c);
         if (pl.p_floats > from.p_floats || pl.kchunk > from.kchunk) continue;
+        if (rt == 1 && pl.kw > 1 && v->rt == 2 && v->ct == 4 && pl.kchunk > 512 && k.N > 64) continue;
         if (!skinny_offsets_fit(g, c, pl)) continue;
         const double us = dot_model_us(k, c);
         if (us < best) {
@@ -427,25 +430,18 @@ void dot_geometry(const GemmCanon &g, const GemmKey &k, hmlSgemmVariant *v) {
           out = c;
         }
       }
-  // Wide products left on split 2x4 tiles: where they come to an odd number
-  // of workgroups per CU (two share one) the last runs alone, with nothing
-  // to hide its loads.  1x4 in the same split (the same chains and partial
-  // sums) is then ahead where it needs no more half rounds and B, which it
-  // reads twice as often, is small.  us, 2x4 / 1x4: 3333 x 1234 x 2345
-  // 216 / 196, 2759 x 1928 x 2880 298 / 277, 3800 x 600 x 4000 193 / 180,
-  // 5000 x 700 x 2300 169 / 161, 3000 x 2900 x 1600 283 / 262; an even number:
-  // 3001 x 2047 x 2500 274 / 286, 4000 x 1000 x 2200 165 / 179; B of 33 MB:
-  // 2759 x 2047 x 4000 391 / 417.
-  if (out.rt == 2 && out.ct == 4 && out.ksplit > 1 && k.N >= 512 &&
-      k.K * k.N * 4 <= (int64_t)28 << 20) {
+  // Wide products left on split 2x4 tiles of short chunks: 1x4 in the same
+  // split (the same chains and partial sums) is ahead, for its loads are
+  // spread over the stage (k_skinny_dot) and a short chunk pays its start and
+  // end per 16 rows.  us, 2x4 / 1x4, chunks of 192: 3346 x 3186 x 687 196 / 159,
+  // 4919 x 2173 x 540 154 / 129; 256: 2510 x 1755 x 877 104 / 86, 5936 x 911 x
+  // 943 133 / 114; 320: 2049 x 1604 x 1264 105 / 91; the other way 576: 3571 x
+  // 1161 x 2358 185 / 210, 896: 1328 x 1001 x 3452 90 / 107 (1x3).
+  if (out.rt == 2 && out.ct == 4 && k.N >= 512) {
     hmlSgemmVariant c = out;
     c.rt = 1;
     const SkinnyPlan p2 = plan_skinny(k, out), p1 = plan_skinny(k, c);
-    const int64_t nb = ceil_div(k.N, 64), nch = ceil_div(k.K, p2.kchunk);
-    const int64_t r2 = ceil_div(ceil_div(k.M, 32) * nb * nch, 1024);
-    const int64_t r1 = ceil_div(ceil_div(k.M, 16) * nb * nch, 1024);
-    if (p1.p_floats <= p2.p_floats && p1.kchunk == p2.kchunk && p1.kw == p2.kw && r2 % 2 == 1 &&
-        r1 <= 2 * r2)
+    if (p2.kw >= 3 && p2.kchunk <= 320 && p1.p_floats <= p2.p_floats && skinny_offsets_fit(g, c, p1))
       out = c;
   }
   *v = out;
