@@ -729,3 +729,44 @@ def test_partial_stage_columns(hml, K):
             hml.sgemm_ex(M, N, K, dA, dB, dC, 2.0, -1.0, lda=K + pad, ldb=N + pad, variant=v)
             hml.synchronize()
             np.testing.assert_array_equal(dC.to_numpy((M, N)), R, err_msg="%r %r" % (v, (M, N, pad)))
+
+
+def micros(hml, M, N, K, variant=None, reps=10):
+    """Best of four timings of an SGEMM on uniform data."""
+    dA, dB, dC = (hml.DeviceBuffer(4 * n) for n in (M * K, K * N, M * N))
+    dA.fill_uniform(M * K, 1)
+    dB.fill_uniform(K * N, 2)
+    best = float("inf")
+    for _ in range(5):
+        e0, e1 = hml.Event(), hml.Event()
+        e0.record()
+        for _ in range(reps):
+            hml.sgemm_ex(M, N, K, dA, dB, dC, variant=variant)
+        e1.record()
+        e1.synchronize()
+        best = min(best, e0.elapsed_ms(e1) / reps * 1e3)
+    return best
+
+
+def test_wide_products_keep_b_in_l2(hml):
+    """256 row tiles, a multiple of the 8 XCDs, are no slower than 257 where B
+    is larger than an XCD's L2 (twice the time when every XCD goes through all
+    of B for a few row tiles): within 1.4 times."""
+    v = (1, 1, 4, 4, 4)
+    assert micros(hml, 4096, 2048, 1024, v) < 1.4 * micros(hml, 4112, 2048, 1024, v)
+
+
+@pytest.mark.parametrize("M,N,K,variant", [(3571, 1161, 2358, (1, 2, 4, 4, 4)), (5120, 1913, 1891, (1, 2, 4, 4, 4)),
+                                           (2675, 2518, 698, (1, 2, 4, 4, 4)), (12777, 74, 9387, (1, 2, 4, 4, 4))])
+def test_geometry_is_not_slower(hml, M, N, K, variant):
+    """What the tile model runs in place of a selected variant takes at most
+    1.2 times its time (1.2 to 1.8 before its exceptions for wide products and
+    long chunks)."""
+    near = hml.GemmShape(2 * M, N, K, 0, 0, 0, 1)
+    hml.check(hml.lib.hmlSgemmConfigAddRule(ctypes.byref(near), ctypes.byref(hml.SgemmVariant(*variant))))
+    try:
+        assert hml.sgemm_select(M, N, K)[0].astuple() == variant
+        got = micros(hml, M, N, K)
+    finally:
+        hml.config_clear()
+    assert got < 1.2 * micros(hml, M, N, K, variant)
