@@ -196,11 +196,12 @@ constexpr float kKmSampleMax = 0x1p60f;
 constexpr int kKmHeadBytes = (2 * kKmWaves + 1) * 256 + kKmWaves * 64;
 
 // KS = k-steps of 16 dims, MULTI = the centroids take several LDS chunks,
-// VEC = dims a multiple of 4.  Several chunks fill a CU's LDS with one
-// workgroup, two waves per SIMD: they may use 256 registers (capped at 128, 64
-// dims spilled 19).
-template <int KS, bool MULTI, bool VEC, bool FUSED>
-__global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(KmParams p) {
+// VEC = dims a multiple of 4.  ROOMY: LDS holds one workgroup per CU, two
+// waves per SIMD, which may use 256 registers (64 dims need 150 to 180; capped
+// at 128, several chunks spilled 19 and took 37 us instead of 33 for 32768 rows
+// 64 x 512, one chunk spills 1 to 8).
+template <int KS, bool MULTI, bool VEC, bool FUSED, bool ROOMY = MULTI>
+__global__ __launch_bounds__(64 * kKmWaves, ROOMY ? 2 : 4) void k_kmeans_screen(KmParams p) {
   constexpr int NQ = KS * 2;  // 1 KB DMA loads per row tile (at most)
   extern __shared__ f4 km_lds4[];
   char *lds = reinterpret_cast<char *>(km_lds4);
@@ -622,10 +623,13 @@ __global__ __launch_bounds__(64 * kKmWaves, MULTI ? 2 : 4) void k_kmeans_screen(
       if ((!MULTI || live) && h == 0 && row0 + r < p.nrows) p.assign[row0 + r] = ans;
     }
   };
-  if (moved)
+  // (both loops in 128 registers spill 8 where rows are read float by float
+  // for 64 dims: 2^23 rows 62 x 55 749 us, one loop 506)
+  constexpr bool kOneLoop = KS == 4 && !VEC && !ROOMY;
+  if (moved || kOneLoop)
     steps(std::true_type());
   else
-    steps(std::false_type());
+    steps(std::integral_constant<bool, kOneLoop>());
 }
 
 typedef void (*KmKernel)(KmParams);
@@ -752,17 +756,20 @@ KmKernel kmd_kernel(int d, bool fused) {
 }
 
 template <int KS, bool FUSED>
-KmKernel kms_pick(bool multi, bool vec) {
+KmKernel kms_pick(bool multi, bool vec, bool roomy) {
+  if constexpr (KS == 4)
+    if (!multi && roomy)
+      return vec ? k_kmeans_screen<KS, false, true, FUSED, true> : k_kmeans_screen<KS, false, false, FUSED, true>;
   if (multi) return vec ? k_kmeans_screen<KS, true, true, FUSED> : k_kmeans_screen<KS, true, false, FUSED>;
   return vec ? k_kmeans_screen<KS, false, true, FUSED> : k_kmeans_screen<KS, false, false, FUSED>;
 }
 
-KmKernel kms_kernel(int ks, bool multi, bool vec, bool fused) {
+KmKernel kms_kernel(int ks, bool multi, bool vec, bool roomy, bool fused) {
   switch (ks) {
-    case 1: return fused ? kms_pick<1, true>(multi, vec) : kms_pick<1, false>(multi, vec);
-    case 2: return fused ? kms_pick<2, true>(multi, vec) : kms_pick<2, false>(multi, vec);
-    case 3: return fused ? kms_pick<3, true>(multi, vec) : kms_pick<3, false>(multi, vec);
-    default: return fused ? kms_pick<4, true>(multi, vec) : kms_pick<4, false>(multi, vec);
+    case 1: return fused ? kms_pick<1, true>(multi, vec, roomy) : kms_pick<1, false>(multi, vec, roomy);
+    case 2: return fused ? kms_pick<2, true>(multi, vec, roomy) : kms_pick<2, false>(multi, vec, roomy);
+    case 3: return fused ? kms_pick<3, true>(multi, vec, roomy) : kms_pick<3, false>(multi, vec, roomy);
+    default: return fused ? kms_pick<4, true>(multi, vec, roomy) : kms_pick<4, false>(multi, vec, roomy);
   }
 }
 
@@ -821,7 +828,7 @@ hipError_t launch_kmeans_assign(const KmeansPlan &pl, uint32_t *assign, const fl
   if (nrows <= 0) return hipSuccess;
   if (pl.direct ? pl.KC < 1 : pl.KC < 32) return hipErrorInvalidValue;
   KmKernel fn = pl.direct ? kmd_kernel(pl.ni, fused)
-                          : kms_kernel(pl.ni, pl.KC < K, D % 4 == 0, fused);
+                          : kms_kernel(pl.ni, pl.KC < K, D % 4 == 0, 2 * pl.lds > kKmLdsBytes, fused);
   if (!fn) return hipErrorInvalidValue;
   const int waves = pl.direct ? kKmDirectWaves : kKmWaves;
   hipError_t e;
