@@ -619,7 +619,7 @@ def bench_kmeans(hml, reps=5, rows=1 << 24, cpu=True):
             gbs = nbytes / ms / 1e6
             tfs = flops / ms / 1e9
             t_hbm = nbytes / (HBM_PEAK_GBS * 1e9)
-            # screened as three bf16 products per pair
+            # screened as three fp16 products per pair (the bf16 rate)
             t_mfma = 3.0 * flops / (BF16_PEAK_TFLOPS * 1e12)
             rec = {"dims": D, "clusters": K, "ms": round(ms, 4),
                    "rows_per_s": round(rows / ms * 1e3, 0), "GB_s": round(gbs, 1),

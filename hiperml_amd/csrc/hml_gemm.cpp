@@ -408,8 +408,9 @@ double dot_model_us(const GemmKey &k, const hmlSgemmVariant &v) {
 // each fill the chip unevenly (2500 x 2500 x 1000 169 us, unsplit 16-row tiles
 // 139).  So do 16-row tiles in place of 2x4 ones where long chunks are split
 // over a workgroup and A is read for several column blocks (12777 x 74 x 9387
-// 292 us, 1x3 361; 6435 x 94 x 13467 230, 1x3 283).  Nor does it take a tile whose rows are too far apart for the skinny
-// kernels' offsets where the chosen variant's are not.
+// 292 us, 1x3 361; 6435 x 94 x 13467 230, 1x3 283).  Nor does it take a tile
+// whose rows are too far apart for the skinny kernels' offsets where the
+// chosen variant's are not.
 void dot_geometry(const GemmCanon &g, const GemmKey &k, hmlSgemmVariant *v) {
   if ((double)k.M * (double)k.N * (double)k.K < 3.5e8) return;
   const SkinnyPlan from = plan_skinny(k, *v);

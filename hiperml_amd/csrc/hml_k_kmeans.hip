@@ -58,11 +58,12 @@
 //     features, 2^20 rows 32 x 64, 135 us, now 61.
 //
 // What bounds it: for few centroids the row stream (2^24 rows, 32 dims x 16
-// clusters: 0.38 ms, 5.8 TB/s, was 0.54), for many the matrix cores and the
-// three vector instructions per (row, centroid) of the trackers, which both
-// are busy 0.4 and 0.7 of the time at 32 x 256 (1.01 ms, was 3.08); 32 x 64
-// 0.46 ms (was 1.04), 64 x 64 0.96 (was 1.75), 2^23 rows 64 x 256 0.92 (was
-// 3.11).  64 rows per wave halve the LDS reads per row but held 2-3 waves
+// clusters: 0.39 ms, 5.6 TB/s), for many the matrix cores and the three vector
+// instructions per (row, centroid) of the trackers.  Where rows have no
+// clusters, more have pairs to compare.  2^24 rows, ms, clustered / uniform: 32
+// x 64 0.45 / 0.49 (FP32 products 1.04 clustered), 64 x 64 0.93 / 1.00 (1.75),
+// 32 x 256 1.08 / 1.13 (3.08), 16 x 256 0.80 / 0.80; 2^23 rows 64 x 256 0.99 /
+// 1.03 (3.11).  64 rows per wave halve the LDS reads per row but held 2-3 waves
 // per SIMD: 2-15% slower.  Four trackers per lane make the second screening
 // rarer and cost registers: up to 10% slower.
 //
@@ -787,12 +788,13 @@ KmeansPlan plan_kmeans(int64_t nrows, int D, int K, int mode) {
   KmeansPlan pl;
   // The direct kernel's time grows with dims x clusters from the row stream
   // up, the screened one's starts at the cost of splitting the rows and
-  // barely grows.  Measured on MI355X over 2^21 rows, dims 2..32 x clusters
-  // 2..128 (screened / direct, us): 5 x 32 32.5 / 33.7, 8 x 24 31.9 / 29.4,
-  // 8 x 32 32.1 / 36.8, 16 x 12 32.5 / 35.3, 24 x 8 44.8 / 38.2, 24 x 12
-  // 44.9 / 45.6, 32 x 8 49.8 / 47.7, 32 x 12 50.2 / 57.8; 4 x 8 30.6 / 11.8
-  // and 16 x 128 58.7 / 219 far from the line.  They cross between 180 and
-  // 290 for every row length.
+  // barely grows.  Measured on MI355X over 2^21 clustered rows (screened /
+  // direct, us; uniform rows within 2): 5 x 24 32.8 / 29.1, 5 x 32 32.1 / 36.2,
+  // 8 x 24 33.4 / 29.9, 8 x 32 33.3 / 37.3, 16 x 12 34.5 / 33.5, 16 x 16 34.5 /
+  // 38.1, 24 x 8 44.7 / 39.0, 24 x 10 45.1 / 44.1, 24 x 12 45.5 / 48.7, 32 x 8
+  // 49.6 / 48.4, 32 x 12 49.1 / 59.1; 4 x 8 31.9 / 11.9 and 16 x 128 64 / 221
+  // far from the line.  They cross near 140 for the shortest rows, between 200
+  // and 300 for most.
   pl.direct = (mode == 2 && D <= kKmDirectMaxDims) ||
               (mode == 0 && D <= kKmDirectMaxDims && (int64_t)K * D < kKmDirectWork);
   if (pl.direct) {
